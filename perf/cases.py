@@ -1,0 +1,650 @@
+"""Timed cases: the calls a user's program makes, with inputs of its kind.
+
+Each case is one program's work through the package's public entry points:
+
+  plain    holograms in device memory -> index volume (``reconstruct_plain``)
+  prep     holograms -> fields and speculars (``preprocess``, the work of
+           ``tomo_pretraitement``)
+  recon    fields -> spectrum volume and counts -> index volume and OTF
+           (``ewald_accumulate`` + ``finalize``, ``tomo_reconstruction``)
+  simul    index contrast -> per-angle spectra -> fields
+           (``forward_spectra`` + ``spectra_to_fields``, ``tomo_simul_holo``)
+  grad     one differentiable forward model and its gradient (torch autograd)
+  tv       geometry plan and n iterations of the adjoint-TV solver
+
+Inputs are made from the seed alone: smooth absorbing phase objects seen
+under each illumination with their parallax, a mild quadratic aberration, a
+tilted reference wave, and the camera's noise and quantisation. ``exact``
+evaluates the same chain in 64 bits with plain torch.
+"""
+import math
+
+import numpy as np
+import torch
+
+import mtd_transmission_amd as mtd
+from mtd_transmission_amd import adjoint
+
+LAM, N0, NA = 6.33e-7, 1.333, 1.2
+DEV = "cuda"
+TV_LAM, TV_EPS = 1e-2, 2e-2  # index units, as the benchmark's solver settings
+
+OFF, VOLKOV, HERRAEZ = 0, 1, 2
+
+
+def listed():
+    return [
+        # one small region of interest, refreshed at video rate: every launch
+        # and every microsecond of host work shows
+        dict(name="plain_tiny", kind="plain", n=128, nx=16, v=64, A=16, dtype="f32", scan="circle",
+             born=1, deroul=OFF),
+        # small acquisition of a 12-bit camera, plain method (Born)
+        dict(name="plain_512", kind="plain", n=512, nx=64, v=256, A=100, dtype="f32",
+             scan="circle", born=1, deroul=OFF),
+        # the full-size plain reconstruction, 600 holograms of 1024^2 -> 512^3
+        dict(name="plain_1024", kind="plain", n=1024, nx=128, v=512, A=600, dtype="u16",
+             scan="fermat", born=1, deroul=OFF),
+        # the largest frames and volume (crop 512, 1024^3)
+        dict(name="plain_2048", kind="plain", n=2048, nx=256, v=1024, A=200, dtype="u16",
+             scan="fermat", born=1, deroul=OFF),
+        # the reference's shipped settings (Rytov, Volkov unwrapping, crop 250,
+        # 512^3) on 8-bit camera frames
+        dict(name="plain_shipped", kind="plain", n=1024, nx=125, v=512, A=300, dtype="u8",
+             scan="fermat", born=0, deroul=VOLKOV),
+        # a camera whose frames and crop have no power-of-two length
+        dict(name="plain_ragged", kind="plain", n=600, nx=91, v=364, A=48, dtype="u16",
+             scan="fermat", born=0, deroul=VOLKOV),
+        # tomo_pretraitement with the shipped settings: the fields that the
+        # iterative reconstruction starts from
+        dict(name="prep_volkov", kind="prep", n=768, nx=64, v=256, A=400, dtype="u16",
+             scan="fermat", born=0, deroul=VOLKOV),
+        # tomo_pretraitement with the quality-guided unwrapping (VOLKOV 0)
+        dict(name="prep_herraez", kind="prep", n=512, nx=64, v=256, A=100, dtype="u8",
+             scan="circle", born=0, deroul=HERRAEZ),
+        # tomo_reconstruction on stored fields, with the OTF volume
+        dict(name="recon_512", kind="recon", n=1024, nx=125, v=512, A=400, scan="fermat"),
+        # tomo_simul_holo's shipped configuration (crop 122, 416^3)
+        dict(name="simul_416", kind="simul", n=1024, nx=61, v=416, A=200, scan="fermat"),
+        # one gradient of the forward model at the size of a gradient check
+        dict(name="grad_64", kind="grad", n=128, nx=16, v=64, A=60, scan="fermat"),
+        # the adjoint-TV solver on 400 angles and a 256^3 unknown
+        dict(name="tv_256", kind="tv", n=768, nx=64, v=256, A=400, scan="fermat", iters=10),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["plain", "plain", "prep", "prep", "recon", "simul", "grad", "tv"])
+    scan = rng.choice(["fermat", "circle"])
+    if kind in ("plain", "prep"):
+        # frame sides the cameras and regions of interest have: the compiled
+        # lengths, or any even side
+        n = rng.choice([256, 512, 768, 1024, 2048, 2 * _log_int(rng, 100, 600)])
+        nx = rng.choice([n // 8, rng.randint(min(100, max(24, n // 14)), min(128, int(0.19 * n)))])
+        A = _log_int(rng, 8, min(600, 600 * 1024 * 1024 // (n * n)))
+        if n % 128:
+            A = min(A, 48)
+        # the unwrapping by quality sorts its edges: crops of that path stay small
+        deroul = rng.choice([OFF, VOLKOV, VOLKOV, HERRAEZ] if nx <= 80 else [OFF, VOLKOV])
+        born = 1 if deroul == OFF else rng.choice([0, 0, 1])
+        v = 4 * nx if rng.random() < 0.5 else 2 * rng.randint(2 * nx, int(2.4 * nx))
+        v = v if v <= 400 else max(32 * (v // 32), 4 * nx)
+        if deroul == HERRAEZ:
+            A = min(A, 100)
+        return dict(kind=kind, n=n, nx=nx, v=v, A=A, dtype=rng.choice(["u8", "u16", "f32"]),
+                    scan=scan, born=born, deroul=deroul)
+    if kind in ("recon", "simul"):
+        nx = rng.choice([32, 61, 64, 96, 125, 128, rng.randint(24, 128)])
+        v = 4 * nx if rng.random() < 0.5 else min(512, 2 * rng.randint(2 * nx, 4 * nx))
+        return dict(kind=kind, n=8 * nx, nx=nx, v=max(v, 4 * nx), A=_log_int(rng, 8, 400),
+                    scan=scan)
+    nx = rng.choice([16, 32, 48, 64, rng.randint(16, 64)])
+    v = 4 * nx if rng.random() < 0.5 else 2 * rng.randint(2 * nx, int(2.5 * nx))
+    c = dict(kind=kind, n=8 * nx, nx=nx, v=v, A=_log_int(rng, 16, 400), scan=scan)
+    if kind == "tv":
+        c["iters"] = rng.randint(3, 10)
+    return c
+
+
+# --------------------------------------------------------------------------
+# geometry
+# --------------------------------------------------------------------------
+def _geometry(case):
+    """The acquisition's constants, as the configuration files give them."""
+    n, nx = case["n"], case["nx"]
+    pix = nx * LAM / (NA * n)
+    cx, cy = n // 2 - round(0.3 * n), n // 2 + round(0.3 * n)
+    f = lambda x: float(np.float32(x))  # noqa: E731  (values pass through a C float)
+    g = dict(n=n, nx=nx, C=2 * nx, V=case["v"], cx=cx, cy=cy, pix=f(pix), n0=f(N0), na=f(NA),
+             lam=f(LAM), R=math.floor(nx * f(N0) / f(NA) + 0.5), born=case.get("born", 1),
+             deroul=case.get("deroul", OFF))
+    g["pixu"] = g["pix"] * n / (2 * nx)
+    g["df"] = 1.0 / (g["pixu"] * 2 * nx)
+    return g
+
+
+def _lib_geometry(g):
+    return mtd.geom_derive(g["n"], g["nx"], g["V"], g["cx"], g["cy"], NA, N0, LAM,
+                           g["nx"] * LAM / (NA * g["n"]), 1.0, 1.0, 1.0, 1.0, g["born"], 1,
+                           g["deroul"])
+
+
+def _scan(case):
+    """Illumination frequencies (bins): a circle or a filled Fermat spiral."""
+    A, nx = case["A"], case["nx"]
+    j = np.arange(A)
+    if case["scan"] == "circle":
+        r, t = 0.9 * nx * np.ones(A), 2 * np.pi * j / A
+    else:
+        r, t = 0.95 * nx * np.sqrt(j / A), j * np.pi * (3 - math.sqrt(5))
+    return np.rint(r * np.cos(t)).astype(np.int64), np.rint(r * np.sin(t)).astype(np.int64)
+
+
+def _posspec(case):
+    kx, ky = _scan(case)
+    return torch.from_numpy(np.concatenate([kx, ky]) + case["nx"]).to(torch.int32).to(DEV)
+
+
+# --------------------------------------------------------------------------
+# inputs
+# --------------------------------------------------------------------------
+def _blobs(case, seed):
+    """Centres and radii (fractions of the field of view), peak phase (rad)
+    and peak attenuation of the object's smooth bumps."""
+    rng = np.random.default_rng(seed)
+    small = case["nx"] < 24
+    k = 2 if small else int(rng.integers(3, 7))
+    peak = 0.5 if case.get("deroul", OFF) == OFF else 6.0
+    c = rng.uniform(-0.16, 0.16, (k, 2))
+    z = rng.uniform(-0.08, 0.08, k)
+    r = rng.uniform(0.07, 0.1, k) if small else rng.uniform(0.1, 0.18, k)
+    return c, z, r, rng.uniform(0.4, 1.0, k) * peak, rng.uniform(0.05, 0.3, k)
+
+
+def _bumps(case, blobs, a0, a1, m, f):
+    """[a1-a0][m][m] sums over the bumps of f(peak phase, peak attenuation)
+    times (1 - r^2)^2, each shifted by its height times the illumination's
+    slope."""
+    c, z, r, ph, at = blobs
+    kx, ky = _scan(case)
+    fov = LAM * case["nx"] / NA  # side of the field of view (metres)
+    ax = (torch.arange(m, device=DEV, dtype=torch.float32) - m / 2) / m
+    out = torch.zeros((a1 - a0, m, m), device=DEV)
+    for i in range(len(z)):
+        s = np.stack([kx[a0:a1], ky[a0:a1]]) * LAM / (fov * N0)
+        s = z[i] * s / np.sqrt(np.maximum(1.0 - (s * s).sum(0), 0.1))
+        sx, sy = (torch.from_numpy(v).to(DEV, torch.float32) for v in s)
+        dx = (ax[None, :] - float(c[i, 0]) - sx[:, None]) / float(r[i])
+        dy = (ax[None, :] - float(c[i, 1]) - sy[:, None]) / float(r[i])
+        q = (1.0 - dx[:, None, :] ** 2 - dy[:, :, None] ** 2).clamp_(min=0.0)
+        out.add_(q.mul_(q), alpha=float(f(ph[i], at[i])))
+    return out
+
+
+def _objects(case, blobs, a0, a1, m):
+    """exp(-i phase - attenuation) of the object under illuminations a0..a1-1."""
+    phi = _bumps(case, blobs, a0, a1, m, lambda p, a: p)
+    att = _bumps(case, blobs, a0, a1, m, lambda p, a: a)
+    return torch.polar(torch.exp(-att), -phi)
+
+
+def _ramp(n, k):
+    """exp(2 pi i k x / n) for integer bins k: complex64 [len(k)][n]."""
+    e = (np.outer(k, np.arange(n)) % n) * (2 * np.pi / n)
+    return torch.from_numpy(np.exp(1j * e).astype(np.complex64)).to(DEV)
+
+
+def _chunks(A, side):
+    step = max(1, (1 << 25) // (side * side))
+    return [(a, min(A, a + step)) for a in range(0, A, step)]
+
+
+def _holograms(case, seed):
+    """[A][n][n] camera frames |R + U|^2 with noise, and the host mask of the
+    background pixels of the fields."""
+    g = _geometry(case)
+    n, C, A = g["n"], g["C"], case["A"]
+    blobs = _blobs(case, seed)
+    kx, ky = _scan(case)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    fcx, fcy = n // 2 - g["cx"], n // 2 - g["cy"]
+    ref = (_ramp(n, np.array([fcy]))[0][:, None] * _ramp(n, np.array([fcx]))[0][None, :])
+    ux, uy = _ramp(n, kx), _ramp(n, ky)
+    # the phase that makes the specular of the crop real and positive
+    psi = torch.from_numpy(np.where(((kx - fcx) + (ky - fcy)) % 2, -1.0, 1.0)).to(
+        DEV, torch.float32)
+    f = torch.fft.fftfreq(n, device=DEV) * n
+    pupil = ((f[None, :] ** 2 + f[:, None] ** 2) < case["nx"] ** 2).to(torch.float32)
+    ax = (torch.arange(n, device=DEV, dtype=torch.float32) - n / 2) * (2.0 / n)
+    aber = 0.3 * (ax[None, :] ** 2 + 0.7 * ax[:, None] ** 2 - 0.5 * ax[None, :] * ax[:, None])
+    aber = torch.polar(torch.ones_like(aber), aber)
+    dt = {"u8": torch.uint8, "u16": torch.uint16, "f32": torch.float32}[case["dtype"]]
+    out = torch.empty((A, n, n), dtype=dt, device=DEV)
+    for a0, a1 in _chunks(A, n):
+        u = _objects(case, blobs, a0, a1, n)
+        u.mul_(ux[a0:a1, None, :]).mul_(uy[a0:a1, :, None])
+        u = torch.fft.ifft2(torch.fft.fft2(u).mul_(pupil)).mul_(aber)
+        u.mul_(psi[a0:a1, None, None]).add_(ref)
+        i = u.real.square() + u.imag.square()
+        del u
+        noise = torch.randn(i.shape, device=DEV, generator=gen)
+        if case["dtype"] == "u16":  # shot noise, 20k photons at the brightest fringe
+            i.mul_(5000.0)
+            i.add_(noise.mul_(i.sqrt())).round_().clamp_(0, 65535)
+            out[a0:a1] = i.to(torch.int32).to(dt)
+        else:  # 8-bit or 12-bit camera, read noise
+            top, sigma = (255.0, 1.0) if case["dtype"] == "u8" else (4095.0, 8.0)
+            i.mul_(0.2 * top).add_(noise.mul_(sigma)).round_().clamp_(0, top)
+            out[a0:a1] = i.to(dt)
+    inside = torch.zeros((C, C), dtype=torch.bool, device=DEV)
+    for a0, a1 in _chunks(A, C):
+        inside |= (_bumps(case, blobs, a0, a1, C, lambda p, a: 1.0) > 0).any(0)
+    mask = np.where(inside.cpu().numpy(), 0, 255).astype(np.uint8)
+    b = 2 if C < 64 else 6  # the frame the hologram window tapers
+    mask[:b] = mask[-b:] = 0
+    mask[:, :b] = mask[:, -b:] = 0
+    return out, mask
+
+
+def _fields(case, seed):
+    """Born fields exp(..) - 1 on the crop grid, with the camera's noise."""
+    A, C = case["A"], 2 * case["nx"]
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    out = torch.empty((A, C, C), dtype=torch.complex64, device=DEV)
+    blobs = _blobs(case, seed)
+    for a0, a1 in _chunks(A, C):
+        noise = torch.randn((a1 - a0, C, C, 2), device=DEV, generator=gen)
+        out[a0:a1] = _objects(case, blobs, a0, a1, C) - 1.0 + 0.02 * torch.view_as_complex(noise)
+    return out
+
+
+def _contrast(case, seed):
+    """Index contrast on the V^3 grid: ellipsoids with smooth edges."""
+    V = case["v"]
+    rng = np.random.default_rng(seed)
+    ax = (torch.arange(V, device=DEV, dtype=torch.float32) - V / 2) / V
+    out = torch.zeros((V, V, V), device=DEV)
+    for _ in range(4):
+        c, r = rng.uniform(-0.12, 0.12, 3), rng.uniform(0.06, 0.15, 3)
+        d = [((ax - float(c[i])) / float(r[i])) ** 2 for i in range(3)]
+        q = d[2][:, None, None] + d[1][None, :, None] + d[0][None, None, :]
+        out.add_((1.0 - q).clamp_(min=0.0), alpha=float(rng.uniform(0.03, 0.09)))
+    return out
+
+
+# --------------------------------------------------------------------------
+# the chain in 64 bits, plain torch
+# --------------------------------------------------------------------------
+def _tukey(n, alpha):
+    """The reference's 1-D window: float arguments, pi written 3.1415."""
+    f = np.float32
+    a, nm1 = f(alpha), f(n - 1)
+    away = lambda x: int(math.floor(float(x) + 0.5))  # noqa: E731
+    b1, b2 = away(f(a * nm1) / f(2)), away(nm1 * f(f(1) - f(a / f(2))))
+    i = np.arange(n)
+    q = ((2 * i).astype(f) / f(a * nm1)).astype(f)
+    lo = 0.5 * (1 + np.cos(3.1415 * (q - f(1)).astype(f).astype(np.float64)))
+    hi = 0.5 * (1 + np.cos(3.1415 * ((q - f(f(2) / a)).astype(f) + f(1)).astype(f)
+                           .astype(np.float64)))
+    return torch.from_numpy(np.where(i < b1 + 1, lo, np.where(i < b2 + 1, 1.0, hi))).to(DEV)
+
+
+def _fit_background(v, xs, ys, C):
+    """Degree-4 polynomial fit of v[A][C][C] at the sample points, on the grid."""
+    def basis(x, y):
+        x, y = x / C - 0.5, y / C - 0.5
+        return torch.stack([x ** i * y ** j for i in range(5) for j in range(5 - i)], -1)
+    B = basis(xs.double(), ys.double())
+    q, r = torch.linalg.qr(B.cpu())
+    coef = torch.linalg.solve_triangular(r, q.T @ v[:, ys, xs].T.cpu(), upper=True).to(DEV)
+    ax = torch.arange(C, device=DEV, dtype=torch.float64)
+    full = basis(ax[None, :].expand(C, C), ax[:, None].expand(C, C))
+    return (full.reshape(C * C, -1) @ coef).T.reshape(-1, C, C)
+
+
+def _volkov(phi):
+    """Unwrapped phase: the gradient of the 2 pi multiples on the even
+    extension, integrated in least squares by FFT."""
+    C = phi.shape[-1]
+    D = 2 * C
+    s = torch.cat([phi.flip(-1), phi], -1)
+    s = torch.cat([s.flip(-2), s], -2)
+    z = torch.polar(torch.ones_like(s), s)
+    k = torch.from_numpy((((np.arange(D) + C) % D) - C) / D).to(DEV)
+    kx, ky = k[None, :], k[:, None]
+    S, Z = torch.fft.fft2(s), torch.fft.fft2(z)
+    t = torch.zeros_like(S)
+    for w in (kx, ky):
+        ds = torch.fft.ifft2(2j * math.pi * w * S).real
+        dz = torch.fft.ifft2(2j * math.pi * w * Z)
+        t += w * torch.fft.fft2(((-1j * dz / z).real - ds) / (2 * math.pi) + 0j)
+    den = 2 * math.pi * (kx * kx + ky * ky)
+    den[0, 0] = 1.0
+    t = -1j * t / den
+    t[:, 0, 0] = 0
+    return phi + 2 * math.pi * torch.fft.ifft2(t).real[:, C:, C:]
+
+
+def _exact_fields(case, seed):
+    g = _geometry(case)
+    n, nx, C, A = g["n"], g["nx"], g["C"], case["A"]
+    holos, mask = _holograms(case, seed)
+    w = _tukey(n, 0.05)
+    w2 = w[:, None] * w[None, :]
+    x0, y0 = g["cx"] - nx, g["cy"] - nx
+    ys, xs = np.mgrid[0:C, 0:C]
+    sel = (ys % 5 == 0) & (xs % 5 == 0) & (mask > 45)
+    ys, xs = torch.from_numpy(ys[sel]).to(DEV), torch.from_numpy(xs[sel]).to(DEV)
+    pos = torch.empty((2 * A,), dtype=torch.int64, device=DEV)
+    out = torch.empty((A, C, C), dtype=torch.complex128, device=DEV)
+    for a0, a1 in _chunks(A, n):
+        F = torch.fft.fft2(torch.fft.fftshift(holos[a0:a1].double() * w2, (-2, -1)))
+        F = torch.fft.fftshift(F, (-2, -1))[:, y0:y0 + C, x0:x0 + C] / (n * n)
+        key = F.abs().reshape(a1 - a0, -1)
+        key[:, 0] = key[:, 0] ** 2
+        p = key.argmax(1)
+        px, py = p % C, p // C
+        pos[a0:a1], pos[A + a0:A + a1] = px, py
+        U = torch.stack([torch.roll(F[i], (-int(py[i]), -int(px[i])), (0, 1))
+                         for i in range(a1 - a0)])
+        U = torch.fft.fftshift(torch.fft.ifft2(U, norm="forward"), (-2, -1))
+        phi = torch.angle(U)
+        if g["deroul"] == VOLKOV:
+            phi = _volkov(phi)
+        amp = U.abs()
+        pc = phi - _fit_background(phi, xs, ys, C)
+        a = amp / (_fit_background(amp, xs, ys, C) + 1e-8)
+        a = torch.where(a.abs() > 10, torch.ones_like(a), a).abs()
+        out[a0:a1] = torch.polar(a, pc) - 1.0 if g["born"] else torch.complex(a.log(), pc)
+    return out, pos
+
+
+def _shift_rows(x, px, py):
+    return torch.stack([torch.roll(x[i], (int(py[i]), int(px[i])), (0, 1))
+                        for i in range(x.shape[0])])
+
+
+def _caps(g, pos, a):
+    """Pupil pixels (row-major mask) of angle a and the voxels they fall on;
+    None when the illumination leaves the Ewald sphere."""
+    nx, V, R = g["nx"], g["V"], g["R"]
+    A = len(pos) // 2
+    fx, fy = int(pos[a]) - nx, int(pos[A + a]) - nx
+    if R * R - fx * fx - fy * fy < 0:
+        return None
+    if "pupil" not in g:
+        ax = torch.arange(-nx, nx, device=DEV)
+        dy, dx = ax[:, None].expand(2 * nx, 2 * nx), ax[None, :].expand(2 * nx, 2 * nx)
+        r2 = dx * dx + dy * dy
+        m = r2 < nx * nx
+        g["pupil"] = (m, dx[m], dy[m], torch.sqrt((R * R - r2[m]).double()))
+    m, dx, dy, h = g["pupil"]
+    d = h - math.sqrt(R * R - fx * fx - fy * fy)
+    z = torch.where(d < 0, -torch.floor(-d + 0.5), torch.floor(d + 0.5)).long()
+    return (dx - fx + V // 2) + V * (dy - fy + V // 2) + V * V * (z + V // 2)
+
+
+def _scatter(g, spec, pos, factor):
+    """Sum of i factor S over the hits of every angle, and the hit counts."""
+    V = g["V"]
+    re, im = (torch.zeros(V ** 3, dtype=torch.float64, device=DEV) for _ in range(2))
+    cnt = torch.zeros(V ** 3, dtype=torch.int32, device=DEV)
+    pos = pos.tolist()
+    for a in range(spec.shape[0]):
+        vox = _caps(g, pos, a)
+        if vox is None:
+            continue
+        m, _, _, h = g["pupil"]
+        s = spec[a][m] * factor(h)
+        re.index_add_(0, vox, -s.imag)
+        im.index_add_(0, vox, s.real)
+        cnt.index_add_(0, vox, torch.ones_like(vox, dtype=torch.int32))
+    return torch.complex(re, im).view(V, V, V), cnt.view(V, V, V)
+
+
+def _centred(x, sign):
+    """Centred 3-D DFT (unnormalised) in place of its argument, axis by axis."""
+    for d in (0, 1, 2):
+        x = torch.fft.ifftshift(x, d)
+        x = torch.fft.fft(x, dim=d) if sign < 0 else torch.fft.ifft(x, dim=d, norm="forward")
+        x = torch.fft.fftshift(x, d)
+    return x
+
+
+def _beta(g):
+    k0 = float(np.float32(np.float32(2 * 3.14159 / g["lam"]) * np.float32(g["n0"])))
+    return lambda h: (k0 / 3.14159) * (-2 * 3.14159) * (h / g["R"])
+
+
+def _exact_spectra(g, fields, pos):
+    C, A = g["C"], fields.shape[0]
+    w = _tukey(C, 0.1)
+    f = torch.fft.fftshift(fields * (w[:, None] * w[None, :]), (-2, -1))
+    return _shift_rows(torch.fft.fft2(f) * g["pixu"] ** 2, pos[:A], pos[A:])
+
+
+def _exact_index(g, vol, cnt):
+    t = _centred(vol / cnt.clamp(min=1), +1)
+    kv = 2 * math.pi / g["lam"]
+    t *= -g["df"] ** 3 / (2 * g["n0"] * kv * kv)
+    return t
+
+
+def _exact_forward(g, dn, pos):
+    """Per-angle spectra [A][C][C] of the contrast dn (calcHolo's model)."""
+    V, C = g["V"], g["C"]
+    tp = 1.0 / (V * g["df"])
+    T = (_centred(dn.to(torch.complex128), -1) * tp ** 3).reshape(-1)
+    A = pos.numel() // 2
+    S = torch.zeros((A, C, C), dtype=torch.complex128, device=DEV)
+    pl = pos.tolist()
+    for a in range(A):
+        vox = _caps(g, pl, a)
+        if vox is not None:
+            m, _, _, h = g["pupil"]
+            S[a][m] = -1j * _q(g, h) * T[vox]
+    return S
+
+
+def _q(g, h):
+    return (2 * 3.14159 / g["lam"]) * g["R"] / h
+
+
+def _exact_adjoint(g, S, pos):
+    V = g["V"]
+    vol, _ = _scatter(g, S, pos, lambda h: _q(g, h))
+    return _centred(vol, +1).real * (1.0 / (V * g["df"])) ** 3
+
+
+def _exact_weights(g, pos):
+    """1 / (q^2 hits) on the cap samples."""
+    C, A = g["C"], pos.numel() // 2
+    _, cnt = _scatter(g, torch.zeros((A, C, C), dtype=torch.complex128, device=DEV), pos,
+                      lambda h: 0.0)
+    cnt = cnt.reshape(-1).double()
+    w = torch.zeros((A, C, C), dtype=torch.float64, device=DEV)
+    pl = pos.tolist()
+    for a in range(A):
+        vox = _caps(g, pl, a)
+        if vox is not None:
+            m, _, _, h = g["pupil"]
+            w[a][m] = 1.0 / (_q(g, h) ** 2 * cnt[vox])
+    return w
+
+
+def _tv_gradient(x, eps):
+    d = [torch.diff(x, dim=i, append=x.narrow(i, x.shape[i] - 1, 1)) for i in range(3)]
+    s = torch.rsqrt(d[0] ** 2 + d[1] ** 2 + d[2] ** 2 + eps * eps)
+    out = torch.zeros_like(x)
+    for i in range(3):
+        q = d[i] * s
+        out -= q
+        out.narrow(i, 1, x.shape[i] - 1).add_(q.narrow(i, 0, x.shape[i] - 1))
+    return out
+
+
+def _tv_inputs(case, seed, g):
+    """Measured spectra of a contrast (with noise), data weights, start volume
+    and the data term's scale."""
+    pos = _posspec(case)
+    dn = _contrast(case, seed)
+    y = _exact_forward(g, dn, pos)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    noise = torch.randn(tuple(y.shape) + (2,), device=DEV, generator=gen, dtype=torch.float64)
+    y = (y + 0.02 * y.abs().square().mean().sqrt() * torch.view_as_complex(noise))
+    w = _exact_weights(g, pos).to(torch.float32)
+    start = 0.5 * dn + 0.002 * torch.randn(dn.shape, device=DEV, generator=gen)
+    kappa = (1.0 / (g["V"] * g["df"])) ** 6 * float(g["V"]) ** 3
+    return pos, y.to(torch.complex64), w, start, 1.0 / kappa
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    g = _geometry(case)
+    A, C = case["A"], g["C"]
+    if case.get("deroul") == HERRAEZ:
+        return None  # whole-number decisions on the 32-bit reliabilities
+    if kind == "prep":
+        return {"fields": _exact_fields(case, seed)[0], "posspec": None}
+    if kind == "plain":
+        fields, pos = _exact_fields(case, seed)
+        spec = _exact_spectra(g, fields, pos)
+        del fields
+        idx = _exact_index(g, *_scatter(g, spec, pos, _beta(g)))
+        return {"index_re": idx.real, "index_im": idx.imag, "posspec": None}
+    if kind == "recon":
+        pos = _posspec(case)
+        spec = _exact_spectra(g, _fields(case, seed).to(torch.complex128), pos)
+        vol, cnt = _scatter(g, spec, pos, _beta(g))
+        idx = _exact_index(g, vol, cnt)
+        return {"vol": vol, "counts": None, "index_re": idx.real, "index_im": idx.imag,
+                "otf": None}
+    if kind == "simul":
+        pos = _posspec(case)
+        S = _exact_forward(g, _contrast(case, seed), pos)
+        f = torch.fft.ifft2(_shift_rows(S, -pos[:A], -pos[A:]), norm="forward")
+        return {"spectra": S, "fields": torch.fft.fftshift(f, (-2, -1)) * g["df"] ** 2}
+    if kind == "grad":
+        pos, y, w, dn, _ = _tv_inputs(case, seed, g)
+        S = _exact_forward(g, dn.double(), pos)
+        # the output gradient is formed by the caller in 32 bits: use those values
+        gs = _grad_of(_exact_forward(g, dn, pos).to(torch.complex64), y, w)
+        return {"spectra": S, "gradient": _exact_adjoint(g, gs.to(torch.complex128), pos)}
+    pos, y, w, x, inv_kappa = _tv_inputs(case, seed, g)
+    y, w, x = y.to(torch.complex128), w.double(), x.double()
+    lam, eps = float(np.float32(TV_LAM)), float(np.float32(TV_EPS))
+    step = 1.0 / (1.0 + 12.0 * lam / eps)
+    x = x.clamp(min=0.0)
+    z, t = x.clone(), 1.0
+    for _ in range(case["iters"]):
+        gd = _exact_adjoint(g, w * (_exact_forward(g, z, pos) - y), pos)
+        xn = (z - step * (inv_kappa * gd + lam * _tv_gradient(z, eps))).clamp_(min=0.0)
+        tn = 0.5 * (1.0 + math.sqrt(1.0 + 4.0 * t * t))
+        z = xn + ((t - 1.0) / tn) * (xn - x)
+        x, t = xn, tn
+    return {"x": x}
+
+
+def _grad_of(S, y, w):
+    return (S - y) * w
+
+
+# --------------------------------------------------------------------------
+# the program's side
+# --------------------------------------------------------------------------
+_CTX = None
+
+
+def _context():
+    """The context a program keeps for all its calls."""
+    global _CTX
+    if _CTX is None:
+        _CTX = mtd.Context(0)
+    return _CTX
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    g = _geometry(case)
+    A, C, V = case["A"], g["C"], g["V"]
+    s = dict(kind=kind, ctx=_context(), g=_lib_geometry(g), V=V, C=C, A=A)
+    new = lambda shape, dt: torch.empty(shape, dtype=dt, device=DEV)  # noqa: E731
+    if kind in ("plain", "prep"):
+        s["holos"], s["mask"] = _holograms(case, seed)
+        s["posspec"] = new((2 * A,), torch.int32)
+        if kind == "prep":
+            s["fields"] = new((A, C, C), torch.complex64)
+    if kind == "recon":
+        s["fields"], s["posspec"] = _fields(case, seed), _posspec(case)
+        s["vol"] = new((V, V, V), torch.complex64)
+        s["counts"] = new((V, V, V), torch.int32)
+        s["otf"] = new((V, V, V), torch.uint8)
+    if kind in ("plain", "recon"):
+        s["index_re"], s["index_im"] = (new((V, V, V), torch.float32) for _ in range(2))
+    if kind == "simul":
+        s["dn"], s["posspec"] = _contrast(case, seed), _posspec(case)
+        s["spectra"], s["fields"] = (new((A, C, C), torch.complex64) for _ in range(2))
+    if kind == "grad":
+        s["posspec"], y, w, s["dn"], _ = _tv_inputs(case, seed, g)
+        S = _exact_forward(g, s["dn"], s["posspec"]).to(torch.complex64)
+        s["grad_out"] = _grad_of(S, y, w)
+    if kind == "tv":
+        s["posspec"], s["y"], s["w"], s["start"], s["inv_kappa"] = _tv_inputs(case, seed, g)
+        s["x"], s["iters"] = torch.empty_like(s["start"]), case["iters"]
+    return s
+
+
+def run(s):
+    kind, ctx, g = s["kind"], s["ctx"], s["g"]
+    if kind == "plain":
+        ctx.reconstruct_plain(g, s["holos"], s["mask"], s["index_re"], s["index_im"],
+                              s["posspec"])
+        return {k: s[k] for k in ("index_re", "index_im", "posspec")}
+    if kind == "prep":
+        ctx.preprocess(g, s["holos"], s["mask"], s["posspec"], s["fields"])
+        return {k: s[k] for k in ("fields", "posspec")}
+    if kind == "recon":
+        ctx.ewald_accumulate(g, s["fields"], s["posspec"], s["vol"], s["counts"])
+        ctx.finalize(g, s["vol"], s["counts"], s["index_re"], s["index_im"], s["otf"])
+        return {k: s[k] for k in ("vol", "counts", "index_re", "index_im", "otf")}
+    if kind == "simul":
+        ctx.forward_spectra(g, s["dn"], None, s["posspec"], s["spectra"])
+        ctx.spectra_to_fields(g, s["spectra"], s["posspec"], s["fields"])
+        return {k: s[k] for k in ("spectra", "fields")}
+    if kind == "grad":
+        dn = s["dn"].detach().requires_grad_(True)
+        S = adjoint.born_spectra(dn, ctx, g, s["posspec"])
+        (gradient,) = torch.autograd.grad(S, dn, grad_outputs=s["grad_out"])
+        return {"spectra": S.detach(), "gradient": gradient}
+    s["x"].copy_(s["start"])
+    ctx.born_plan(g, s["posspec"])
+    ctx.tv_solve(g, s["y"], s["w"], s["x"], s["iters"], TV_LAM, TV_EPS, s["inv_kappa"])
+    return {"x": s["x"]}
+
+
+def work(case):
+    """Bytes: every input read once and every output written once (the
+    solver's iterates once per iteration: an iteration needs all of the one
+    before). Operations: 5 L log2 L per complex transform of length L, half
+    for real input, over the lines a path has to transform."""
+    kind, n, C, V, A = case["kind"], case["n"], 2 * case["nx"], case["v"], case["A"]
+    b = {"u8": 1, "u16": 2, "f32": 4}.get(case.get("dtype"), 0)
+    fft = lambda length, lines: 5.0 * length * math.log2(length) * lines  # noqa: E731
+    holo = fft(n, A * (n / 2 + C)) + fft(C, A * 2 * C)
+    spec = fft(C, A * 2 * C)
+    vol = fft(V, 3 * V * V)
+    if kind == "plain":
+        return dict(bytes=A * b * n * n + 8 * A + 8 * V ** 3, flops=holo + spec + vol)
+    if kind == "prep":
+        return dict(bytes=A * b * n * n + 8 * A + 8 * A * C * C, flops=holo)
+    if kind == "recon":
+        return dict(bytes=8 * A * C * C + 8 * A + (2 * 12 + 8 + 1) * V ** 3, flops=spec + vol)
+    if kind == "simul":
+        return dict(bytes=4 * V ** 3 + 8 * A + 3 * 8 * A * C * C, flops=vol / 2 + spec)
+    if kind == "grad":
+        return dict(bytes=8 * V ** 3 + 8 * A + 16 * A * C * C, flops=vol)
+    return dict(bytes=case["iters"] * (12 * A * C * C + 16 * V ** 3) + 8 * V ** 3,
+                flops=case["iters"] * vol)
