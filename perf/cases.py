@@ -83,7 +83,7 @@ def draw(rng):
         # frame sides the cameras and regions of interest have: the compiled
         # lengths, or any even side
         n = rng.choice([256, 512, 768, 1024, 2048, 2 * _log_int(rng, 100, 600)])
-        nx = rng.choice([n // 8, rng.randint(min(100, max(24, n // 14)), min(128, int(0.19 * n)))])
+        nx = rng.choice([n // 8 if n % 128 == 0 else n // 12, rng.randint(min(100, max(24, n // 14)), min(128, int(0.19 * n)))])
         A = _log_int(rng, 8, min(600, 600 * 1024 * 1024 // (n * n)))
         if n % 128:
             A = min(A, 48)
@@ -91,7 +91,9 @@ def draw(rng):
         deroul = rng.choice([OFF, VOLKOV, VOLKOV, HERRAEZ] if nx <= 80 else [OFF, VOLKOV])
         born = 1 if deroul == OFF else rng.choice([0, 0, 1])
         v = 4 * nx if rng.random() < 0.5 else 2 * rng.randint(2 * nx, int(2.4 * nx))
-        v = v if v <= 400 else max(32 * (v // 32), 4 * nx)
+        v = min(v if v <= 400 else max(32 * (v // 32), 4 * nx), 1024)
+        if deroul == VOLKOV:
+            A = min(A, max(8, 300 * 1024 * 1024 // (n * n)))
         if deroul == HERRAEZ:
             A = min(A, 100)
         return dict(kind=kind, n=n, nx=nx, v=v, A=A, dtype=rng.choice(["u8", "u16", "f32"]),
