@@ -278,11 +278,11 @@ hipError_t launch_form_field(int C, const float2* iu, const float2* crop,
                              const int* posx, const int* posy, int A,
                              const double* coef, int mode, const float* phu, float2* fields,
                              hipStream_t s);
-// Volkov unwrapping of the wrapped phase of IU into phu; scratch buffers:
-// gx, gy [A][2C][2C] float, P [A][2C][2C] float2, Q [A][2C][C] float2;
-// tw2C: twiddles of length 2C.
-hipError_t launch_unwrap(int C, const float2* iu, int A, const FftTab& ft2C, float* gx,
-                         float* gy, float2* P, float2* Q, float* phu, hipStream_t s);
+// Volkov unwrapping of the phase of IU into phu (U frame, up to a constant
+// per angle); scratch of unwrap_scratch_bytes(C, A); ftC: tables of length C;
+// tw4: twiddles of length 4C.
+hipError_t launch_unwrap(int C, const float2* iu, int A, const FftTab& ftC, const float2* tw4,
+                         void* scratch, float* phu, hipStream_t s);
 size_t unwrap_scratch_bytes(int C, int A);
 // Herraez unwrapping of the wrapped phase of IU into phu (U frame);
 // border: the angles' border reliabilities (herraez_border_table), scratch

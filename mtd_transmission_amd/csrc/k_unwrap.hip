@@ -2,26 +2,50 @@
 // pretraitement_hors_axe_CPU/src/deroulement_volkov4.cpp:14-92).
 //
 // For each angle the wrapped phase phi = atan2(U) of the C x C demodulated
-// field is mirror-extended to D x D (D = 2C, Symetrise_mirror :221-240), the
-// FFT gradients of phi_s and of Z = exp(i phi_s) give the gradient of the
-// field of 2 pi multiples, g = (Re(-i grad Z / Z) - Re(grad phi_s)) / 2 pi,
-// which is integrated by the FFT least-squares (Poisson) solve of integ_grad4
+// field is mirror-extended to 2C x 2C (Symetrise_mirror :221-240), the FFT
+// gradients of phi_s and of Z = exp(i phi_s) give the gradient of the field of
+// 2 pi multiples, g = (Im(grad Z / Z) - grad phi_s) / 2 pi, which is
+// integrated by the FFT least-squares (Poisson) solve of integ_grad4
 // (:162-191); the original quadrant of the result times 2 pi is added to phi.
 //
-// GPU restructuring (same mathematics):
-//  - a gradient along x only involves x frequencies: the reference's 2-D
-//    forward FFT (scaled 1/D^2), multiplication by 2 pi i kx and unnormalised
-//    2-D backward FFT equal a 1-D forward FFT along each row, 2 pi i kx / D,
-//    and a 1-D backward FFT. k_grad_rows / k_grad_cols do both transforms in
-//    one kernel per line, for phi_s and Z together;
-//  - the two real gradient fields are packed as gx + i gy into one 2-D
-//    forward FFT and separated with the Hermitian symmetry inside the
-//    integration's first inverse pass;
-//  - only the [C,2C)^2 quadrant of the integral is needed: the inverse row
-//    pass keeps the right half, the inverse column pass the lower half.
-// The mirror images are index arithmetic on load (no D x D phase is stored).
-// The reference's zero frequency reads one element past its array (:189);
-// it only adds a constant that the phase fit always removes; here it is 0.
+// Two identities take this to four passes of C-point transforms:
+//  - The spectral gradient and the spectral least-squares integration undo
+//    each other, so integrating -grad phi_s gives mean(phi) - phi exactly:
+//    the unwrapped phase is the integral of Im(grad Z / Z) plus the constant
+//    mean(phi). Unwrapping only runs ahead of the polynomial phase fit, whose
+//    constant monomial removes any constant (as it removes the reference's
+//    arbitrary zero frequency, :189, read one element past its array), so
+//    the constant is left out and phi itself is never needed: Z = U / |U|.
+//  - On the even extension every transform is a cosine or sine transform of
+//    the C original samples. The Nyquist terms vanish: the extension has
+//    none, and a gradient's, halved by its one-sided frequency -1/2, only
+//    gives an imaginary part, which the reference discards. A C-point DCT-II
+//    is one C-point complex FFT of the reordered line (J. Makhoul, "A fast
+//    cosine transform in one and two dimensions", IEEE Trans. ASSP 28, 1980):
+//    position m holds sample n(m) = 2m (m < C/2) or 2(C-1-m)+1, and with
+//    V = FFT(v), t = pi k / 2C, P = e^{-it} V[k], Q = e^{it} V[C-k] (V[C] =
+//    V[0]), the DCT-II is X[k] = (P + Q) / 2 and X[C-k] = i (P - Q) / 2, for
+//    complex lines too (two real lines in one transform). The DST-II of x is
+//    the DCT-II of (-1)^n x, read at C - k. The inverse of real Y[k] is the
+//    backward FFT of e^{it} (Y[k] - i Y[C-k]), Y[C] = 0, whose position m
+//    holds Y[0] + 2 sum_k Y[k] cos(pi k (2n+1) / 2C) at n = n(m).
+//  So the derivative of a line of Z is: FFT, W[k] = -(i pi / 2C)
+//  ((1 - 2k/C) V[k] - e^{i pi k/C} V[C-k]), backward FFT, sign -1 on the odd
+//  samples.
+// Passes (C x C per angle; each one reads and writes memory once):
+//  A rows     gx = Im(dZ/dx conj Z)                               8 + 4 bytes
+//  B columns  gy the same way, in registers; DCT-II along y of gx and
+//             DST-II along y of gy from one packed FFT: H        12 + 8
+//  C rows     DST-II along x of the first, DCT-II along x of the second from
+//             one packed FFT, the Poisson quotient, inverse along x: R  8 + 4
+//  D columns  inverse along y, two columns in one FFT: the phase   4 + 4
+// 52 bytes per pixel bound the passes. The same method on the 2C x 2C extension
+// (half-empty transforms, both gradients with their trigonometry on every
+// pixel three times) moved about 300. Measured, all unwrapping kernels, that
+// form against this one: 300 crops of 250^2 3217 -> 610 us, 400 of 128^2 813 ->
+// 144 us, 48 of 182^2 (runtime-length FFTs) 986 -> 182 us.
+#include <cfloat>
+
 #include "dft.hpp"
 #include "gen_fft.hpp"
 #include "internal.hpp"
@@ -29,393 +53,449 @@
 
 namespace mtd {
 
-// source index in [0, C) of position i in [0, 2C) of the even extension
-__device__ __forceinline__ int mirror_src(int i, int C) {
-  return i < C ? C - 1 - i : i - C;
-}
-template <int C>
-__device__ __forceinline__ int mirror_src(int i) {
-  return mirror_src(i, C);
+// sample held by position m of the reordered line (C even)
+__device__ __forceinline__ int dct_src(int m, int C) { return m < C / 2 ? 2 * m : 2 * (C - 1 - m) + 1; }
+
+// exp(i atan2(u.y, u.x)) without the angle: u / |u|. Outside the range where
+// |u|^2 is a normal float (and for zeros, infinities and NaN) u is brought
+// into range first, so that every value gives what the angle would.
+__device__ __forceinline__ float2 unit_phasor(float2 u) {
+  float m = u.x * u.x + u.y * u.y;
+  if (!(m > FLT_MIN && m < FLT_MAX)) {
+    if (m != m) return make_float2(m, m);
+    const float s = fmaxf(fabsf(u.x), fabsf(u.y));
+    if (s == 0.f) return make_float2(copysignf(1.f, u.x), u.y);
+    if (s > FLT_MAX) {
+      u = make_float2(copysignf(fabsf(u.x) > FLT_MAX ? 1.f : 0.f, u.x),
+                      copysignf(fabsf(u.y) > FLT_MAX ? 1.f : 0.f, u.y));
+    } else {
+      const int e = -ilogbf(s);
+      u = make_float2(ldexpf(u.x, e), ldexpf(u.y, e));
+    }
+    m = u.x * u.x + u.y * u.y;
+  }
+  const float r = __builtin_amdgcn_rsqf(m);
+  return make_float2(u.x * r, u.y * r);
 }
 
-// wrapped phase of U[y][x], U held in the IU frame
-__device__ __forceinline__ float wrapped_phase(const float2* __restrict__ iu_a, int y, int x,
-                                               int C) {
-  const float2 u = iu_a[((y + C / 2) % C) * C + (x + C / 2) % C];
-  return atan2f(u.y, u.x);
-}
-template <int C>
-__device__ __forceinline__ float wrapped_phase(const float2* __restrict__ iu_a, int y, int x) {
-  return wrapped_phase(iu_a, y, x, C);
-}
-
-// frequency in cycles per pixel of FFT index k (init_kvect_shift,
-// FFT_fonctions.cpp:7-17; the Nyquist index gets -1/2)
-__device__ __forceinline__ float kfreq(int k, int D) {
-  return (float)(((k + D / 2) % D) - D / 2) / (float)D;
-}
-template <int D>
-__device__ __forceinline__ float kfreq(int k) {
-  return kfreq(k, D);
+// derivative spectrum in the reordered line's terms: W[k] from V[k] and
+// V[C-k]; tw4[j] = exp(-2 pi i j / 4C)
+__device__ __forceinline__ float2 deriv_bin(float2 V, float2 Vr, int k, int C,
+                                            const float2* __restrict__ tw4) {
+  const float2 e = tw4[2 * k];  // exp(-i pi k / C)
+  const float a = (float)(C - 2 * k) / (float)C;
+  // a V - conj(e) Vr
+  const float sx = a * V.x - (e.x * Vr.x + e.y * Vr.y);
+  const float sy = a * V.y - (e.x * Vr.y - e.y * Vr.x);
+  const float w = (float)(3.14159265358979323846 / 2.0) / (float)C;
+  return make_float2(w * sy, -w * sx);
 }
 
-// d/dx of one line held in the two-step layout: v (input layout) in, u
-// (threads n2 < L1 hold positions n2 + L1*k2) out. Forward FFT, times
-// 2 pi i k / D, back to the input layout through the exchange storage x,
-// backward FFT.
-template <int D, class X>
-__device__ __forceinline__ void line_derivative(X x, const float2* __restrict__ tw, int n2,
-                                                float2 (&v)[Fft2<D, false>::L1],
-                                                float2 (&u)[Fft2<D, false>::L2]) {
-  using F = Fft2<D, false>;
-  using B = Fft2<D, true>;
-  const float two_pi = (float)(2.0 * 3.14159265358979323846);
+// P = e^{-it} V[k] and Q = e^{it} V[C-k], e = e^{-it}
+__device__ __forceinline__ float2 dct_p(float2 V, float2 e) { return cmul(V, e); }
+__device__ __forceinline__ float2 dct_q(float2 Vr, float2 e) {
+  return make_float2(Vr.x * e.x + Vr.y * e.y, Vr.y * e.x - Vr.x * e.y);
+}
+
+// Bin (kx, ky) of the integration: from P and Q of the packed row transform
+// (real part: DST-II along x of gx's y-cosine terms, imaginary part: DCT-II
+// along x of gy's y-sine terms), the potential's cosine coefficients at kx and
+// at C - kx, and the inverse transform's input e^{it} (Y[kx] - i Y[C-kx]).
+__device__ __forceinline__ float2 poisson_bin(float2 P, float2 Q, float2 e, int kx, int ky, int C) {
+  const float fx = (float)kx, fy = (float)ky, fr = (float)(C - kx);
+  const float s = (float)(-1.0 / (2.0 * 3.14159265358979323846)) / (float)C;
+  float y0 = 0.f, y1 = 0.f;
+  if (kx | ky) y0 = s * ((fy - fx) * P.y + (fy + fx) * Q.y) / (fx * fx + fy * fy);
+  if (kx) y1 = s * ((fy + fr) * P.x - (fy - fr) * Q.x) / (fr * fr + fy * fy);
+  // e^{it} = conj(e); times (y0 - i y1)
+  return make_float2(e.x * y0 - e.y * y1, -e.y * y0 - e.x * y1);
+}
+
+// Moves bins from Fft2's output layout (threads n2 < L1, u[k2] at k = n2 +
+// L1 k2) to its input layout, each with its mirror bin: v[n1] at k = L2 n1 +
+// n2, r[n1] at (C - k) mod C. Starts and ends with a barrier.
+template <int C, class X>
+__device__ __forceinline__ void bins_to_input(const float2 (&u)[Fft2<C, false>::L2],
+                                              float2 (&v)[Fft2<C, false>::L1],
+                                              float2 (&r)[Fft2<C, false>::L1], int n2, X x) {
+  constexpr int L1 = Fft2<C, false>::L1, L2 = Fft2<C, false>::L2;
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+    __syncthreads();
+    if (n2 < L1) {
+#pragma unroll
+      for (int k2 = 0; k2 < L2; ++k2) *x.lin(n2 + L1 * k2) = part ? u[k2].y : u[k2].x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n1 = 0; n1 < L1; ++n1) {
+      const int k = L2 * n1 + n2, m = k ? C - k : 0;
+      (part ? v[n1].y : v[n1].x) = *x.lin(k);
+      (part ? r[n1].y : r[n1].x) = *x.lin(m);
+    }
+  }
+  __syncthreads();
+}
+
+// the line of phasors z (input layout, reordered) -> Im(dZ conj Z) without
+// the odd samples' sign, at the same positions. v and u: work registers.
+template <int C, class X>
+__device__ __forceinline__ void line_gradient(const float2 (&z)[Fft2<C, false>::L1],
+                                              float (&g)[Fft2<C, false>::L1], int n2, X x,
+                                              const float2* __restrict__ tw,
+                                              const float2* __restrict__ tw4) {
+  using F = Fft2<C, false>;
+  using B = Fft2<C, true>;
+  float2 v[F::L1], u[F::L2];
+#pragma unroll
+  for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = z[n1];
   F::run(v, u, n2, x, tw);
-  if (n2 < F::L1) {
+  {
+    float2 r[F::L1];
+    bins_to_input<C>(u, v, r, n2, x);
 #pragma unroll
-    for (int k2 = 0; k2 < F::L2; ++k2) {
-      const float f = two_pi * kfreq<D>(n2 + F::L1 * k2) / (float)D;
-      u[k2] = make_float2(-f * u[k2].y, f * u[k2].x);
-    }
+    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = deriv_bin(v[n1], r[n1], F::L2 * n1 + n2, C, tw4);
   }
-  fft2_relayout<D>(u, v, n2, x);
   B::run(v, u, n2, x, tw);
+  fft2_relayout<C>(u, v, n2, x);
+#pragma unroll
+  for (int n1 = 0; n1 < F::L1; ++n1) g[n1] = v[n1].y * z[n1].x - v[n1].x * z[n1].y;
 }
 
-// Gradient along one line of the extension: at the outputs held by threads
-// n2 < L1 (positions n2 + L1*k2), g = (Im(dZ / Z) - Re(dphi_s)) / (2 pi),
-// Z = exp(i phi_s). `pos(i)` maps line position i to the (y, x) of the U
-// image; x is this line's exchange storage. The two derivatives run one
-// after the other so that only the real part of the first stays live.
-template <int D, class Pos, class X>
-__device__ __forceinline__ void line_gradient(const float2* __restrict__ iu_a, Pos pos, int n2,
-                                              X x, const float2* __restrict__ tw,
-                                              float (&g)[Fft2<D, false>::L2]) {
-  using F = Fft2<D, false>;
-  constexpr int C = D / 2;
-  const float two_pi = (float)(2.0 * 3.14159265358979323846);
-  float dphi[F::L2];
-  {
-    float2 v[F::L1], u[F::L2];
+// Column blocks: NC adjacent columns, 32 where that keeps the block within
+// MAXT threads and divides C, else 16 (the last block may run past C). The
+// gradient passes hold a line's phasors beside a transform: waves per SIMD
+// that leave them in registers (at 4 waves, crops of 160 to 256 spilled up to
+// 138 of them), in blocks of at most 256 threads so that 3 fit.
+template <int C, int MAXT>
+constexpr int unw_nc() {
+  return 32 * Fft2<C, false>::T <= MAXT && C % 32 == 0 ? 32 : 16;
+}
+template <int C, int MAXT>
+constexpr int unw_threads() {
+  return unw_nc<C, MAXT>() * Fft2<C, false>::T;
+}
+template <int C>
+constexpr int unw_waves() {
+  return C <= 128 ? 4 : C <= 256 ? 3 : 2;
+}
+constexpr int kUnwGrad = 256, kUnwOut = 512;  // thread caps of passes B and D
+
+// pass A: rows of the U frame, U[y][x] = IU[(y + C/2) % C][(x + C/2) % C]
+template <int C>
+__global__ void __launch_bounds__(256, unw_waves<C>())
+k_unw_gx(const float2* __restrict__ iu, const float2* __restrict__ tw,
+         const float2* __restrict__ tw4, float* __restrict__ gx) {
+  using F = Fft2<C, false>;
+  constexpr int NT = rows_nt<C>();
+  __shared__ float lds[NT * F::LDS_ROW];
+  const int2 ab = xcd_block();
+  const int a = ab.x, t = threadIdx.x / F::T, n2 = threadIdx.x % F::T;
+  const int y = ab.y * NT + t;
+  const float2* row = iu + ((size_t)a * C + (y + C / 2) % C) * C;
+  float2 z[F::L1];
 #pragma unroll
-    for (int n1 = 0; n1 < F::L1; ++n1) {
-      int y, xx;
-      pos(F::L2 * n1 + n2, y, xx);
-      v[n1] = make_float2(wrapped_phase<C>(iu_a, y, xx), 0.f);
-    }
-    line_derivative<D>(x, tw, n2, v, u);
+  for (int n1 = 0; n1 < F::L1; ++n1)
+    z[n1] = unit_phasor(row[(dct_src(F::L2 * n1 + n2, C) + C / 2) % C]);
+  float g[F::L1];
+  line_gradient<C>(z, g, n2, typename F::Row{lds + t * F::LDS_ROW}, tw, tw4);
+  float* o = gx + ((size_t)a * C + y) * C;
 #pragma unroll
-    for (int k2 = 0; k2 < F::L2; ++k2) dphi[k2] = u[k2].x;
+  for (int n1 = 0; n1 < F::L1; ++n1) {
+    const int m = F::L2 * n1 + n2;
+    o[dct_src(m, C)] = m < C / 2 ? g[n1] : -g[n1];
   }
-  __syncthreads();  // the exchange storage is reused
+}
+
+// pass B: columns; H[ky][x] = (DCT-II along y of gx, DST-II along y of gy)
+template <int C>
+__global__ void __launch_bounds__((unw_threads<C, kUnwGrad>()), unw_waves<C>())
+k_unw_gy(const float2* __restrict__ iu, const float* __restrict__ gx,
+         const float2* __restrict__ tw, const float2* __restrict__ tw4, float2* __restrict__ H) {
+  using F = Fft2<C, false>;
+  constexpr int NC = unw_nc<C, kUnwGrad>();
+  __shared__ float lds[NC * F::LDS_COL];
+  const int2 ab = xcd_block();
+  const int a = ab.x, cl = threadIdx.x % NC, n2 = threadIdx.x / NC;
+  const int c = ab.y * NC + cl;
+  const bool live = C % NC == 0 || c < C;
+  const int cc = live ? c : C - 1;
+  const typename F::template Col<NC> x{lds + cl};
+  const float2* col = iu + (size_t)a * C * C + (cc + C / 2) % C;
+  const float* gcol = gx + (size_t)a * C * C + cc;
+  float2 z[F::L1];
+#pragma unroll
+  for (int n1 = 0; n1 < F::L1; ++n1)
+    z[n1] = unit_phasor(col[(size_t)((dct_src(F::L2 * n1 + n2, C) + C / 2) % C) * C]);
+  float g[F::L1];
+  line_gradient<C>(z, g, n2, x, tw, tw4);
+  // gy's odd samples carry -1 twice: the derivative's and the DST's
+  float2 v[F::L1], u[F::L2];
+#pragma unroll
+  for (int n1 = 0; n1 < F::L1; ++n1)
+    v[n1] = make_float2(gcol[(size_t)dct_src(F::L2 * n1 + n2, C) * C], g[n1]);
+  F::run(v, u, n2, x, tw);
+  float2 r[F::L1];
+  bins_to_input<C>(u, v, r, n2, x);
+  if (!live) return;
+  float2* o = H + (size_t)a * C * C + c;
+#pragma unroll
+  for (int n1 = 0; n1 < F::L1; ++n1) {
+    const int k = F::L2 * n1 + n2;
+    const float2 e = tw4[k];
+    const float2 P = dct_p(v[n1], e), Q = dct_q(r[n1], e);
+    o[(size_t)k * C] = make_float2(0.5f * (P.x + Q.x), 0.5f * (P.x - Q.x));
+  }
+}
+
+// pass C: rows (ky); R[ky][x]
+template <int C>
+__global__ void __launch_bounds__(256, unw_waves<C>())
+k_unw_poisson(const float2* __restrict__ H, const float2* __restrict__ tw,
+              const float2* __restrict__ tw4, float* __restrict__ R) {
+  using F = Fft2<C, false>;
+  using B = Fft2<C, true>;
+  constexpr int NT = rows_nt<C>();
+  __shared__ float lds[NT * F::LDS_ROW];
+  const int2 ab = xcd_block();
+  const int a = ab.x, t = threadIdx.x / F::T, n2 = threadIdx.x % F::T;
+  const int ky = ab.y * NT + t;
+  const typename F::Row x{lds + t * F::LDS_ROW};
+  const float2* h = H + ((size_t)a * C + ky) * C;
   float2 v[F::L1], u[F::L2];
 #pragma unroll
   for (int n1 = 0; n1 < F::L1; ++n1) {
-    int y, xx;
-    pos(F::L2 * n1 + n2, y, xx);
-    float zs, zc;
-    sincosf(wrapped_phase<C>(iu_a, y, xx), &zs, &zc);
-    v[n1] = make_float2(zc, zs);
+    const int m = F::L2 * n1 + n2;
+    v[n1] = h[dct_src(m, C)];
+    if (m >= C / 2) v[n1].x = -v[n1].x;
   }
-  line_derivative<D>(x, tw, n2, v, u);
-  if (n2 < F::L1) {
+  F::run(v, u, n2, x, tw);
+  {
+    float2 r[F::L1];
+    bins_to_input<C>(u, v, r, n2, x);
 #pragma unroll
-    for (int k2 = 0; k2 < F::L2; ++k2) {
-      int y, xx;
-      pos(n2 + F::L1 * k2, y, xx);
-      float zi, zr;
-      sincosf(wrapped_phase<C>(iu_a, y, xx), &zi, &zr);
-      // -i (dZ / Z): its real part is Im(dZ / Z)
-      const float2 dz = u[k2];
-      const float im_q = (dz.y * zr - dz.x * zi) / (zr * zr + zi * zi);
-      g[k2] = (im_q - dphi[k2]) / two_pi;
+    for (int n1 = 0; n1 < F::L1; ++n1) {
+      const int k = F::L2 * n1 + n2;
+      const float2 e = tw4[k];
+      v[n1] = poisson_bin(dct_p(v[n1], e), dct_q(r[n1], e), e, k, ky, C);
     }
   }
-}
-
-// rows of the extension: gx[a][r][c]
-template <int C>
-__global__ void __launch_bounds__(256)
-k_grad_rows(const float2* __restrict__ iu, const float2* __restrict__ tw, float* __restrict__ gx) {
-  constexpr int D = 2 * C;
-  using F = Fft2<D, false>;
-  constexpr int NT = rows_nt<D>();
-  __shared__ float lds[NT * F::LDS_ROW];
-  const int2 ab = xcd_block();
-  const int a = ab.x;
-  const int t = threadIdx.x / F::T, n2 = threadIdx.x % F::T;
-  const int r = ab.y * NT + t;
-  const float2* iu_a = iu + (size_t)a * C * C;
-  const int ys = mirror_src<C>(r);
-  auto pos = [ys](int i, int& y, int& x) { y = ys; x = mirror_src<C>(i); };
-  float g[F::L2];
-  line_gradient<D>(iu_a, pos, n2, typename F::Row{lds + t * F::LDS_ROW}, tw, g);
+  B::run(v, u, n2, x, tw);
   if (n2 < F::L1) {
-    float* o = gx + ((size_t)a * D + r) * D;
+    float* o = R + ((size_t)a * C + ky) * C;
 #pragma unroll
-    for (int k2 = 0; k2 < F::L2; ++k2) o[n2 + F::L1 * k2] = g[k2];
+    for (int k2 = 0; k2 < F::L2; ++k2) o[dct_src(n2 + F::L1 * k2, C)] = u[k2].x;
   }
 }
 
-// columns per block of the gradient kernels: two transforms' registers
-// are live, so at most 256 threads
-template <int D>
-constexpr int grad_nc() {
-  constexpr int by_thr = 256 / Fft2<D, false>::T;
-  constexpr int by_lds = kLdsBlockMax / (Fft2<D, false>::LDS_COL * 4);
-  return divisor_le(D, by_thr < by_lds ? by_thr : by_lds);
-}
-
-// columns of the extension: gy[a][r][c]; NC adjacent columns per block
+// pass D: pairs of columns; the phase phu[y][x] of the U frame
 template <int C>
-__global__ void __launch_bounds__(256)
-k_grad_cols(const float2* __restrict__ iu, const float2* __restrict__ tw, float* __restrict__ gy) {
-  constexpr int D = 2 * C;
-  using F = Fft2<D, false>;
-  constexpr int NC = grad_nc<D>();
+__global__ void __launch_bounds__((unw_threads<C, kUnwOut>()), 4)
+k_unw_out(const float* __restrict__ R, const float2* __restrict__ tw,
+          const float2* __restrict__ tw4, float* __restrict__ phu) {
+  using F = Fft2<C, true>;
+  constexpr int NC = unw_nc<C, kUnwOut>();
   __shared__ float lds[NC * F::LDS_COL];
   const int2 ab = xcd_block();
-  const int a = ab.x;
-  const int cl = threadIdx.x % NC, n2 = threadIdx.x / NC;
-  const int c = ab.y * NC + cl;
-  const float2* iu_a = iu + (size_t)a * C * C;
-  const int xs = mirror_src<C>(c);
-  auto pos = [xs](int i, int& y, int& x) { y = mirror_src<C>(i); x = xs; };
-  float g[F::L2];
-  line_gradient<D>(iu_a, pos, n2, typename F::template Col<NC>{lds + cl}, tw, g);
-  if (n2 < F::L1) {
-    float* o = gy + (size_t)a * D * D + c;
+  const int a = ab.x, cl = threadIdx.x % NC, n2 = threadIdx.x / NC;
+  const int c = ab.y * NC + cl;  // columns 2c, 2c + 1
+  const bool live = c < C / 2;
+  const float2* q = (const float2*)(R + (size_t)a * C * C) + (live ? c : 0);
+  float2 v[F::L1], u[F::L2];
 #pragma unroll
-    for (int k2 = 0; k2 < F::L2; ++k2) o[(size_t)(n2 + F::L1 * k2) * D] = g[k2];
+  for (int n1 = 0; n1 < F::L1; ++n1) {
+    const int k = F::L2 * n1 + n2;
+    const float2 y0 = q[(size_t)k * (C / 2)];
+    const float2 y1 = k ? q[(size_t)(C - k) * (C / 2)] : make_float2(0.f, 0.f);
+    v[n1] = dct_q(make_float2(y0.x + y1.y, y0.y - y1.x), tw4[k]);
   }
+  F::run(v, u, n2, typename F::template Col<NC>{lds + cl}, tw);
+  if (!live || n2 >= F::L1) return;
+  float2* o = (float2*)(phu + (size_t)a * C * C) + c;
+#pragma unroll
+  for (int k2 = 0; k2 < F::L2; ++k2)
+    o[(size_t)dct_src(n2 + F::L1 * k2, C) * (C / 2)] = u[k2];
 }
 
-// integration pass 1: rows of gx + i gy, forward
-template <int DT>
-struct PackRowOp {
-  const float* gx;
-  const float* gy;
-  float2* out;
-  const float2* tw;
-  __device__ void begin(int) {}
-  __device__ float2 load(int a, int r, int c) const {
-    const size_t i = ((size_t)a * D + r) * D + c;
-    return make_float2(gx[i], gy[i]);
-  }
-  __device__ void store(int a, int r, int k, float2 v) const { out[((size_t)a * D + r) * D + k] = v; }
-  Dim<DT> D{};
-};
-
-// integration pass 2: columns, forward, in place
-template <int DT>
-struct InPlaceColOp {
-  float2* buf;
-  const float2* tw;
-  __device__ void begin(int) {}
-  __device__ float2 load(int a, int c, int r) const { return buf[((size_t)a * D + r) * D + c]; }
-  __device__ void store(int a, int c, int r, float2 v) const { buf[((size_t)a * D + r) * D + c] = v; }
-  Dim<DT> D{};
-};
-
-// integration pass 3: P = FFT2(gx + i gy) (unnormalised). Per frequency,
-// TFx = (P[k] + conj(P[-k])) / (2 D^2), TFy = (P[k] - conj(P[-k])) / (2i D^2),
-// T = -i (TFx kx + TFy ky) / (2 pi |k|^2), T[0] = 0; backward along rows,
-// keeping x in [C, 2C): Q[a][ky][x - C].
-template <int DT>
-struct PoissonRowOp {
-  const float2* P;
-  float2* Q;
-  const float2* tw;
-  __device__ void begin(int) {}
-  __device__ float2 load(int a, int ky, int kx) const {
-    if (ky == 0 && kx == 0) return make_float2(0.f, 0.f);
-    const float2* Pa = P + (size_t)a * D * D;
-    const float2 p = Pa[(size_t)ky * D + kx];
-    const float2 m = Pa[(size_t)((D - ky) % D) * D + (D - kx) % D];
-    const float inv = 1.0f / (2.0f * (float)D * (float)D);
-    // TFx = (p + conj(m)) * inv, TFy = (p - conj(m)) * inv / i
-    const float2 fx = make_float2((p.x + m.x) * inv, (p.y - m.y) * inv);
-    const float2 fy = make_float2((p.y + m.y) * inv, -(p.x - m.x) * inv);
-    const float kxf = kfreq(kx, D), kyf = kfreq(ky, D);
-    const float2 num = make_float2(fx.x * kxf + fy.x * kyf, fx.y * kxf + fy.y * kyf);
-    const float den = (float)(2.0 * 3.14159265358979323846) * (kxf * kxf + kyf * kyf);
-    return make_float2(num.y / den, -num.x / den);  // -i num / den
-  }
-  __device__ void store(int a, int ky, int x, float2 v) const {
-    const int C = D / 2;
-    if (x >= C) Q[((size_t)a * D + ky) * C + (x - C)] = v;
-  }
-  Dim<DT> D{};
-};
-
-// integration pass 4: backward along columns of Q, keeping y in [C, 2C);
-// unwrapped phase = phi + 2 pi Re(.), in the U frame: phu[a][y][x]
-template <int DT>
-struct UnwrapColOp {
-  const float2* Q;
-  const float2* iu;
-  float* phu;
-  const float2* tw;
-  __device__ void begin(int) {}
-  __device__ float2 load(int a, int c, int ky) const {
-    const int C = D / 2;
-    if (c >= C) return make_float2(0.f, 0.f);
-    return Q[((size_t)a * D + ky) * C + c];
-  }
-  __device__ void store(int a, int c, int y, float2 v) const {
-    const int C = D / 2;
-    if (c >= C || y < C) return;
-    const int yy = y - C;
-    const float ph = wrapped_phase(iu + (size_t)a * C * C, yy, c, C);
-    phu[((size_t)a * C + yy) * C + c] = ph + (float)(2.0 * 3.14159265358979323846) * v.x;
-  }
-  Dim<DT> D{};
-};
-
 template <int C>
-static hipError_t unwrap_c(const float2* iu, int A, const float2* tw, float* gx, float* gy,
-                           float2* P, float2* Q, float* phu, hipStream_t s) {
-  constexpr int D = 2 * C;
+static hipError_t unwrap_c(const float2* iu, int A, const float2* tw, const float2* tw4,
+                           float* gx, float2* H, float* phu, hipStream_t s) {
+  constexpr int NB = unw_nc<C, kUnwGrad>(), ND = unw_nc<C, kUnwOut>();
   {
-    Timed tm("unwrap_grad", s);
-    hipLaunchKernelGGL((k_grad_rows<C>), rows_grid<D>(A), rows_block<D>(), 0, s, iu, tw, gx);
-    constexpr int GNC = grad_nc<D>();
-    hipLaunchKernelGGL((k_grad_cols<C>), dim3(D / GNC, A), dim3(GNC * Fft2<D, false>::T), 0, s,
-                       iu, tw, gy);
+    Timed tm("unwrap_gx", s);
+    hipLaunchKernelGGL((k_unw_gx<C>), rows_grid<C>(A), rows_block<C>(), 0, s, iu, tw, tw4, gx);
   }
   {
-    Timed tm("unwrap_fwd", s);
-    PackRowOp<D> r{gx, gy, P, tw};
-    hipLaunchKernelGGL((k_rows<D, false, PackRowOp<D>>), rows_grid<D>(A), rows_block<D>(), 0, s, r);
-    InPlaceColOp<D> c{P, tw};
-    hipLaunchKernelGGL((k_cols<D, false, InPlaceColOp<D>>), cols_grid<D>(A), cols_block<D>(), 0,
-                       s, c);
+    Timed tm("unwrap_gy", s);
+    hipLaunchKernelGGL((k_unw_gy<C>), dim3((C + NB - 1) / NB, A),
+                       dim3((unw_threads<C, kUnwGrad>())), 0, s, iu, gx, tw, tw4, H);
   }
-  Timed tm("unwrap_inv", s);
-  PoissonRowOp<D> pr{P, Q, tw};
-  hipLaunchKernelGGL((k_rows<D, true, PoissonRowOp<D>>), rows_grid<D>(A), rows_block<D>(), 0, s,
-                     pr);
-  // only the C columns of Q: ceil(C / NC) column groups
-  constexpr int NC = cols_nc<D>();
-  UnwrapColOp<D> uc{Q, iu, phu, tw};
-  hipLaunchKernelGGL((k_cols<D, true, UnwrapColOp<D>>), dim3((C + NC - 1) / NC, A),
-                     cols_block<D>(), 0, s, uc);
+  {
+    Timed tm("unwrap_poisson", s);
+    hipLaunchKernelGGL((k_unw_poisson<C>), rows_grid<C>(A), rows_block<C>(), 0, s, H, tw, tw4, gx);
+  }
+  Timed tm("unwrap_out", s);
+  hipLaunchKernelGGL((k_unw_out<C>), dim3((C / 2 + ND - 1) / ND, A),
+                     dim3((unw_threads<C, kUnwOut>())), 0, s, gx, tw, tw4, phu);
   return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// Crop sides without compiled 2C-point FFTs: the same four steps with the
-// runtime-length FFTs. The gradient kernel holds nl lines of the extension
-// in LDS and runs both derivatives there (forward transform, times
-// 2 pi i k / D^2, backward transform); the first derivative's real part goes
-// to the output array and is read back by the same thread for the second.
+// Crop sides without a compiled C-point FFT: the same four passes with the
+// runtime-length FFTs, nl lines in LDS per block (gen_fft.hpp), a line's
+// positions reordered on load.
 // ---------------------------------------------------------------------------
-template <bool ROWS>
-__global__ void __launch_bounds__(kGenThreads)
-k_grad_gen(const float2* __restrict__ iu, GenPlan p, int C, float* __restrict__ g, int nl) {
-  extern __shared__ float2 gen_lds[];
-  const int D = 2 * C;
-  const int a = blockIdx.y, line0 = blockIdx.x * nl;
-  const int nact = min(nl, D - line0);
-  float2* A = gen_lds;
-  float2* B = gen_lds + (size_t)nl * p.W;
-  const float2* iu_a = iu + (size_t)a * C * C;
-  const float two_pi = (float)(2.0 * 3.14159265358979323846);
-  auto at = [&](int t, int& l, int& i) {
-    if (ROWS) { l = t / D; i = t - l * D; } else { i = t / nl; l = t - i * nl; }
-  };
-  auto phase = [&](int l, int i) {
-    const int line = line0 + l;
-    return ROWS ? wrapped_phase(iu_a, mirror_src(line, C), mirror_src(i, C), C)
-                : wrapped_phase(iu_a, mirror_src(i, C), mirror_src(line, C), C);
-  };
-  auto out = [&](int l, int i) -> size_t {
-    return ROWS ? ((size_t)a * D + line0 + l) * D + i : ((size_t)a * D + i) * D + line0 + l;
-  };
-  for (int pass = 0; pass < 2; ++pass) {  // 0: phi_s, 1: Z = exp(i phi_s)
-    for (int t = threadIdx.x; t < nl * D; t += blockDim.x) {
-      int l, i;
-      at(t, l, i);
-      float2 v = make_float2(0.f, 0.f);
-      if (l < nact) {
-        const float ph = phase(l, i);
-        if (pass == 0) {
-          v.x = ph;
-        } else {
-          sincosf(ph, &v.y, &v.x);
-        }
-      }
-      A[l * p.W + i] = v;
-    }
-    __syncthreads();
-    float2* R = gen_fft<false>(A, B, nl, p);
-    for (int t = threadIdx.x; t < nl * D; t += blockDim.x) {
-      const int l = t / D, k = t - l * D;
-      const float f = two_pi * kfreq(k, D) / (float)D;
-      const float2 u = R[l * p.W + k];
-      R[l * p.W + k] = make_float2(-f * u.y, f * u.x);
-    }
-    __syncthreads();
-    const float2* R2 = gen_fft<true>(R, R == A ? B : A, nl, p);
-    for (int t = threadIdx.x; t < nl * D; t += blockDim.x) {
-      int l, i;
-      at(t, l, i);
-      if (l >= nact) continue;
-      if (pass == 0) {
-        g[out(l, i)] = R2[l * p.W + i].x;  // d phi_s
-      } else {
-        float zi, zr;
-        sincosf(phase(l, i), &zi, &zr);
-        const float2 dz = R2[l * p.W + i];
-        const float im_q = (dz.y * zr - dz.x * zi) / (zr * zr + zi * zi);
-        const size_t o = out(l, i);
-        g[o] = (im_q - g[o]) / two_pi;
-      }
-    }
-    __syncthreads();  // A and B are reused
+// this thread's elements (line l of the block, position i) of nl lines: rows
+// run along the lines, columns across them
+template <bool ROWS, class Fn>
+__device__ __forceinline__ void gen_each(int nl, int C, Fn&& fn) {
+  for (int t = threadIdx.x; t < nl * C; t += blockDim.x) {
+    int l, i;
+    if (ROWS) { l = t / C; i = t - l * C; } else { i = t / nl; l = t - i * nl; }
+    fn(l, i);
   }
 }
 
-static hipError_t unwrap_gen(int C, const float2* iu, int A, const GenPlan& p, float* gx,
-                             float* gy, float2* P, float2* Q, float* phu, hipStream_t s) {
-  const int D = 2 * C;
-  const Dim<0> d(D);
-  {
-    Timed tm("unwrap_grad", s);
-    const int nl = gen_lines_per_block(p.W);
-    const size_t lds = (size_t)2 * nl * p.W * sizeof(float2);
-    const dim3 grid((D + nl - 1) / nl, A);
-    hipLaunchKernelGGL((k_grad_gen<true>), grid, dim3(kGenThreads), lds, s, iu, p, C, gx, nl);
-    hipLaunchKernelGGL((k_grad_gen<false>), grid, dim3(kGenThreads), lds, s, iu, p, C, gy, nl);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+// Pair pass over bins k and C - k of each line, in place: fn(k, V[k], V[C-k])
+// gives both bins' new values (k = 0 and C/2 are their own mirrors).
+template <class Fn>
+__device__ __forceinline__ void gen_pairs(float2* R, int nl, int W, int C, Fn&& fn) {
+  const int h = C / 2 + 1;
+  for (int t = threadIdx.x; t < nl * h; t += blockDim.x) {
+    const int l = t / h, k = t - l * h, m = k ? C - k : 0;
+    float2* r = R + l * W;
+    const float2 a = r[k], b = r[m];
+    r[k] = fn(l, k, a, b);
+    if (m != k) r[m] = fn(l, m, b, a);
   }
-  hipError_t e;
-  {
-    Timed tm("unwrap_fwd", s);
-    e = launch_gen<false, true>(PackRowOp<0>{gx, gy, P, nullptr, d}, p, D, A, s);
-    if (e == hipSuccess) e = launch_gen<false, false>(InPlaceColOp<0>{P, nullptr, d}, p, D, A, s);
+  __syncthreads();
+}
+
+template <bool ROWS>
+__global__ void __launch_bounds__(kGenThreads)
+k_unw_grad_gen(const float2* __restrict__ iu, GenPlan p, int C, const float2* __restrict__ tw4,
+               float* __restrict__ gx, float2* __restrict__ H, int nl) {
+  extern __shared__ float2 gen_lds[];
+  const int a = blockIdx.y, line0 = blockIdx.x * nl;
+  const int nact = min(nl, C - line0);
+  float2* A = gen_lds;
+  float2* B = gen_lds + (size_t)nl * p.W;
+  const float2* iu_a = iu + (size_t)a * C * C;
+  const size_t base = (size_t)a * C * C;
+  auto phasor = [&](int l, int m) {
+    const int i = (dct_src(m, C) + C / 2) % C, j = (line0 + l + C / 2) % C;
+    return unit_phasor(ROWS ? iu_a[(size_t)j * C + i] : iu_a[(size_t)i * C + j]);
+  };
+  gen_each<ROWS>(nl, C, [&](int l, int m) {
+    A[l * p.W + m] = l < nact ? phasor(l, m) : make_float2(0.f, 0.f);
+  });
+  __syncthreads();
+  float2* R = gen_fft<false>(A, B, nl, p);
+  gen_pairs(R, nl, p.W, C,
+            [&](int, int k, float2 V, float2 Vr) { return deriv_bin(V, Vr, k, C, tw4); });
+  float2* D = gen_fft<true>(R, R == A ? B : A, nl, p);
+  gen_each<ROWS>(nl, C, [&](int l, int m) {
+    if (l >= nact) return;
+    const float2 w = D[l * p.W + m], z = phasor(l, m);
+    const float g = w.y * z.x - w.x * z.y;
+    const int n = dct_src(m, C);
+    if (ROWS) gx[base + (size_t)(line0 + l) * C + n] = m < C / 2 ? g : -g;
+    else D[l * p.W + m] = make_float2(gx[base + (size_t)n * C + line0 + l], g);
+  });
+  if (ROWS) return;  // uniform
+  __syncthreads();
+  R = gen_fft<false>(D, D == A ? B : A, nl, p);
+  gen_pairs(R, nl, p.W, C, [&](int, int k, float2 V, float2 Vr) {
+    const float2 e = tw4[k], P = dct_p(V, e), Q = dct_q(Vr, e);
+    return make_float2(0.5f * (P.x + Q.x), 0.5f * (P.x - Q.x));
+  });
+  gen_each<ROWS>(nl, C, [&](int l, int k) {
+    if (l < nact) H[base + (size_t)k * C + line0 + l] = R[l * p.W + k];
+  });
+}
+
+__global__ void __launch_bounds__(kGenThreads)
+k_unw_poisson_gen(const float2* __restrict__ H, GenPlan p, int C, const float2* __restrict__ tw4,
+                  float* __restrict__ out, int nl) {
+  extern __shared__ float2 gen_lds[];
+  const int a = blockIdx.y, line0 = blockIdx.x * nl;
+  const int nact = min(nl, C - line0);
+  float2* A = gen_lds;
+  float2* B = gen_lds + (size_t)nl * p.W;
+  const size_t base = ((size_t)a * C + line0) * C;
+  gen_each<true>(nl, C, [&](int l, int m) {
+    float2 v = make_float2(0.f, 0.f);
+    if (l < nact) v = H[base + (size_t)l * C + dct_src(m, C)];
+    A[l * p.W + m] = make_float2(m < C / 2 ? v.x : -v.x, v.y);
+  });
+  __syncthreads();
+  float2* R = gen_fft<false>(A, B, nl, p);
+  gen_pairs(R, nl, p.W, C, [&](int l, int k, float2 V, float2 Vr) {
+    const float2 e = tw4[k];
+    return poisson_bin(dct_p(V, e), dct_q(Vr, e), e, k, line0 + l, C);
+  });
+  const float2* D = gen_fft<true>(R, R == A ? B : A, nl, p);
+  gen_each<true>(nl, C, [&](int l, int m) {
+    if (l < nact) out[base + (size_t)l * C + dct_src(m, C)] = D[l * p.W + m].x;
+  });
+}
+
+struct UnwOutGenOp {  // pairs of columns (2 col, 2 col + 1)
+  const float* R;
+  const float2* tw4;
+  float* phu;
+  int C;
+  __device__ void begin(int) {}
+  __device__ float2 load(int a, int col, int k) const {
+    const float2* q = (const float2*)(R + (size_t)a * C * C) + col;
+    const float2 y0 = q[(size_t)k * (C / 2)];
+    const float2 y1 = k ? q[(size_t)(C - k) * (C / 2)] : make_float2(0.f, 0.f);
+    return dct_q(make_float2(y0.x + y1.y, y0.y - y1.x), tw4[k]);
   }
+  __device__ void store(int a, int col, int m, float2 v) const {
+    ((float2*)(phu + (size_t)a * C * C))[(size_t)dct_src(m, C) * (C / 2) + col] = v;
+  }
+};
+
+static hipError_t unwrap_gen(int C, const float2* iu, int A, const GenPlan& p, const float2* tw4,
+                             float* gx, float2* H, float* phu, hipStream_t s) {
+  const int nl = gen_lines_per_block(p.W);
+  const size_t lds = (size_t)2 * nl * p.W * sizeof(float2);
+  const dim3 grid((C + nl - 1) / nl, A), block(kGenThreads);
+  {
+    Timed tm("unwrap_gx", s);
+    hipLaunchKernelGGL((k_unw_grad_gen<true>), grid, block, lds, s, iu, p, C, tw4, gx, H, nl);
+  }
+  {
+    Timed tm("unwrap_gy", s);
+    hipLaunchKernelGGL((k_unw_grad_gen<false>), grid, block, lds, s, iu, p, C, tw4, gx, H, nl);
+  }
+  {
+    Timed tm("unwrap_poisson", s);
+    hipLaunchKernelGGL(k_unw_poisson_gen, grid, block, lds, s, H, p, C, tw4, gx, nl);
+  }
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  Timed tm("unwrap_inv", s);
-  e = launch_gen<true, true>(PoissonRowOp<0>{P, Q, nullptr, d}, p, D, A, s);
-  if (e != hipSuccess) return e;
-  return launch_gen<true, false>(UnwrapColOp<0>{Q, iu, phu, nullptr, d}, p, C, A, s);
+  Timed tm("unwrap_out", s);
+  return launch_gen<true, false>(UnwOutGenOp{gx, tw4, phu, C}, p, C / 2, A, s);
 }
 
 #define MTD_UNWRAP_SIZES(X) \
   X(16) X(32) X(64) X(128) X(160) X(192) X(224) X(250) X(256) X(288) X(320) X(352) X(384) \
   X(512)
 
-hipError_t launch_unwrap(int C, const float2* iu, int A, const FftTab& ft2C, float* gx,
-                         float* gy, float2* P, float2* Q, float* phu, hipStream_t s) {
+hipError_t launch_unwrap(int C, const float2* iu, int A, const FftTab& ftC, const float2* tw4,
+                         void* scratch, float* phu, hipStream_t s) {
+  if (A <= 0) return hipSuccess;
+  float2* H = (float2*)scratch;
+  float* gx = (float*)(H + (size_t)A * C * C);
   switch (C) {
-#define X(n) case n: return unwrap_c<n>(iu, A, ft2C.tw, gx, gy, P, Q, phu, s);
+#define X(n) case n: return unwrap_c<n>(iu, A, ftC.tw, tw4, gx, H, phu, s);
     MTD_UNWRAP_SIZES(X)
 #undef X
   }
-  if (!ft2C.gen) return hipErrorInvalidValue;
-  return unwrap_gen(C, iu, A, *ft2C.gen, gx, gy, P, Q, phu, s);
+  if (!ftC.gen) return hipErrorInvalidValue;
+  return unwrap_gen(C, iu, A, *ftC.gen, tw4, gx, H, phu, s);
 }
 
 bool unwrap_len_supported(int C) {
@@ -428,9 +508,8 @@ bool unwrap_len_supported(int C) {
 }
 
 size_t unwrap_scratch_bytes(int C, int A) {
-  const size_t D = 2 * (size_t)C, n = (size_t)(A > 0 ? A : 1);
-  // gx, gy (float D^2), P (float2 D^2), Q (float2 D*C)
-  return n * (2 * D * D * sizeof(float) + D * D * sizeof(float2) + D * C * sizeof(float2));
+  // H (float2), gx, then the integral's rows (float), C^2 each
+  return (size_t)(A > 0 ? A : 1) * C * C * (sizeof(float2) + sizeof(float));
 }
 
 }  // namespace mtd

@@ -689,18 +689,12 @@ static int front_chunk(mtd_ctx* ctx, const mtd_geom* g, const float2* crop, int 
   // reference only unwraps when the aberration correction runs (main.cpp:253-277)
   float* phu = nullptr;
   if (g->c_aber && g->deroul == MTD_DEROUL_VOLKOV) {
-    FftTab tw2;
-    const bool tabs2 = fft_tab(ctx, 2 * C, unwrap_len_supported(C), &tw2);
+    const float2* tw4 = twiddle(ctx, 4 * C);
     phu = (float*)ws_get(ctx, WS_PHU, (size_t)n * C * C * sizeof(float));
-    char* us = (char*)ws_get(ctx, WS_UNWRAP, unwrap_scratch_bytes(C, n));
-    if (!tabs2 || !phu || !us)
+    void* us = ws_get(ctx, WS_UNWRAP, unwrap_scratch_bytes(C, n));
+    if (!tw4 || !phu || !us)
       return set_err(ctx, MTD_ERR_HIP, "out of device memory (unwrapping)");
-    const size_t D2 = (size_t)4 * C * C * n;  // (2C)^2 per angle
-    float* gx = (float*)us;
-    float* gy = gx + D2;
-    float2* P = (float2*)(gy + D2);
-    float2* Q = P + D2;
-    MTD_TRY(hip_check(ctx, launch_unwrap(C, iu, n, tw2, gx, gy, P, Q, phu, ctx->stream),
+    MTD_TRY(hip_check(ctx, launch_unwrap(C, iu, n, twC, tw4, us, phu, ctx->stream),
                       "phase unwrapping"));
   } else if (g->c_aber && g->deroul == MTD_DEROUL_HERRAEZ) {
     const float* border = herraez_border_table(ctx, C, a0, n);
