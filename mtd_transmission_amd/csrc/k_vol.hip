@@ -63,6 +63,7 @@ struct GatherArgs {
   int r2max;            // largest r2 inside the pupil
   float2* vol;
   int32_t* cnt;
+  uint32_t specb;       // bytes of all spectra if below 2 GiB, else 0
 };
 
 constexpr int GT = 16;  // tile side (columns per block = 256)
@@ -94,26 +95,6 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? l
 // h(r2) = sqrt(R^2 - r2) for 0 <= r2 <= R^2: IEEE sqrt of the same exact
 // double, so the host height table's value bit for bit
 __device__ __forceinline__ double height(double R2, int r2) { return sqrt(R2 - (double)r2); }
-
-// Height offset round(h(r2) - fz) of a hit (before + V/2), as the reference
-// computes it: FP64, round half away from zero. First in FP32: with R^2 <
-// 2^24, R^2 - r2 is an exact float; the hardware square root (v_sqrt_f32,
-// within 1 ulp, not correctly rounded) of it is within 1 ulp(R), fz32 is fz
-// rounded once and the difference is rounded once, each within half an ulp
-// of R (h, fz and |h - fz| are at most R): the FP32 difference is within
-// 2 ulp(R) of the FP64 one. Wherever the fractional part of |difference| is
-// farther than thr = 8 ulp(R) from 1/2 both round alike; near 1/2 (*near is
-// set) the caller takes the FP64 path.
-__device__ __forceinline__ int height_off_f32(float R2f, int r2, float fz32, float thr,
-                                              bool* near) {
-  const float d = __builtin_amdgcn_sqrtf(R2f - (float)r2) - fz32;
-  const float ad = fabsf(d);
-  const float fl = floorf(ad);
-  const float fr = ad - fl;  // exact (Sterbenz)
-  *near = fabsf(fr - 0.5f) < thr;
-  const int zr = (int)fl + (fr >= 0.5f ? 1 : 0);
-  return d < 0.f ? -zr : zr;
-}
 
 // Does angle a's pupil disc touch the 16x16 column tile at (qx0, qy0)? If so,
 // the nearest and farthest pupil radii^2 of the tile box (the farthest
@@ -175,92 +156,154 @@ k_tile_angles(GatherArgs g, int ntx, TileEntry* __restrict__ list, int4* __restr
   if (lane == 0) tinfo[tile] = make_int4(off, zmin, zmax, 0);
 }
 
-// 8 bytes of a spectrum at byte offset off from base; an offset past nbytes
-// returns zeros without a memory access (a buffer load's range check)
-__device__ __forceinline__ float2 load_or_zero(const float2* base, uint32_t nbytes, uint32_t off) {
+// 8 bytes at byte offset off + uni (uni uniform) from base; an offset past
+// nbytes returns zeros without a memory access (a buffer load's range check)
+__device__ __forceinline__ float2 load_or_zero(const float2* base, uint32_t nbytes, uint32_t off,
+                                               uint32_t uni = 0) {
   const __amdgpu_buffer_rsrc_t r =
       __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)nbytes, 0x00020000);
-  const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+  const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, (int)uni, 0);
   return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
+}
+__device__ __forceinline__ float load_or_zero(const float* base, uint32_t nbytes, uint32_t off) {
+  const __amdgpu_buffer_rsrc_t r =
+      __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)nbytes, 0x00020000);
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
 }
 constexpr uint32_t kMissOffset = 0x80000000u;  // past every spectrum (< 2^31 bytes)
 
-// one column's fixed data for the gather's hit tests
+// one column's fixed data for the gather's hit tests; lengths in FP32 are exact
+// integers (R^2 < 2^24: rayon is below half the volume side)
 struct GatherCol {
-  int qx, qy;       // lateral column (voxel - V/2)
-  int zbase;        // the window's first height - V/2
-  uint32_t fixed;   // byte offset of the column's element in the unshifted frame
-  float R2f, thr;   // R^2 in FP32 and the FP32 height path's margin
-  double R2;
+  float qx, qy;    // lateral column (voxel - V/2)
+  int zbase;       // the window's first height - V/2
+  uint32_t fixed;  // byte offset of the column's element in the unshifted frame
+  float R2f;       // R^2
+  float xmin;      // R^2 - r2max: the smallest R^2 - |fd|^2 inside the pupil
+  float half;      // 1/2 - 4 ulp(R) (see gather_fill)
+  bool square;     // the pupil reaches past the crop's square: test that too
 };
 
 // A batch of KB list entries: per entry the window slot of this column's hit
-// (-1: none), the angle, the spectrum element's byte offset (kMissOffset for
-// a miss) and, after issue(), the loaded value (and beta when !PRE).
+// (ZW, a slot of its own, for a miss), the angle and the spectrum element's
+// byte offset (kMissOffset for a miss: such a load fetches nothing and gives
+// zeros) and, after issue(), the loaded value (and beta when !PRE).
 template <int KB>
 struct GBatch {
   int kv[KB], ea[KB];
-  uint32_t el[KB];
+  uint32_t el[KB], br[KB];
   float2 sp[KB];
   float b[KB];
+  template <bool PRE>
   __device__ __forceinline__ void issue(const GatherArgs& g, size_t C2, uint32_t C2b) {
+    // spectra below 2 GiB in all: one buffer view, the angle in the scalar
+    // offset (a view per angle costs a dozen scalar instructions a load)
+    if (g.specb) {
 #pragma unroll
-    for (int t = 0; t < KB; ++t) sp[t] = load_or_zero(g.spec + (size_t)ea[t] * C2, C2b, el[t]);
+      for (int t = 0; t < KB; ++t)
+        sp[t] = load_or_zero(g.spec, g.specb, el[t], (uint32_t)ea[t] * C2b);
+    } else {
+#pragma unroll
+      for (int t = 0; t < KB; ++t) sp[t] = load_or_zero(g.spec + (size_t)ea[t] * C2, C2b, el[t]);
+    }
+    if constexpr (!PRE) {
+#pragma unroll
+      for (int t = 0; t < KB; ++t)
+        b[t] = load_or_zero(g.beta, (uint32_t)(g.r2max + 1) * 4u, br[t]);
+    }
     // keep the loads ahead of what follows (the other batch's sums): the
     // scheduler would otherwise sink them below those independent LDS ops
     __builtin_amdgcn_sched_barrier(0);
   }
-  // Only hits update their LDS slot (a lane-masked read-modify-write: the
-  // misses of a wave move no LDS data); the loads were issued before the
-  // scheduling barrier in issue(), so the branch cannot sink them.
-  template <bool PRE, int ZW>
-  __device__ __forceinline__ void apply(float2 (&acc)[ZW][256], unsigned short (&cn)[ZW][256],
-                                        int tid) const {
+  // The sums, four entries at a time: the four slots' old values are read
+  // together, an entry whose slot an earlier one of the four also hits takes
+  // that one's new sum instead (each voxel's sum still takes its hits in
+  // angle order), and the new sums are written in order. One wait for LDS per
+  // four entries instead of one per hit; groups without a hit in the wave
+  // are skipped. Counts: one LDS add per entry, two 16-bit counts a word.
+  template <bool PRE, bool COUNT, int ZW>
+  __device__ __forceinline__ void apply(float2 (*acc)[256], unsigned (*cn)[256], int tid) const {
 #pragma clang fp contract(off)
 #pragma unroll
-    for (int t = 0; t < KB; ++t) {
-      if (kv[t] >= 0) {
-        const int kc = kv[t];
+    for (int q = 0; q < KB; q += 4) {
+      if (!__any((kv[q] < ZW) | (kv[q + 1] < ZW) | (kv[q + 2] < ZW) | (kv[q + 3] < ZW))) continue;
+      float2 s[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] = acc[kv[q + i]][tid];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < i; ++j)
+          if (kv[q + i] == kv[q + j]) s[i] = s[j];
         // value (-b Si, b Sr)
-        const float pim = PRE ? sp[t].y : b[t] * sp[t].y;
-        const float pre = PRE ? sp[t].x : b[t] * sp[t].x;
-        float2 s = acc[kc][tid];
-        s.x = s.x + -pim;
-        s.y = s.y + pre;
-        acc[kc][tid] = s;
-        cn[kc][tid] = (unsigned short)(cn[kc][tid] + 1);
+        const float pim = PRE ? sp[q + i].y : b[q + i] * sp[q + i].y;
+        const float pre = PRE ? sp[q + i].x : b[q + i] * sp[q + i].x;
+        s[i].x = s[i].x + -pim;
+        s[i].y = s[i].y + pre;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc[kv[q + i]][tid] = s[i];
+        if constexpr (COUNT)
+          __hip_atomic_fetch_add(&cn[kv[q + i] >> 1][tid], 1u << ((kv[q + i] & 1) * 16),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
       }
     }
   }
 };
 
-// Batch bi of a segment's compacted entries (seg[0 .. total), angle order):
-// entries i0 .. i0 + KB - 1, those past total miss (angle 0, no load). The
-// entries are read from LDS at a uniform address (a broadcast).
-template <int ZW, bool PRE, int KB>
-__device__ __forceinline__ void gather_fill(GBatch<KB>& B, const int4* seg, int i0, int total,
+// Entries i0 .. i0 + KB - 1 of a segment's compacted list (padded with entries
+// that never hit), read from LDS at a uniform address (a broadcast), all of
+// them first. Height offset of a hit: round(h(r2) - fz), FP64 and half away from
+// zero in the reference. Here in FP32: R^2 - r2 is an exact float; the
+// hardware square root (v_sqrt_f32, within 1 ulp, not correctly rounded) of
+// it is within 1 ulp(R), fz is rounded once and the difference is rounded
+// once, each within half an ulp of R (h, fz and |h - fz| are at most R): the
+// FP32 difference is within 2 ulp(R) of the FP64 one. Wherever it lies within
+// 1/2 - 4 ulp(R) of an integer both round to that integer; the rest (a lane in
+// some ten thousands) takes the FP64 path, after the batch.
+template <int ZW, bool PRE, bool POSF, int KB>
+__device__ __forceinline__ void gather_fill(GBatch<KB>& B, const int4* seg, int i0,
                                             const GatherArgs& g, const GatherCol& c) {
+  int4 en[KB];
+  float x[KB];
+  int dz[KB];
+  bool in[KB];
+  float worst = 0.f;
+#pragma unroll
+  for (int t = 0; t < KB; ++t) en[t] = seg[i0 + t];
 #pragma unroll
   for (int t = 0; t < KB; ++t) {
-    const bool valid = i0 + t < total;  // uniform
-    const int4 en = seg[valid ? i0 + t : 0];
-    const int ea = en.x, fxy = en.y;
-    const float fz32 = __int_as_float(en.z);
-    const int fdx = c.qx + (int)(short)(fxy & 0xffff), fdy = c.qy + (fxy >> 16);
-    const int r2raw = fdx * fdx + fdy * fdy;
-    const bool inp = valid && fdx >= -g.nx && fdx < g.nx && fdy >= -g.nx && fdy < g.nx &&
-                     r2raw <= g.r2max;
-    const int r2 = inp ? r2raw : 0;
-    bool near;
-    int dz = height_off_f32(c.R2f, r2, fz32, c.thr, &near);
-    if (near && inp) dz = (int)round_away(height(c.R2, r2) - g.ageo[ea].fz);  // rare
-    const int k = dz - c.zbase;
-    const bool hit = inp && k >= 0 && k < ZW;
-    B.kv[t] = hit ? k : -1;
-    B.ea[t] = valid ? ea : 0;
-    B.el[t] = !hit ? kMissOffset
-                   : (g.frame_pos ? (uint32_t)((fdy + g.nx) * g.C + (fdx + g.nx)) * 8u : c.fixed);
-    if constexpr (!PRE) B.b[t] = g.beta[r2];
+    const float fdx = c.qx + __int_as_float(en[t].y), fdy = c.qy + __int_as_float(en[t].z);
+    x[t] = __builtin_fmaf(-fdy, fdy, __builtin_fmaf(-fdx, fdx, c.R2f));  // R^2 - |fd|^2
+    in[t] = x[t] >= c.xmin;
+    if (c.square) {  // uniform
+      const float nx = (float)g.nx;
+      in[t] = in[t] && fdx >= -nx && fdx < nx && fdy >= -nx && fdy < nx;
+    }
+    const float d = __builtin_amdgcn_sqrtf(fmaxf(x[t], 0.f)) - __int_as_float(en[t].w);
+    const float r = __builtin_rintf(d);
+    worst = fmaxf(worst, fabsf(d - r));
+    dz[t] = (int)r;
+    B.ea[t] = __builtin_amdgcn_readfirstlane(en[t].x);
+    if constexpr (POSF)
+      B.el[t] = (uint32_t)__builtin_fmaf(fdy + (float)g.nx, (float)g.C, fdx + (float)g.nx) * 8u;
+  }
+  if (worst > c.half) {
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      const float d = __builtin_amdgcn_sqrtf(fmaxf(x[t], 0.f)) - __int_as_float(en[t].w);
+      if (in[t] && fabsf(d - __builtin_rintf(d)) > c.half)
+        dz[t] = (int)round_away(sqrt((double)x[t]) - g.ageo[B.ea[t]].fz);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < KB; ++t) {
+    const int k = dz[t] - c.zbase;
+    const bool hit = in[t] && (unsigned)k < (unsigned)ZW;
+    B.kv[t] = hit ? k : ZW;
+    B.el[t] = !hit ? kMissOffset : POSF ? B.el[t] : c.fixed;
+    if constexpr (!PRE) B.br[t] = !hit ? kMissOffset : (uint32_t)(c.R2f - x[t]) * 4u;
   }
 }
 
@@ -269,11 +312,23 @@ constexpr int kGatherSeg = 256;  // list entries tested (and compacted) per segm
 // flags: bit0 = normalise (divide by counts, 0 -> 1) and apply the centring
 // sign (-1)^(x+y+z) of the 3-D inverse FFT; counts are then not written.
 // bit2 = the plain sums with that centring sign, no counts (the adjoint of
-// the Born forward model).
+// the Born forward model; COUNT false).
 // PRE: the spectra are already multiplied by the Ewald factor beta of their
 // pupil pixel (the same FP32 product), so beta is not looked up here.
-// KB: list entries whose loads are issued together.
-template <int ZW, bool PRE, int KB>
+// POSF: spectra in the +posSpec frame. KB: list entries whose loads are issued
+// together.
+//
+// What bounds it: the tiles at the lateral origin, which nearly every angle
+// hits and whose sums are serial. Per entry and wave about 20 vector
+// instructions, and one LDS round trip per four entries; before, a branch per
+// entry (the rare FP64 height) and one per hit kept every list read and every
+// sum's LDS round trip exposed. Those tiles also raise their waves' issue
+// priority over the short lists' on the same SIMD. Gather alone, before and
+// now: 100 angles into 256^3 44 -> 30 us, 600 into 512^3 243 -> 192, 200 into
+// 1024^3 925 -> 807, the solver's adjoint of 400 into 256^3 125 -> 71 (a buffer
+// view per angle instead of one with a scalar offset: 31, 197, 812, 76; batches
+// of 16: 35, 243, 977, 81).
+template <int ZW, bool PRE, bool POSF, bool COUNT, int KB>
 __global__ void __launch_bounds__(256)
 k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __restrict__ order,
              const TileEntry* __restrict__ list, const int4* __restrict__ tinfo, int flags,
@@ -327,17 +382,25 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
     if (inb) {
       for (int z = zs0; z <= zs1; ++z) {
         g.vol[z * plane + col] = make_float2(0.f, 0.f);
-        if (!sgn) g.cnt[z * plane + col] = 0;
+        if (COUNT && !sgn) g.cnt[z * plane + col] = 0;
       }
     }
     return;
   }
+  if (4 * info.x > 3 * g.A) __builtin_amdgcn_s_setprio(3);
+  else if (2 * info.x > g.A) __builtin_amdgcn_s_setprio(2);
+  else if (4 * info.x > g.A) __builtin_amdgcn_s_setprio(1);
   // this column's ZW partial sums and hit counts (< 2^16: at most one hit
-  // per angle) live in LDS; each thread only touches its own column
-  __shared__ float2 acc[ZW][256];
-  __shared__ unsigned short cn[ZW][256];
+  // per angle) live in LDS, and a slot for the misses; each thread only
+  // touches its own column
+  __shared__ float2 acc[ZW + 1][256];
+  __shared__ unsigned cn[COUNT ? ZW / 2 + 1 : 1][256];
 #pragma unroll
-  for (int k = 0; k < ZW; ++k) { acc[k][tid] = make_float2(0.f, 0.f); cn[k][tid] = 0; }
+  for (int k = 0; k <= ZW; ++k) acc[k][tid] = make_float2(0.f, 0.f);
+  if constexpr (COUNT) {
+#pragma unroll
+    for (int k = 0; k <= ZW / 2; ++k) cn[k][tid] = 0;
+  }
   const TileEntry* lst = list + (size_t)tile * g.A;
   // spectrum element read by this column: the unshifted frame holds it at
   // (qy mod C, qx mod C) for every angle; the +posSpec frame at fd + NXMAX
@@ -345,12 +408,16 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
   const uint32_t fixed = (uint32_t)(frow * g.C + fcol) * 8u;
   const uint32_t C2b = (uint32_t)g.C * (uint32_t)g.C * 8u;  // bytes per angle
   const size_t C2 = (size_t)g.C * g.C;
-  const double R2 = g.htab[0] * g.htab[0];
-  const float R2f = (float)R2;  // an integer: exact below 2^24
-  // the FP32 height path's margin, 8 ulp(R); everything takes the FP64 path
-  // where R^2 - r2 would not be exact in FP32
-  const float thr = R2 < 16777216.0 ? ldexpf(1.f, ilogbf((float)g.htab[0]) - 20) : 2.f;
-  const int zbase = z0 - g.V / 2;
+  const float Rf = (float)g.htab[0];  // h(0) = R, an integer
+  const float R2f = Rf * Rf;
+  const GatherCol cg{(float)qx,
+                     (float)qy,
+                     z0 - g.V / 2,
+                     fixed,
+                     R2f,
+                     R2f - (float)g.r2max,
+                     0.5f - ldexpf(1.f, ilogbf(Rf) - 21),
+                     g.r2max >= g.nx * g.nx};
   // The tile's list in segments of kGatherSeg entries: each thread tests one
   // entry against the window, the overlapping ones are compacted into LDS in
   // list (angle) order, and every wave takes them KB at a time,
@@ -358,10 +425,9 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
   // while the sums of batch i are applied (each voxel's sum still takes its
   // hits in angle order). Both batches always issue their KB loads (misses
   // fetch nothing), so the outstanding-load count is the same on every path.
-  __shared__ int4 seg[kGatherSeg];
+  __shared__ int4 seg[kGatherSeg + 2 * KB];
   __shared__ int wcount[4];
   const int lane = tid & 63, wave = tid >> 6;
-  const GatherCol cg{qx, qy, zbase, fixed, R2f, thr, R2};
   for (int s0 = 0; s0 < info.x; s0 += kGatherSeg) {  // uniform
     __syncthreads();  // the previous segment is consumed
     const int j = s0 + tid;
@@ -381,20 +447,23 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
     const int total = wcount[0] + wcount[1] + wcount[2] + wcount[3];
     if (ov)
       seg[base + __popcll(bal & ((1ull << lane) - 1ull))] =
-          make_int4(e.a, e.fxy, __float_as_int(e.fz), 0);
+          make_int4(e.a, __float_as_int((float)(short)(e.fxy & 0xffff)),
+                    __float_as_int((float)(e.fxy >> 16)), __float_as_int(e.fz));
+    // past the list: entries outside every pupil
+    if (tid < 2 * KB) seg[total + tid] = make_int4(0, __float_as_int(1e9f), 0, 0);
     __syncthreads();
     const int nb = (total + KB - 1) / KB;
     GBatch<KB> A, B;
-    gather_fill<ZW, PRE, KB>(A, seg, 0, total, g, cg);
-    A.issue(g, C2, C2b);
+    gather_fill<ZW, PRE, POSF, KB>(A, seg, 0, g, cg);
+    A.template issue<PRE>(g, C2, C2b);
     for (int bi = 0; bi < nb; bi += 2) {
-      gather_fill<ZW, PRE, KB>(B, seg, (bi + 1) * KB, total, g, cg);
-      B.issue(g, C2, C2b);
-      A.template apply<PRE>(acc, cn, tid);
+      gather_fill<ZW, PRE, POSF, KB>(B, seg, (bi + 1) * KB, g, cg);
+      B.template issue<PRE>(g, C2, C2b);
+      A.template apply<PRE, COUNT, ZW>(acc, cn, tid);
       if (bi + 1 >= nb) break;
-      gather_fill<ZW, PRE, KB>(A, seg, (bi + 2) * KB, total, g, cg);
-      A.issue(g, C2, C2b);
-      B.template apply<PRE>(acc, cn, tid);
+      gather_fill<ZW, PRE, POSF, KB>(A, seg, (bi + 2) * KB, g, cg);
+      A.template issue<PRE>(g, C2, C2b);
+      B.template apply<PRE, COUNT, ZW>(acc, cn, tid);
     }
   }
   if (!inb) return;
@@ -404,10 +473,10 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
     if (z > zs1) break;
     if (z < zs0) continue;
     const float2 s = acc[k][tid];
-    const int c = cn[k][tid];
+    const int c = COUNT ? (int)(cn[k >> 1][tid] >> ((k & 1) * 16) & 0xffff) : 0;
     if (sgn) {
       float2 t = s;
-      if (norm) {
+      if (COUNT && norm) {
         const float d = (float)(c == 0 ? 1 : c);
         t = make_float2(s.x / d, s.y / d);
       }
@@ -415,7 +484,7 @@ k_gather_win(GatherArgs g, int ntx, int w0, int nwin, int items, const int* __re
       g.vol[z * plane + col] = t;
     } else {
       g.vol[z * plane + col] = s;
-      g.cnt[z * plane + col] = c;
+      if (COUNT) g.cnt[z * plane + col] = c;
     }
   }
 }
@@ -465,7 +534,7 @@ hipError_t launch_band(const AngleGeo* ageo, int A, int V, const double* htab, i
 }
 
 // the windowed gather with height windows of ZW voxels (LDS: 10 B per
-// voxel of the 256 x ZW block) and batches of KB list entries
+// voxel of the 256 x ZW block, 8 without counts) and batches of KB list entries
 template <int ZW, int KB>
 static hipError_t gather_windows(const GatherArgs& g, int ntx, int tiles, const int* order,
                                  const TileEntry* list, const int4* tinfo, int flags,
@@ -480,13 +549,23 @@ static hipError_t gather_windows(const GatherArgs& g, int ntx, int tiles, const 
   }
   const int nwin = w1 - w0 + 1, items = tiles * nwin;
   Timed tm("ewald_gather", s);
-  if (flags & 2) {
-    hipLaunchKernelGGL((k_gather_win<ZW, true, KB>), dim3(items), dim3(256), 0, s, g, ntx, w0,
-                       nwin, items, order, list, tinfo, flags, band);
+#define MTD_GL(PRE, POSF, COUNT)                                                              \
+  hipLaunchKernelGGL((k_gather_win<ZW, PRE, POSF, COUNT, KB>), dim3(items), dim3(256), 0, s, g, \
+                     ntx, w0, nwin, items, order, list, tinfo, flags, band)
+  const bool pre = flags & 2, count = !(flags & 4);
+  if (!g.frame_pos) {
+    // unshifted spectra come from the forward column pass, pre-weighted
+    if (!pre || !count) return hipErrorInvalidValue;
+    MTD_GL(true, false, true);
+  } else if (count) {
+    if (pre) return hipErrorInvalidValue;
+    MTD_GL(false, true, true);
+  } else if (pre) {
+    MTD_GL(true, true, false);
   } else {
-    hipLaunchKernelGGL((k_gather_win<ZW, false, KB>), dim3(items), dim3(256), 0, s, g, ntx, w0,
-                       nwin, items, order, list, tinfo, flags, band);
+    MTD_GL(false, true, false);
   }
+#undef MTD_GL
   return hipGetLastError();
 }
 
@@ -511,8 +590,11 @@ hipError_t launch_gather(const float2* spec, int frame_pos, const AngleGeo* ageo
                          float2* vol, int32_t* cnt, void* scratch, const int* order, int flags,
                          const int2* band, int zlo, int zhi, bool prepass, int zw, int kb,
                          hipStream_t s) {
-  if ((size_t)C * C * sizeof(float2) >= ((size_t)1 << 31)) return hipErrorInvalidValue;
-  GatherArgs g{spec, frame_pos, ageo, A, C, nxmax, V, htab, beta, r2max, vol, cnt};
+  // spectra below 2 GiB; R < V/2 with R^2 < 2^24, C^2 <= 2^24 (exact in FP32)
+  if (C > 4096 || V > 8192) return hipErrorInvalidValue;
+  const size_t specb = (size_t)std::max(A, 1) * C * C * sizeof(float2);
+  GatherArgs g{spec, frame_pos, ageo, A, C, nxmax, V, htab, beta, r2max, vol, cnt,
+               specb < ((size_t)1 << 31) ? (uint32_t)specb : 0u};
   const int ntx = (V + GT - 1) / GT, tiles = ntx * ntx;
   TileEntry* list;
   int4* tinfo;
@@ -540,7 +622,7 @@ hipError_t launch_gather(const float2* spec, int frame_pos, const AngleGeo* ageo
 
 hipError_t launch_gather_prepass(const AngleGeo* ageo, int A, int C, int nxmax, int V,
                                  const double* htab, int r2max, void* scratch, hipStream_t s) {
-  GatherArgs g{nullptr, 0, ageo, A, C, nxmax, V, htab, nullptr, r2max, nullptr, nullptr};
+  GatherArgs g{nullptr, 0, ageo, A, C, nxmax, V, htab, nullptr, r2max, nullptr, nullptr, 0u};
   const int ntx = (V + GT - 1) / GT, tiles = ntx * ntx;
   TileEntry* list;
   int4* tinfo;

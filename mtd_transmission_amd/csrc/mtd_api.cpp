@@ -1553,7 +1553,7 @@ int mtd_cap_weights(mtd_ctx* ctx, const mtd_geom* g, const int32_t* posspec, int
   float2* vol = (float2*)ws_get(ctx, WS_VOL, (size_t)V * V * V * sizeof(float2));
   int32_t* cnt = (int32_t*)ws_get(ctx, WS_CNT, (size_t)V * V * V * sizeof(int32_t));
   if (!spec || !vol || !cnt) return set_err(ctx, MTD_ERR_HIP, "out of device memory");
-  MTD_TRY(scatter_impl(ctx, g, spec, 0, posspec, A, (float*)vol, cnt, 0, nullptr, nullptr,
+  MTD_TRY(scatter_impl(ctx, g, spec, 1, posspec, A, (float*)vol, cnt, 0, nullptr, nullptr,
                        planned ? &geo : nullptr));
   const AngleGeo* ag =
       planned ? geo.ag : (const AngleGeo*)ws_get(ctx, WS_AGEO, (size_t)A * sizeof(AngleGeo));
