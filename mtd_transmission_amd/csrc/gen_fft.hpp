@@ -4,195 +4,265 @@
 // (pretraitement_hors_axe_CPU/main.cpp:103, src/FFTW_init.cpp:70-71,
 // Reconstruction/src/FFT_encaps.cpp:33-53).
 //
-// A block transforms nl lines held in LDS (two buffers of nl x W complex):
-//  - direct: L factors into radices 2, 3, 4, 5, 7, 8, 11, 13; Stockham
-//    autosort passes (each a full out-of-place pass between the two LDS
-//    buffers, one barrier per pass), twiddles from the length-L table;
+// A block transforms nl lines (a power of two) held in LDS, line fastest:
+//  - direct: L is a product of radices up to 32 (gen_radix_ok: every product
+//    of 2, 3, 5, 7, 11, 13 up to there), as few and as even as they come (two
+//    for nearly every length up to 1024). Each is one Stockham autosort pass: a
+//    thread reads the R values of one butterfly into registers, and after a
+//    barrier writes its register DFT back to the same buffer;
 //  - Bluestein (chirp-z) for lengths with a larger prime factor, written
 //    from the published method: X_k = w_k sum_n (x_n w_n) conj(w_(k-n)) with
 //    w_m = exp(-i pi m^2 / L), the convolution done as a cyclic one of length
-//    W = a power of two >= 2L - 1 with two forward length-W Stockham FFTs
-//    (the inverse through conjugation) and the host-computed spectrum of the
-//    chirp (scaled 1/W). The backward transform is conj(forward(conj(x))).
+//    W >= 2L - 1, the cheapest product of radices up to the next power of two,
+//    with two forward length-W FFTs (the inverse through conjugation) and the
+//    host-computed spectrum of the chirp (scaled 1/W).
+// The backward transform is the forward one with real and imaginary parts
+// exchanged on the way in and out.
 // Operations load and store through the same op interface as the compiled
 // passes (passes.hpp): load(batch, line, element), store(batch, line,
-// element, value), optional begin/skip/line.
+// element, value), optional begin/skip/line; an op that defines
+// store2(batch, line, element k, X[k], X[(L - k) % L]) gets both bins at once.
+//
+// What bounds it: the passes' LDS round trips and register DFTs at two or three
+// blocks per CU, not HBM (a 364-point line takes about 2 ns of the chip, twice
+// its memory time). With radices up to 13 only, out of place between two LDS
+// buffers, integer divisions in every pass, and as many columns per block as
+// the two buffers held (11 at 364), the 364^3 inverse passes took 911 us, now
+// 527; hologram rows of 600 one at a time 219, now packed in pairs 88; crop-122
+// rows and columns (Bluestein over 256 points, now 243) 238, now 178.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <utility>
 
 #include "dft.hpp"
 #include "passes.hpp"
 
 namespace mtd {
 
-constexpr int kGenMaxPasses = 24;
-constexpr int kGenThreads = 256;
-// LDS of a block: two buffers of nl x W complex values
-constexpr int kGenLdsBytes = 65536;
+constexpr int kGenMaxPasses = 8;
+constexpr int kGenThreads = 512;     // most threads of a block
+constexpr int kGenLdsBytes = 65536;  // most LDS of a block
+constexpr int kGenMaxRadix = 32;
+constexpr int kGenMaxLen = 4096;     // most points of a line in LDS
 
 struct GenPlan {
   int L;                   // transform length
   int W;                   // working length: L (direct) or the Bluestein length
   int nf;                  // radix passes over W
   int f[kGenMaxPasses];    // radices
+  int bfly;                // most butterflies of a pass over one line
   const float2* tw;        // exp(-2 pi i k / W), k < W
   const float2* chirp;     // Bluestein: exp(-i pi n^2 / L), n < L; nullptr: direct
   const float2* bk;        // Bluestein: FFT_W of the wrapped conj(chirp), times 1/W
 };
 
-// Lines per block: as many as the two LDS buffers hold (at most 64).
-__host__ __device__ inline int gen_lines_per_block(int W) {
-  int nl = kGenLdsBytes / (2 * W * (int)sizeof(float2));
-  if (nl > 64) nl = 64;
-  return nl < 1 ? 1 : nl;
+// a product of 2, 3, 5, 7, 11, 13, at most kGenMaxRadix
+__host__ __device__ constexpr bool gen_radix_ok(int R) {
+  if (R < 2 || R > kGenMaxRadix) return false;
+  for (int p : {2, 3, 5, 7, 11, 13})
+    while (R % p == 0) R /= p;
+  return R == 1;
 }
 
-template <int R, bool INV>
-__device__ __forceinline__ void gen_butterfly(const float2* __restrict__ src,
-                                              float2* __restrict__ dst, int j, int nb, int Ns,
-                                              int step, const float2* __restrict__ tw) {
+// The lines of a block in LDS: element n of line l at p[n * pitch + l]. Rows
+// are loaded along n (odd pitch: no bank conflicts), columns along l. The LDS
+// address space is in the pointer's type: the passes are calls.
+typedef float gen_v2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) gen_v2 gen_lds_v2;
+struct GenLines {
+  gen_lds_v2* p;
+  int lnl, pitch;  // log2 of the lines, and the distance of two elements
+  __device__ __forceinline__ int nl() const { return 1 << lnl; }
+  __device__ __forceinline__ float2 get(int l, int n) const {
+    const gen_v2 v = p[n * pitch + l];
+    return make_float2(v.x, v.y);
+  }
+  __device__ __forceinline__ void set(int l, int n, float2 v) const {
+    p[n * pitch + l] = gen_v2{v.x, v.y};
+  }
+};
+
+inline int gen_pitch(int lnl, bool rows) { return rows && lnl > 0 ? (1 << lnl) + 1 : 1 << lnl; }
+
+// log2 of the lines per block: up to 32 (128-byte segments of float columns)
+// as far as LDS and the threads allow, 16 where 32 would leave a CU fewer than
+// four blocks
+inline int gen_lnl(const GenPlan& p, bool rows) {
+  int l = 5;
+  auto bytes = [&](int k) { return (size_t)gen_pitch(k, rows) * p.W * sizeof(float2); };
+  if (bytes(5) > 40960) l = 4;
+  while (l > 0 && (bytes(l) > (size_t)kGenLdsBytes || (p.bfly << l) > kGenThreads)) --l;
+  return l;
+}
+
+inline int gen_threads(const GenPlan& p, int lnl) { return ((p.bfly << lnl) + 63) / 64 * 64; }
+
+// One Stockham pass of radix R over the block's lines, Ns the product of the
+// radices before it. A call: inlined into the loop over passes, the constants
+// of all radices' DFTs were kept in registers across it (800 spilled).
+template <int R>
+__device__ __attribute__((noinline)) void gen_pass_r(gen_lds_v2* p, int lnl, int pitch, int W,
+                                                     int Ns, const float2* __restrict__ tw) {
+  const GenLines x{p, lnl, pitch};
+  const int nb = W / R;  // uniform: one scalar division
+  const int l = threadIdx.x & (x.nl() - 1), j = threadIdx.x >> x.lnl;
+  const bool act = j < nb;
   float2 v[R];
-  const int k = j % Ns;
+  int d = j * R;
+  if (act) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    v[r] = src[j + r * nb];
-    if (r > 0 && k > 0) {
-      float2 w = tw[r * k * step];  // W_(Ns R)^(r k) = W_W^(r k step), r k step < W
-      if (INV) w.y = -w.y;
-      v[r] = cmul(v[r], w);
+    for (int r = 0; r < R; ++r) v[r] = x.get(l, j + r * nb);
+    if (Ns > 1) {  // uniform
+      // the last pass has Ns = nb: each butterfly is its own k
+      int k = j;
+      d = j;
+      if (nb != Ns) {
+        const int q = j / Ns;
+        k = j - q * Ns;
+        d = q * Ns * R + k;
+      }
+      const int step = k * (W / (Ns * R));  // W_(Ns R)^(r k) = W_W^(r step)
+#pragma unroll
+      for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[r * step]);
     }
   }
-  Dft<R, INV>::run(v);
-  const int d = (j / Ns) * Ns * R + k;
+  __syncthreads();
+  if (act) {
+    RegFFT<R, false>::run(v);
 #pragma unroll
-  for (int r = 0; r < R; ++r) dst[d + r * Ns] = v[r];
+    for (int r = 0; r < R; ++r) x.set(l, d + r * Ns, v[r]);
+  }
+  __syncthreads();
 }
 
-// Stockham passes over nl lines of length W (line l at in + l * W); returns
-// the buffer holding the result (in or out). All threads of the block call
-// it; it begins with the caller's data in place (barrier done by the caller)
-// and ends with a barrier.
-template <bool INV>
-__device__ float2* gen_stockham(float2* in, float2* out, int nl, int W, const int* f, int nf,
-                                const float2* __restrict__ tw) {
+__device__ __forceinline__ void gen_stockham(const GenLines& x, const GenPlan& p) {
   int Ns = 1;
-  for (int p = 0; p < nf; ++p) {
-    const int R = f[p];
-    const int nb = W / R;
-    const int step = W / (Ns * R);
-    for (int t = threadIdx.x; t < nl * nb; t += blockDim.x) {
-      const int l = t / nb, j = t - l * nb;
-      const float2* s = in + l * W;
-      float2* d = out + l * W;
-      switch (R) {
-        case 2: gen_butterfly<2, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 3: gen_butterfly<3, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 4: gen_butterfly<4, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 5: gen_butterfly<5, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 7: gen_butterfly<7, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 8: gen_butterfly<8, INV>(s, d, j, nb, Ns, step, tw); break;
-        case 11: gen_butterfly<11, INV>(s, d, j, nb, Ns, step, tw); break;
-        default: gen_butterfly<13, INV>(s, d, j, nb, Ns, step, tw); break;
+  for (int i = 0; i < p.nf; ++i) {
+    const int R = p.f[i];
+    switch (R) {
+#define X(r) \
+  case r: gen_pass_r<r>(x.p, x.lnl, x.pitch, p.W, Ns, p.tw); break;
+      X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(18)
+      X(20) X(21) X(22) X(24) X(25) X(26) X(27) X(28) X(30) X(32)
+#undef X
+    }
+    Ns *= R;
+  }
+}
+
+// Forward transforms of the block's lines, in place (elements [0, L) of each).
+// Begins after the caller's barrier, ends with one.
+__device__ __forceinline__ void gen_fft(const GenLines& x, const GenPlan& p) {
+  if (!p.chirp) {
+    gen_stockham(x, p);
+    return;
+  }
+  const int L = p.L, W = p.W, l = threadIdx.x & (x.nl() - 1);
+  const int n0 = threadIdx.x >> x.lnl, dn = blockDim.x >> x.lnl;
+  // x_n w_n, zero-padded to W
+  for (int n = n0; n < W; n += dn)
+    x.set(l, n, n < L ? cmul(x.get(l, n), p.chirp[n]) : make_float2(0.f, 0.f));
+  __syncthreads();
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    gen_stockham(x, p);
+    if (half == 0) {
+      // times the chirp's spectrum, conjugated: the inverse length-W FFT is
+      // conj(FFT(conj(.)))
+      for (int k = n0; k < W; k += dn) {
+        const float2 z = cmul(x.get(l, k), p.bk[k]);
+        x.set(l, k, make_float2(z.x, -z.y));
+      }
+    } else {
+      for (int k = n0; k < L; k += dn) {
+        const float2 c = x.get(l, k);
+        x.set(l, k, cmul(make_float2(c.x, -c.y), p.chirp[k]));
       }
     }
     __syncthreads();
-    float2* t = in;
-    in = out;
-    out = t;
-    Ns *= R;
   }
-  return in;
 }
 
-// Transforms nl lines of length p.L held at a + l * p.W (elements [0, L) of
-// each line; b is the second buffer). Returns the buffer whose lines hold
-// the result in [0, L). Begins after the caller's barrier, ends with one.
+// real and imaginary parts exchanged: before and after gen_fft, the backward
+// transform
 template <bool INV>
-__device__ float2* gen_fft(float2* a, float2* b, int nl, const GenPlan& p) {
-  if (!p.chirp) return gen_stockham<INV>(a, b, nl, p.W, p.f, p.nf, p.tw);
-  const int L = p.L, W = p.W;
-  // x_n w_n (conj(x) for the backward transform), zero-padded to W
-  for (int t = threadIdx.x; t < nl * W; t += blockDim.x) {
-    const int l = t / W, n = t - l * W;
-    float2 v = make_float2(0.f, 0.f);
-    if (n < L) {
-      v = a[l * W + n];
-      if (INV) v.y = -v.y;
-      v = cmul(v, p.chirp[n]);
-    }
-    a[l * W + n] = v;
-  }
-  __syncthreads();
-  float2* r = gen_stockham<false>(a, b, nl, W, p.f, p.nf, p.tw);
-  float2* o = r == a ? b : a;
-  // times the chirp's spectrum, conjugated: the inverse length-W FFT is
-  // conj(FFT(conj(.)))
-  for (int t = threadIdx.x; t < nl * W; t += blockDim.x) {
-    const int k = t % W;
-    const float2 z = cmul(r[t], p.bk[k]);
-    r[t] = make_float2(z.x, -z.y);
-  }
-  __syncthreads();
-  r = gen_stockham<false>(r, o, nl, W, p.f, p.nf, p.tw);
-  for (int t = threadIdx.x; t < nl * W; t += blockDim.x) {
-    const int l = t / W, k = t - l * W;
-    if (k < L) {
-      const float2 c = r[l * W + k];
-      float2 y = cmul(make_float2(c.x, -c.y), p.chirp[k]);
-      if (INV) y.y = -y.y;
-      r[l * W + k] = y;
-    }
-  }
-  __syncthreads();
-  return r;
+__device__ __forceinline__ float2 gen_swap(float2 v) {
+  return INV ? make_float2(v.y, v.x) : v;
 }
 
-// Batched 1-D transforms of nlines lines per batch (grid: line groups x
-// batches). ROWS: a block's lines are consecutive rows and element loads run
-// along each line; otherwise its lines are adjacent columns and the loads of
-// one element index run across them (coalesced either way).
+// Calls fn(line of the block, element) for this thread's share of nl lines of
+// n elements: rows run along the lines, columns across them.
+template <bool ROWS, class Fn>
+__device__ __forceinline__ void gen_each(int lnl, int n, Fn&& fn) {
+  if (ROWS) {
+    for (int l = 0; l < 1 << lnl; ++l)
+      for (int i = threadIdx.x; i < n; i += blockDim.x) fn(l, i);
+  } else {
+    const int l = threadIdx.x & ((1 << lnl) - 1);
+    for (int i = threadIdx.x >> lnl; i < n; i += blockDim.x >> lnl) fn(l, i);
+  }
+}
+
+template <class Op, class = void>
+struct has_store2 : std::false_type {};
+template <class Op>
+struct has_store2<Op, std::void_t<decltype(&Op::store2)>> : std::true_type {};
+
+// Batched 1-D transforms of nlines lines per batch (grid: line groups, rounded
+// up to 8 of them, x batches; see xcd_block). ROWS: a block's lines are
+// consecutive rows and element loads run along each line; otherwise its lines
+// are adjacent columns and the loads of one element index run across them
+// (coalesced either way).
 template <bool INV, bool ROWS, class Op>
-__global__ void __launch_bounds__(kGenThreads) k_gen(Op op, GenPlan p, int nlines, int nl) {
+__global__ void __launch_bounds__(kGenThreads, 4)
+k_gen(Op op, GenPlan p, int nlines, int lnl, int pitch) {
   extern __shared__ float2 gen_lds[];
-  const int a = blockIdx.y, line0 = blockIdx.x * nl;
+  const int2 ab = xcd_block();
+  const int a = ab.x, line0 = ab.y << lnl;
+  if (line0 >= nlines) return;
   if (skip_batch(op, a)) return;  // block-uniform, before any barrier
   op.begin(a);
-  float2* A = gen_lds;
-  float2* B = gen_lds + (size_t)nl * p.W;
-  const int nact = min(nl, nlines - line0);
-  const int L = p.L;
-  for (int t = threadIdx.x; t < nl * L; t += blockDim.x) {
-    int l, n;
-    if (ROWS) { l = t / L; n = t - l * L; } else { n = t / nl; l = t - n * nl; }
-    float2 v = make_float2(0.f, 0.f);
-    if (l < nact) {
-      if constexpr (has_line<Op>::value) {
-        Op o = op;
-        o.line(a, line0 + l);
-        v = o.load(a, line0 + l, n);
-      } else {
-        v = op.load(a, line0 + l, n);
-      }
+  const GenLines x{(gen_lds_v2*)gen_lds, lnl, pitch};
+  const int nact = min(1 << lnl, nlines - line0), L = p.L;
+  static_assert(ROWS || !has_line<Op>::value, "per-line state is for rows");
+  if constexpr (has_line<Op>::value) {
+    for (int l = 0; l < 1 << lnl; ++l) {
+      if (l < nact) op.line(a, line0 + l);
+      for (int n = threadIdx.x; n < L; n += blockDim.x)
+        x.set(l, n, l < nact ? gen_swap<INV>(op.load(a, line0 + l, n)) : make_float2(0.f, 0.f));
     }
-    A[l * p.W + n] = v;
+  } else {
+    gen_each<ROWS>(lnl, L, [&](int l, int n) {
+      x.set(l, n, l < nact ? gen_swap<INV>(op.load(a, line0 + l, n)) : make_float2(0.f, 0.f));
+    });
   }
   __syncthreads();
-  const float2* R = gen_fft<INV>(A, B, nl, p);
-  for (int t = threadIdx.x; t < nl * L; t += blockDim.x) {
-    int l, n;
-    if (ROWS) { l = t / L; n = t - l * L; } else { n = t / nl; l = t - n * nl; }
-    if (l < nact) op.store(a, line0 + l, n, R[l * p.W + n]);
-  }
+  gen_fft(x, p);
+  gen_each<ROWS>(lnl, L, [&](int l, int n) {
+    if (l >= nact) return;
+    if constexpr (has_store2<Op>::value) {
+      op.store2(a, line0 + l, n, gen_swap<INV>(x.get(l, n)),
+                gen_swap<INV>(x.get(l, n ? L - n : 0)));
+    } else {
+      op.store(a, line0 + l, n, gen_swap<INV>(x.get(l, n)));
+    }
+  });
+}
+
+// line groups of a launch, rounded up to a multiple of 8
+inline unsigned gen_groups(int nlines, int lnl) {
+  return (unsigned)(((nlines + (1 << lnl) - 1) >> lnl) + 7) / 8 * 8;
 }
 
 template <bool INV, bool ROWS, class Op>
 inline hipError_t launch_gen(const Op& op, const GenPlan& p, int nlines, int batches,
                              hipStream_t s) {
   if (nlines <= 0 || batches <= 0) return hipSuccess;
-  const int nl = gen_lines_per_block(p.W);
-  const size_t lds = (size_t)2 * nl * p.W * sizeof(float2);
-  hipLaunchKernelGGL((k_gen<INV, ROWS, Op>), dim3((nlines + nl - 1) / nl, batches),
-                     dim3(kGenThreads), lds, s, op, p, nlines, nl);
+  const int lnl = gen_lnl(p, ROWS), pitch = gen_pitch(lnl, ROWS);
+  hipLaunchKernelGGL((k_gen<INV, ROWS, Op>), dim3(gen_groups(nlines, lnl), batches),
+                     dim3(gen_threads(p, lnl)), (size_t)pitch * p.W * sizeof(float2), s, op, p,
+                     nlines, lnl, pitch);
   return hipGetLastError();
 }
 

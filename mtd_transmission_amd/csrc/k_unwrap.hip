@@ -345,98 +345,101 @@ static hipError_t unwrap_c(const float2* iu, int A, const float2* tw, const floa
 // runtime-length FFTs, nl lines in LDS per block (gen_fft.hpp), a line's
 // positions reordered on load.
 // ---------------------------------------------------------------------------
-// this thread's elements (line l of the block, position i) of nl lines: rows
-// run along the lines, columns across them
-template <bool ROWS, class Fn>
-__device__ __forceinline__ void gen_each(int nl, int C, Fn&& fn) {
-  for (int t = threadIdx.x; t < nl * C; t += blockDim.x) {
-    int l, i;
-    if (ROWS) { l = t / C; i = t - l * C; } else { i = t / nl; l = t - i * nl; }
-    fn(l, i);
-  }
-}
-
-// Pair pass over bins k and C - k of each line, in place: fn(k, V[k], V[C-k])
-// gives both bins' new values (k = 0 and C/2 are their own mirrors).
+// Pair pass over bins k and C - k of each line, in place: fn(line, k, V[k],
+// V[C-k]) gives both bins' new values (k = 0 and C/2 are their own mirrors).
 template <class Fn>
-__device__ __forceinline__ void gen_pairs(float2* R, int nl, int W, int C, Fn&& fn) {
-  const int h = C / 2 + 1;
-  for (int t = threadIdx.x; t < nl * h; t += blockDim.x) {
-    const int l = t / h, k = t - l * h, m = k ? C - k : 0;
-    float2* r = R + l * W;
-    const float2 a = r[k], b = r[m];
-    r[k] = fn(l, k, a, b);
-    if (m != k) r[m] = fn(l, m, b, a);
+__device__ __forceinline__ void gen_pairs(const GenLines& x, int C, Fn&& fn) {
+  const int l = threadIdx.x & (x.nl() - 1);
+  for (int k = threadIdx.x >> x.lnl; k <= C / 2; k += blockDim.x >> x.lnl) {
+    const int m = k ? C - k : 0;
+    const float2 a = x.get(l, k), b = x.get(l, m);
+    x.set(l, k, fn(l, k, a, b));
+    if (m != k) x.set(l, m, fn(l, m, b, a));
   }
   __syncthreads();
 }
 
 template <bool ROWS>
-__global__ void __launch_bounds__(kGenThreads)
+__global__ void __launch_bounds__(kGenThreads, 4)
 k_unw_grad_gen(const float2* __restrict__ iu, GenPlan p, int C, const float2* __restrict__ tw4,
-               float* __restrict__ gx, float2* __restrict__ H, int nl) {
+               float* __restrict__ gx, float2* __restrict__ H, int lnl, int pitch) {
   extern __shared__ float2 gen_lds[];
-  const int a = blockIdx.y, line0 = blockIdx.x * nl;
-  const int nact = min(nl, C - line0);
-  float2* A = gen_lds;
-  float2* B = gen_lds + (size_t)nl * p.W;
+  const int2 ab = xcd_block();
+  const int a = ab.x, line0 = ab.y << lnl;
+  if (line0 >= C) return;
+  const int nact = min(1 << lnl, C - line0);
+  const GenLines x{(gen_lds_v2*)gen_lds, lnl, pitch};
   const float2* iu_a = iu + (size_t)a * C * C;
   const size_t base = (size_t)a * C * C;
+  const int h = C / 2;
+  auto wrap = [C](int i) { return i < C ? i : i - C; };
   auto phasor = [&](int l, int m) {
-    const int i = (dct_src(m, C) + C / 2) % C, j = (line0 + l + C / 2) % C;
+    const int i = wrap(dct_src(m, C) + h), j = wrap(line0 + l + h);
     return unit_phasor(ROWS ? iu_a[(size_t)j * C + i] : iu_a[(size_t)i * C + j]);
   };
-  gen_each<ROWS>(nl, C, [&](int l, int m) {
-    A[l * p.W + m] = l < nact ? phasor(l, m) : make_float2(0.f, 0.f);
+  gen_each<ROWS>(lnl, C, [&](int l, int m) {
+    x.set(l, m, l < nact ? phasor(l, m) : make_float2(0.f, 0.f));
   });
   __syncthreads();
-  float2* R = gen_fft<false>(A, B, nl, p);
-  gen_pairs(R, nl, p.W, C,
-            [&](int, int k, float2 V, float2 Vr) { return deriv_bin(V, Vr, k, C, tw4); });
-  float2* D = gen_fft<true>(R, R == A ? B : A, nl, p);
-  gen_each<ROWS>(nl, C, [&](int l, int m) {
-    if (l >= nact) return;
-    const float2 w = D[l * p.W + m], z = phasor(l, m);
-    const float g = w.y * z.x - w.x * z.y;
-    const int n = dct_src(m, C);
-    if (ROWS) gx[base + (size_t)(line0 + l) * C + n] = m < C / 2 ? g : -g;
-    else D[l * p.W + m] = make_float2(gx[base + (size_t)n * C + line0 + l], g);
-  });
-  if (ROWS) return;  // uniform
-  __syncthreads();
-  R = gen_fft<false>(D, D == A ? B : A, nl, p);
-  gen_pairs(R, nl, p.W, C, [&](int, int k, float2 V, float2 Vr) {
-    const float2 e = tw4[k], P = dct_p(V, e), Q = dct_q(Vr, e);
-    return make_float2(0.5f * (P.x + Q.x), 0.5f * (P.x - Q.x));
-  });
-  gen_each<ROWS>(nl, C, [&](int l, int k) {
-    if (l < nact) H[base + (size_t)k * C + line0 + l] = R[l * p.W + k];
-  });
+  // forward, derivative, backward (through the exchange of parts), and for
+  // the columns the packed forward transform
+#pragma unroll 1
+  for (int pass = 0; pass < (ROWS ? 2 : 3); ++pass) {
+    gen_fft(x, p);
+    if (pass == 0) {
+      gen_pairs(x, C, [&](int, int k, float2 V, float2 Vr) {
+        return gen_swap<true>(deriv_bin(V, Vr, k, C, tw4));
+      });
+    } else if (pass == 1) {
+      gen_each<ROWS>(lnl, C, [&](int l, int m) {
+        if (l >= nact) return;
+        const float2 w = gen_swap<true>(x.get(l, m)), z = phasor(l, m);
+        const float g = w.y * z.x - w.x * z.y;
+        const int n = dct_src(m, C);
+        if (ROWS) gx[base + (size_t)(line0 + l) * C + n] = m < h ? g : -g;
+        else x.set(l, m, make_float2(gx[base + (size_t)n * C + line0 + l], g));
+      });
+      __syncthreads();
+    } else {
+      gen_pairs(x, C, [&](int, int k, float2 V, float2 Vr) {
+        const float2 e = tw4[k], P = dct_p(V, e), Q = dct_q(Vr, e);
+        return make_float2(0.5f * (P.x + Q.x), 0.5f * (P.x - Q.x));
+      });
+      gen_each<ROWS>(lnl, C, [&](int l, int k) {
+        if (l < nact) H[base + (size_t)k * C + line0 + l] = x.get(l, k);
+      });
+    }
+  }
 }
 
-__global__ void __launch_bounds__(kGenThreads)
+__global__ void __launch_bounds__(kGenThreads, 4)
 k_unw_poisson_gen(const float2* __restrict__ H, GenPlan p, int C, const float2* __restrict__ tw4,
-                  float* __restrict__ out, int nl) {
+                  float* __restrict__ out, int lnl, int pitch) {
   extern __shared__ float2 gen_lds[];
-  const int a = blockIdx.y, line0 = blockIdx.x * nl;
-  const int nact = min(nl, C - line0);
-  float2* A = gen_lds;
-  float2* B = gen_lds + (size_t)nl * p.W;
+  const int2 ab = xcd_block();
+  const int a = ab.x, line0 = ab.y << lnl;
+  if (line0 >= C) return;
+  const int nact = min(1 << lnl, C - line0);
+  const GenLines x{(gen_lds_v2*)gen_lds, lnl, pitch};
   const size_t base = ((size_t)a * C + line0) * C;
-  gen_each<true>(nl, C, [&](int l, int m) {
+  gen_each<true>(lnl, C, [&](int l, int m) {
     float2 v = make_float2(0.f, 0.f);
     if (l < nact) v = H[base + (size_t)l * C + dct_src(m, C)];
-    A[l * p.W + m] = make_float2(m < C / 2 ? v.x : -v.x, v.y);
+    x.set(l, m, make_float2(m < C / 2 ? v.x : -v.x, v.y));
   });
   __syncthreads();
-  float2* R = gen_fft<false>(A, B, nl, p);
-  gen_pairs(R, nl, p.W, C, [&](int l, int k, float2 V, float2 Vr) {
-    const float2 e = tw4[k];
-    return poisson_bin(dct_p(V, e), dct_q(Vr, e), e, k, line0 + l, C);
-  });
-  const float2* D = gen_fft<true>(R, R == A ? B : A, nl, p);
-  gen_each<true>(nl, C, [&](int l, int m) {
-    if (l < nact) out[base + (size_t)l * C + dct_src(m, C)] = D[l * p.W + m].x;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    gen_fft(x, p);
+    if (pass == 0) {
+      gen_pairs(x, C, [&](int l, int k, float2 V, float2 Vr) {
+        const float2 e = tw4[k];
+        return gen_swap<true>(poisson_bin(dct_p(V, e), dct_q(Vr, e), e, k, line0 + l, C));
+      });
+    }
+  }
+  gen_each<true>(lnl, C, [&](int l, int m) {
+    if (l < nact) out[base + (size_t)l * C + dct_src(m, C)] = gen_swap<true>(x.get(l, m)).x;
   });
 }
 
@@ -459,20 +462,22 @@ struct UnwOutGenOp {  // pairs of columns (2 col, 2 col + 1)
 
 static hipError_t unwrap_gen(int C, const float2* iu, int A, const GenPlan& p, const float2* tw4,
                              float* gx, float2* H, float* phu, hipStream_t s) {
-  const int nl = gen_lines_per_block(p.W);
-  const size_t lds = (size_t)2 * nl * p.W * sizeof(float2);
-  const dim3 grid((C + nl - 1) / nl, A), block(kGenThreads);
+  const int lr = gen_lnl(p, true), lc = gen_lnl(p, false);
+  const int pr = gen_pitch(lr, true), pc = gen_pitch(lc, false);
+  const size_t mr = (size_t)pr * p.W * sizeof(float2), mc = (size_t)pc * p.W * sizeof(float2);
+  const dim3 gr(gen_groups(C, lr), A), gc(gen_groups(C, lc), A);
+  const dim3 br(gen_threads(p, lr)), bc(gen_threads(p, lc));
   {
     Timed tm("unwrap_gx", s);
-    hipLaunchKernelGGL((k_unw_grad_gen<true>), grid, block, lds, s, iu, p, C, tw4, gx, H, nl);
+    hipLaunchKernelGGL((k_unw_grad_gen<true>), gr, br, mr, s, iu, p, C, tw4, gx, H, lr, pr);
   }
   {
     Timed tm("unwrap_gy", s);
-    hipLaunchKernelGGL((k_unw_grad_gen<false>), grid, block, lds, s, iu, p, C, tw4, gx, H, nl);
+    hipLaunchKernelGGL((k_unw_grad_gen<false>), gc, bc, mc, s, iu, p, C, tw4, gx, H, lc, pc);
   }
   {
     Timed tm("unwrap_poisson", s);
-    hipLaunchKernelGGL(k_unw_poisson_gen, grid, block, lds, s, H, p, C, tw4, gx, nl);
+    hipLaunchKernelGGL(k_unw_poisson_gen, gr, br, mr, s, H, p, C, tw4, gx, lr, pr);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
