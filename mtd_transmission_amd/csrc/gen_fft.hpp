@@ -233,9 +233,15 @@ k_gen(Op op, GenPlan p, int nlines, int lnl, int pitch) {
         x.set(l, n, l < nact ? gen_swap<INV>(op.load(a, line0 + l, n)) : make_float2(0.f, 0.f));
     }
   } else {
+    bool any = false;
     gen_each<ROWS>(lnl, L, [&](int l, int n) {
-      x.set(l, n, l < nact ? gen_swap<INV>(op.load(a, line0 + l, n)) : make_float2(0.f, 0.f));
+      const float2 v = l < nact ? op.load(a, line0 + l, n) : make_float2(0.f, 0.f);
+      if constexpr (has_keep<Op>::value) any = any || v.x != 0.f || v.y != 0.f;
+      x.set(l, n, gen_swap<INV>(v));
     });
+    if constexpr (has_keep<Op>::value) {
+      if (op.scans() && !op.keep(a, line0, nact, __syncthreads_or(any))) return;
+    }
   }
   __syncthreads();
   gen_fft(x, p);

@@ -176,7 +176,7 @@ enum WsSlot {
   WS_T1 = 0, WS_CROP, WS_WORK, WS_IU, WS_POS, WS_COEF, WS_AGEO, WS_F,
   WS_VOL, WS_CNT, WS_VWORK, WS_HOLOTMP, WS_GATHER, WS_ARGMAX, WS_BAND, WS_PHU, WS_UNWRAP, WS_HOLOPART,
   WS_PLANPOS, WS_PLANAGEO, WS_PLANBAND, WS_PLANGATHER, WS_HSTAGE, WS_BATCHTS,
-  WS_TVZ, WS_TVZN, WS_TVGD, WS_TVS
+  WS_TVZ, WS_TVZN, WS_TVGD, WS_TVS, WS_OCC
 };
 
 int set_err(mtd_ctx* ctx, int code, const std::string& msg);
@@ -352,10 +352,11 @@ hipError_t launch_cap_sample(const float2* vol, const AngleGeo* ageo, int A, con
                              const float* q2, int r2max, int nx, int C, int V, float2* spec,
                              hipStream_t s);
 // prenorm=1: vol already divided by counts and centring-signed (gather flag 1).
-// band != nullptr: heights outside the band are zero and are not read.
+// band: heights outside it are zero and are not read. occ != nullptr (V^2
+// bytes): the band is not known and is found by the first pass into *band.
 hipError_t launch_finalize(int V, const float2* vol, const int32_t* cnt,
-                           int prenorm, const int2* band, float2* work, float df3, float cte,
-                           float gsign, float* out_re, float* out_im,
+                           int prenorm, int2* band, uint8_t* occ, float2* work, float df3,
+                           float cte, float gsign, float* out_re, float* out_im,
                            uint8_t* otf, const FftTab& ft, int2 tiles, hipStream_t s);
 
 }  // namespace mtd

@@ -1423,12 +1423,18 @@ int mtd_ewald_accumulate(mtd_ctx* ctx, const mtd_geom* g, const float* fields,
 
 // scale > 0: output factor in place of delta_f^3 * (-1/(2 n0 kv^2)).
 static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
-                         const int32_t* counts, int prenorm, const int2* band, float* index_re,
+                         const int32_t* counts, int prenorm, int2* band, float* index_re,
                          float* index_im, uint8_t* otf, double scale = 0) {
   const int V = g->dim_final;
   float2* work = (float2*)ws_get(ctx, WS_VWORK, (size_t)V * V * V * sizeof(float2));
   FftTab twV;
   const bool tabs = fft_tab(ctx, V, vol_len_supported(V), &twV);
+  uint8_t* occ = nullptr;
+  if (!band) {
+    band = (int2*)ws_get(ctx, WS_BAND, sizeof(int2));
+    occ = (uint8_t*)ws_get(ctx, WS_OCC, (size_t)V * V);
+    if (!band || !occ) return set_err(ctx, MTD_ERR_HIP, "out of device memory (volume band)");
+  }
   if (!work || !tabs) return set_err(ctx, MTD_ERR_HIP, "out of device memory (volume work)");
   // Reconstruction/main.cpp:346-347 (PI = M_PI there) and the delta_f^3 of
   // TF3Dcplx_INV (src/FFT_fonctions.cpp:399)
@@ -1436,7 +1442,7 @@ static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
   const double cte = scale > 0 ? 1.0 : -1.0 / (2 * g->n0 * kv * kv);
   const float df3 = scale > 0 ? (float)scale : (float)std::pow(g->delta_f, 3);
   const float gsign = ((V / 2) & 1) ? -1.f : 1.f;
-  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, prenorm, band, work, df3,
+  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, prenorm, band, occ, work, df3,
                                         (float)cte, gsign, index_re, index_im, otf, twV,
                                         make_int2(ctx->vol_rows_tile, ctx->vol_cols_tile),
                                         ctx->stream),

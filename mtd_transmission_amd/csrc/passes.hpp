@@ -155,6 +155,16 @@ struct has_line : std::false_type {};
 template <class Op>
 struct has_line<Op, std::void_t<decltype(std::declval<Op&>().line(0, 0))>> : std::true_type {};
 
+// An operation may define keep(batch, first line, lines, any), called once by
+// every thread of a row block after its loads, with whether any loaded value
+// of the block's lines is not zero (NaN is not zero): the block then leaves
+// its lines alone when it returns false.
+template <class Op, class = void>
+struct has_keep : std::false_type {};
+template <class Op>
+struct has_keep<Op, std::void_t<decltype(std::declval<const Op&>().keep(0, 0, 0, false))>>
+    : std::true_type {};
+
 template <int L, bool INV, class Op, int TV = 0>
 __global__ void __launch_bounds__(256) k_rows(Op op) {
   using F = Fft2<L, INV>;
@@ -170,6 +180,14 @@ __global__ void __launch_bounds__(256) k_rows(Op op) {
   float2 v[F::L1], u[F::L2];
 #pragma unroll
   for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.load(a, line, F::L2 * n1 + n2);
+  if constexpr (has_keep<Op>::value) {
+    if (op.scans()) {  // uniform
+      bool any = false;
+#pragma unroll
+      for (int n1 = 0; n1 < F::L1; ++n1) any = any || v[n1].x != 0.f || v[n1].y != 0.f;
+      if (!op.keep(a, ab.y * NT, NT, __syncthreads_or(any))) return;  // block-uniform
+    }
+  }
   F::run(v, u, n2, typename F::Row{lds + r * F::LDS_ROW}, op.tw);
   if (n2 < F::L1) {
 #pragma unroll

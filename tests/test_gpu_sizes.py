@@ -61,3 +61,51 @@ def test_plain_at_size(gpu_ctx, n, nx, V, A):
         e64, bound = rel_l2(got.ravel()[sel], o64), fp64_bound(o32, o64)
     _say(f"  index rel-L2 vs f32 {e32:.3e}  vs f64 {e64:.3e} (bound {bound:.2e})")
     assert e32 < TOL and e64 <= bound
+
+
+@pytest.mark.parametrize("V", [64, 128, 256, 364, 512])
+@pytest.mark.parametrize("kind", ["band", "rows", "empty", "nan"])
+def test_finalize_sparse(gpu_ctx, V, kind):
+    """finalize of spectra with empty rows and planes (found by its first pass)
+    against the dense transform in 64 bits: a band, scattered rows at the
+    block edges of a few planes (first and last among them), nothing at all,
+    and a NaN (real part), which spreads over the volume. The bound is the 1e-5 parity bar."""
+    import torch
+    import mtd_transmission_amd as m
+    nx = V // 4
+    g = m.geom_derive(8 * nx, nx, V, 4 * nx, 4 * nx, 1.2, 1.333, 6.33e-7, nx * 6.33e-7 / 9.6 / nx)
+    print(f"finalize sparse V={V} {kind}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    keep = torch.zeros((V, V, V), dtype=torch.bool, device="cuda")
+    if kind == "band":
+        keep[V // 3:V // 2, V // 4:-V // 4, 3:] = True
+    elif kind == "rows":
+        for z in (0, V // 2 + 1, V - 1):
+            for y in (0, 7, 8, V // 2, V - 1):
+                keep[z, y, z % 5::7] = True
+    elif kind == "nan":
+        keep[V // 2, 3, 5] = True
+    vol = torch.randn((V, V, V), dtype=torch.complex64, device="cuda", generator=gen) * keep
+    if kind == "nan":
+        vol[V // 2, 3, 5] = float("nan")
+    cnt = torch.randint(0, 4, (V, V, V), dtype=torch.int32, device="cuda", generator=gen)
+    re = torch.full((V, V, V), 7.0, device="cuda")
+    im = torch.full((V, V, V), 7.0, device="cuda")
+    otf = torch.full((V, V, V), 9, dtype=torch.uint8, device="cuda")
+    for _ in range(2):  # the second call finds the first one's work volume
+        gpu_ctx.finalize(g, vol, cnt, re, im, otf)
+    torch.cuda.synchronize()
+    assert torch.equal(otf.bool(), (vol.real != 0) & (otf < 2))
+    if kind == "nan":
+        # one part of the voxel: quarter turns move it to the other part whole
+        assert bool((re.isnan() | im.isnan()).all())
+        return
+    t = vol.to(torch.complex128) / cnt.clamp(min=1)
+    t = torch.fft.fftshift(torch.fft.ifftn(torch.fft.ifftshift(t), norm="forward"))
+    kv = 2 * np.pi / g.lambda_
+    t *= -g.delta_f ** 3 / (2 * g.n0 * kv * kv)
+    got = torch.complex(re, im).to(torch.complex128)
+    if kind == "empty":
+        assert not bool(got.any())
+    else:
+        assert float((got - t).norm() / t.norm()) < 1e-5
