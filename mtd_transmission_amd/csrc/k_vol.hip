@@ -769,7 +769,17 @@ struct ZOutOp {  // lines along z; a = y, col = x, row = z
   const float2* tw;
   float df3, cte, gsign;
   const int2* band;
+  int only;  // 1: launched for bands that fit the folded pass, 2: for the others
   int lo, hi;
+  __device__ bool skip(int) const {
+    if constexpr (cols_fold_fits<VT>()) {
+      if (only) {
+        const int2 b = *band;
+        return cols_fold_narrow<VT>(b.x, b.y) != (only == 1);
+      }
+    }
+    return false;
+  }
   __device__ void begin(int) {
     if (band) {
       const int2 b = *band;
@@ -789,6 +799,18 @@ struct ZOutOp {  // lines along z; a = y, col = x, row = z
     const size_t i = ((size_t)z * V + y) * V + x;
     re[i] = (v.x * sg * df3) * cte;
     if (im) im[i] = (v.y * sg * df3) * cte;  // uniform: NULL skips the imaginary part
+  }
+  // the same for column x0 + c, with y, x0 and z uniform over the wave and
+  // c < 64 its lane: scalar addresses
+  __device__ __forceinline__ float2 load_wave(int y, int x0, int c, int z) const {
+    const bool in = z >= lo && z <= hi;
+    return BufView(buf + ((size_t)(in ? z : 0) * V + y) * V + x0, in ? 64 * 8 : 0).f2(c * 8, 0);
+  }
+  __device__ __forceinline__ void store_wave(int y, int x0, int c, int z, float2 v) const {
+    const float sg = ((x0 + c + y + z) & 1) ? -gsign : gsign;
+    const size_t i = ((size_t)z * V + y) * V + x0;
+    (re + i)[c] = (v.x * sg * df3) * cte;
+    if (im) (im + i)[c] = (v.y * sg * df3) * cte;
   }
   Dim<VT> V{};
 };
@@ -847,9 +869,32 @@ static hipError_t vol_cols(Dim<VT> V, const Op& op, const FftTab& ft, const char
   }
 }
 
+// The height pass. Volumes of 512 and 1024 fold the band (k_cols_fold): planes is
+// the band's height expected from the geometry, 0 where only the device knows
+// (then both forms are launched and the blocks of the one that does not apply
+// return). 512^3, band 151: 335 -> 278 us; 1024^3, band 302: 5.05 -> 2.43 ms.
+template <int VT>
+static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, int tile,
+                        hipStream_t s) {
+  if constexpr (VT > 0 && cols_fold_fits<VT>()) {
+    // the band may begin at any element of its first group of T
+    constexpr int T = Fft2<VT / cols_fold_r<VT>(), false>::T;
+    if (planes == 0 || cols_fold_narrow<VT>(T - 1, T - 1 + planes - 1)) {
+      Timed tm("vol_z", s);
+      z.only = planes ? 0 : 1;
+      hipLaunchKernelGGL((k_cols_fold<VT, true, ZOutOp<VT>>), dim3(VT / cols_fold_nc<VT>(), VT),
+                         dim3(cols_fold_threads<VT>()), 0, s, z);
+      const hipError_t e = hipGetLastError();
+      if (planes || e != hipSuccess) return e;
+      z.only = 2;
+    }
+  }
+  return vol_cols<VT, true, true>(V, z, ft, "vol_z", tile, s);
+}
+
 template <int VT>
 static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt, int prenorm,
-                             int2* band, uint8_t* occ, float2* work,
+                             int2* band, uint8_t* occ, int planes, float2* work,
                              float df3, float cte, float gsign, float* re,
                              float* im, uint8_t* otf, const FftTab& ft, int2 tiles,
                              hipStream_t s) {
@@ -859,11 +904,11 @@ static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt, i
   }
   NormXOp<VT> x{vol, cnt, work, otf, ft.tw, prenorm, occ ? nullptr : band, occ, band, V};
   PlaneYOp<VT> y{work, ft.tw, band, occ, V};
-  ZOutOp<VT> z{work, re, im, ft.tw, df3, cte, gsign, band, 0, V - 1, V};
+  ZOutOp<VT> z{work, re, im, ft.tw, df3, cte, gsign, band, 0, 0, V - 1, V};
   hipError_t e;
   if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
   if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
-  return vol_cols<VT, true, true>(V, z, ft, "vol_z", tiles.y, s);
+  return vol_z<VT>(V, z, planes, ft, tiles.y, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1002,19 +1047,19 @@ k_cap_weights(const int32_t* __restrict__ cnt, const AngleGeo* __restrict__ ageo
   X(1024)
 
 hipError_t launch_finalize(int V, const float2* vol, const int32_t* cnt,
-                           int prenorm, int2* band, uint8_t* occ, float2* work, float df3,
-                           float cte, float gsign, float* out_re, float* out_im,
+                           int prenorm, int2* band, uint8_t* occ, int planes, float2* work,
+                           float df3, float cte, float gsign, float* out_re, float* out_im,
                            uint8_t* otf, const FftTab& ft, int2 tiles, hipStream_t s) {
   switch (V) {
 #define X(n)                                                                                   \
   case n:                                                                                      \
-    return finalize_v<n>(Dim<n>{}, vol, cnt, prenorm, band, occ, work, df3, cte, gsign,        \
+    return finalize_v<n>(Dim<n>{}, vol, cnt, prenorm, band, occ, planes, work, df3, cte, gsign, \
                          out_re, out_im, otf, ft, tiles, s);
     MTD_VOL_SIZES(X)
 #undef X
   }
-  return finalize_v<0>(Dim<0>(V), vol, cnt, prenorm, band, occ, work, df3, cte, gsign, out_re,
-                       out_im, otf, ft, tiles, s);
+  return finalize_v<0>(Dim<0>(V), vol, cnt, prenorm, band, occ, planes, work, df3, cte, gsign,
+                       out_re, out_im, otf, ft, tiles, s);
 }
 
 hipError_t launch_contrast_spectrum(int V, const float* re, const float* im, float2* work,

@@ -1442,8 +1442,11 @@ static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
   const double cte = scale > 0 ? 1.0 : -1.0 / (2 * g->n0 * kv * kv);
   const float df3 = scale > 0 ? (float)scale : (float)std::pow(g->delta_f, 3);
   const float gsign = ((V / 2) & 1) ? -1.f : 1.f;
-  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, prenorm, band, occ, work, df3,
-                                        (float)cte, gsign, index_re, index_im, otf, twV,
+  // the caps of illuminations inside the pupil span this many planes
+  const double R = g->rayon, nx = g->nxmax;
+  const int planes = occ ? 0 : 2 * (int)std::ceil(R - std::sqrt(std::max(R * R - nx * nx, 0.0))) + 1;
+  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, prenorm, band, occ, planes,
+                                        work, df3, (float)cte, gsign, index_re, index_im, otf, twV,
                                         make_int2(ctx->vol_rows_tile, ctx->vol_cols_tile),
                                         ctx->stream),
                    "finalize");

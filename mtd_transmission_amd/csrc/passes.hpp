@@ -272,6 +272,137 @@ inline dim3 cols_b_block() {
   return dim3(cols_b_nc<L>() * Fft2B<L, false>::T);
 }
 
+// The column pass of a transform whose input fills a band of its elements
+// [op.lo, op.hi] (set by op.begin; load() gives zeros outside): the first radix
+// R = cols_fold_r is taken by decimation in frequency, X[R*q + r] being the
+// (L/R)-point transform over z mod L/R of x[z] exp(+-2 pi i r z / L), folded. A
+// block loads its band once into registers (NB values a thread) and then runs R
+// short transforms, so it holds 64 columns where the whole transform held 16 or
+// 32: the stores, one plane after the other, become 256-byte pieces. A band of
+// more than NB*T elements is folded from memory, read once per residue (correct,
+// but on a dense spectrum 1.6 -> 2.0 ms for all three passes at 512^3, 15 -> 25 ms
+// at 1024^3): callers that expect one take the whole transform (cols_fold_narrow).
+//
+// The float outputs' piece is what bounds the height pass. Storing two V^3 float
+// volumes column by column and reading a band of 0.295 V planes, with no
+// transform, takes at V = 1024 4.8, 2.85 and 2.23 ms with 16, 32 and 64 columns
+// a block (64-, 128- and 256-byte pieces), at V = 512 459, 254 and 241 us.
+template <int L>
+constexpr int cols_fold_r() {
+  return L / 256;
+}
+template <int L>
+constexpr int cols_fold_nc() {
+  return 64;
+}
+// registers for a band of 0.36 L: heights span 0.3135 L at 4 bins per pupil
+// radius (the smallest volume) and NA / n0 = 0.9
+template <int L>
+constexpr int cols_fold_nb() {
+  return (36 * L / 100 + Fft2<L / cols_fold_r<L>(), false>::T - 1) /
+         Fft2<L / cols_fold_r<L>(), false>::T;
+}
+template <class Op, class = void>
+struct op_cols_fold : std::false_type {};
+template <class Op>
+struct op_cols_fold<Op, std::void_t<decltype(Op::kFoldCols)>>
+    : std::integral_constant<bool, Op::kFoldCols> {};
+template <int L>
+constexpr bool cols_fold_fits() {
+  return L == 512 || L == 1024;
+}
+// band elements [lo, hi] in the register path
+template <int L>
+__host__ __device__ constexpr bool cols_fold_narrow(int lo, int hi) {
+  constexpr int T = Fft2<L / cols_fold_r<L>(), false>::T;
+  return hi < lo || hi / T - (lo > 0 ? lo / T : 0) + 1 <= cols_fold_nb<L>();
+}
+template <int L>
+constexpr int cols_fold_threads() {
+  return cols_fold_nc<L>() * Fft2<L / cols_fold_r<L>(), false>::T;
+}
+template <int L, bool INV, class Op>
+__global__ void __launch_bounds__(cols_fold_threads<L>(), 4) k_cols_fold(Op op) {
+  constexpr int R = cols_fold_r<L>(), M = L / R, NC = cols_fold_nc<L>(), NB = cols_fold_nb<L>();
+  using F = Fft2<M, INV>;
+  constexpr int L1 = F::L1, L2 = F::L2, T = F::T;
+  static_assert(L1 == L2 && NC == 64, "all threads in both steps, one column element a wave");
+  __shared__ float lds[NC * F::LDS_COL];
+  const int2 ab = xcd_block();
+  const int a = ab.x, c0 = ab.y * NC;
+  if (skip_batch(op, a)) return;  // block-uniform, before the barrier
+  const int c = threadIdx.x % NC;
+  // the wave's element: uniform, so every twiddle is a scalar load
+  const int n2 = __builtin_amdgcn_readfirstlane(threadIdx.x / NC);
+  op.begin(a);
+  // input index z = T*(b + j) + n2; n1 = (b + j) mod L1: the rotation by b of
+  // the first step's input is a phase on its output k1, W_L1^(b k1), which the
+  // step twiddle takes along
+  const int b = op.lo > 0 ? op.lo / T : 0;
+  const int nj = op.hi >= op.lo ? op.hi / T - b + 1 : 0;
+  const bool fits = cols_fold_narrow<L>(op.lo, op.hi);
+  float2 e[NB];
+  if (fits) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) e[j] = op.load_wave(a, c0, c, T * (b + j) + n2);
+  }
+  // the table is constant: scalar loads
+  typedef float v2f __attribute__((ext_vector_type(2)));
+  const auto* tw = (const __attribute__((address_space(4))) v2f*)op.tw;
+  const typename F::template Col<NC> x{lds + c};
+#pragma unroll 1
+  for (int r = 0; r < R; ++r) {
+    float2 v[L1], u[L2];
+    if (fits) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const v2f q = tw[r * (T * (b + j) + n2) % L];
+        const float2 w = make_float2(q.x, INV ? -q.y : q.y);
+        const float2 t = cmul(e[j], w);
+        if (j < L1) v[j] = t;
+        else v[j % L1] = make_float2(v[j % L1].x + t.x, v[j % L1].y + t.y);
+      }
+#pragma unroll
+      for (int j = NB; j < L1; ++j) v[j] = make_float2(0.f, 0.f);
+    } else {
+#pragma unroll
+      for (int j = 0; j < L1; ++j) v[j] = make_float2(0.f, 0.f);
+      for (int j0 = 0; j0 < nj; j0 += L1) {
+#pragma unroll
+        for (int j = 0; j < L1; ++j) {
+          const int z = T * (b + j0 + j) + n2;
+          const v2f q = tw[(r * z) % L];
+          const float2 w = make_float2(q.x, INV ? -q.y : q.y);
+          const float2 t = cmul(op.load_wave(a, c0, c, z), w);
+          v[j] = make_float2(v[j].x + t.x, v[j].y + t.y);
+        }
+      }
+    }
+    RegFFT<L1, INV>::run(v);
+#pragma unroll
+    for (int k1 = 1; k1 < L1; ++k1) {
+      const v2f q = tw[R * ((n2 + T * b) * k1) % L];
+      const float2 w = make_float2(q.x, INV ? -q.y : q.y);
+      v[k1] = cmul(v[k1], w);
+    }
+    if (r) __syncthreads();  // the last residue's reads
+#pragma unroll
+    for (int k1 = 0; k1 < L1; ++k1) *x.at(k1, n2) = v[k1].x;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < L2; ++n) u[n].x = *x.at(n2, n);
+    __syncthreads();
+#pragma unroll
+    for (int k1 = 0; k1 < L1; ++k1) *x.at(k1, n2) = v[k1].y;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < L2; ++n) u[n].y = *x.at(n2, n);
+    RegFFT<L2, INV>::run(u);
+#pragma unroll
+    for (int k2 = 0; k2 < L2; ++k2) op.store_wave(a, c0, c, R * (n2 + L1 * k2) + r, u[k2]);
+  }
+}
+
 // An operation may define mid_line(batch, line), called once per transform
 // between the first transform and its mid() calls: per-line state that only
 // mid() reads is then not held in registers through the first transform.
