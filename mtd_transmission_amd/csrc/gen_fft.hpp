@@ -236,11 +236,11 @@ k_gen(Op op, GenPlan p, int nlines, int lnl, int pitch) {
     bool any = false;
     gen_each<ROWS>(lnl, L, [&](int l, int n) {
       const float2 v = l < nact ? op.load(a, line0 + l, n) : make_float2(0.f, 0.f);
-      if constexpr (has_keep<Op>::value) any = any || v.x != 0.f || v.y != 0.f;
+      if constexpr (op_scans<Op>::value) any = any || v.x != 0.f || v.y != 0.f;
       x.set(l, n, gen_swap<INV>(v));
     });
-    if constexpr (has_keep<Op>::value) {
-      if (op.scans() && !op.keep(a, line0, nact, __syncthreads_or(any))) return;
+    if constexpr (op_scans<Op>::value) {
+      if (!op.keep(a, line0, nact, __syncthreads_or(any))) return;
     }
   }
   __syncthreads();

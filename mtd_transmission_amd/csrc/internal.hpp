@@ -351,13 +351,14 @@ hipError_t launch_cap_weights(const int32_t* cnt, const AngleGeo* ageo, int A,
 hipError_t launch_cap_sample(const float2* vol, const AngleGeo* ageo, int A, const double* htab,
                              const float* q2, int r2max, int nx, int C, int V, float2* spec,
                              hipStream_t s);
-// prenorm=1: vol already divided by counts and centring-signed (gather flag 1).
-// band: heights outside it are zero and are not read. occ != nullptr (V^2
-// bytes): the band is not known and is found by the first pass into *band.
+// band: heights outside it are zero and are not read; vol is then already divided
+// by its counts and centring-signed (gather flag 1). occ != nullptr (V^2 bytes,
+// rounded up to 16): the band is not known and is found by the first pass into
+// *band; vol and cnt are a spectrum and its counts.
 // planes: the band's expected height (a rule's input, not a bound), 0: unknown.
 hipError_t launch_finalize(int V, const float2* vol, const int32_t* cnt,
-                           int prenorm, int2* band, uint8_t* occ, int planes, float2* work,
-                           float df3, float cte, float gsign, float* out_re, float* out_im,
+                           int2* band, uint8_t* occ, int planes, float2* work, float df3,
+                           float cte, float gsign, float* out_re, float* out_im,
                            uint8_t* otf, const FftTab& ft, int2 tiles, hipStream_t s);
 
 }  // namespace mtd

@@ -693,47 +693,95 @@ __device__ __forceinline__ bool outside_band(const int2* band, int z) {
 // A spectrum volume from outside (mtd_finalize) comes without its hit band.
 // The x pass, which reads every voxel, finds out: occ[z][y] says whether the
 // row's block held anything but zeros (blocks of zero rows stop there), and
-// the band grows over the planes that did. The y pass reads no empty row and
-// skips the planes outside, the height pass reads the band alone. On a spectrum
-// of 400 angles at 512^3, band about a third: x 733 -> 560, y 450 -> 160, z 532 ->
-// 337 us.
-__global__ void k_band_start(int V, int2* __restrict__ band) { *band = make_int2(V, -1); }
+// k_band_found takes the band of planes that did from it. The y pass reads no
+// empty row and skips the planes outside, the height pass reads the band alone.
+// On a spectrum of 400 angles at 512^3, band about a third, with the OTF: x 733 ->
+// 393, y 450 -> 114, z 532 -> 280 us; on a dense spectrum all three 1.61 -> 1.69 ms.
+// (With every voxel's count read and divided by before the scan, the OTF stored a
+// byte at a time and two atomics on one word for the band: x 557 us.)
+constexpr int kBandThreads = 1024;
+// occ: V^2 bytes, readable to the next multiple of 16
+__global__ void __launch_bounds__(kBandThreads)
+k_band_found(const uint4* __restrict__ occ, int V, int2* __restrict__ band) {
+  const int n = V * V;
+  int lo = n, hi = -1;  // first and last occupied row
+  constexpr int KB = 8;  // words in flight
+  for (int i0 = threadIdx.x; 16 * i0 < n; i0 += KB * kBandThreads) {
+    uint4 w[KB];
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      const int i = i0 + k * kBandThreads;
+      w[k] = 16 * i < n ? occ[i] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      const uint32_t q[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int b = 16 * (i0 + k * kBandThreads) + 4 * j;
+        if (q[j] && b < n) {  // V is even: whole words
+          lo = min(lo, b + __builtin_ctz(q[j]) / 8);
+          hi = max(hi, b + 3 - __builtin_clz(q[j]) / 8);
+        }
+      }
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  __shared__ int2 red[kBandThreads / 64];
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = make_int2(lo, hi);
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < kBandThreads / 64; ++w) {
+    lo = min(lo, red[w].x);
+    hi = max(hi, red[w].y);
+  }
+  *band = hi < 0 ? make_int2(V, -1) : make_int2(lo / V, hi / V);
+}
 
-template <int VT>
+template <int VT, bool SCAN>
 struct NormXOp {  // rows along x; a = z, line = y
+  // SCAN: a spectrum and its counts, band not known; otherwise the gather's
+  // normalised volume, already times (-1)^(x+y+z)
+  static constexpr bool kScans = SCAN;
   const float2* vol;
   const int32_t* cnt;
   float2* out;
   uint8_t* otf;
   const float2* tw;
-  int prenorm;
   const int2* band;
-  uint8_t* occ;  // nullptr: the band is known
-  int2* found;
-  __device__ bool skip(int z) const { return outside_band(band, z); }
+  uint8_t* occ;  // SCAN
+  __device__ bool skip(int z) const { return !SCAN && outside_band(band, z); }
   __device__ void begin(int) {}
-  __device__ bool scans() const { return occ != nullptr; }
+  // The OTF (nonzero real parts) goes through LDS to whole words, and only the
+  // rows that hold something read their counts and divide.
+  __device__ bool flags() const { return otf != nullptr; }
+  __device__ void store_flags(int z, int y0, int n, const uint8_t* f) const {
+    uint8_t* o = otf + ((size_t)z * V + y0) * V;
+    if ((uintptr_t)o % 16 == 0 && n * V % 16 == 0) {  // uniform
+      for (int i = threadIdx.x; i < n * V / 16; i += blockDim.x)
+        ((uint4*)o)[i] = f ? ((const uint4*)f)[i] : make_uint4(0, 0, 0, 0);
+    } else {
+      for (int i = threadIdx.x; i < n * V; i += blockDim.x) o[i] = f ? f[i] : 0;
+    }
+  }
   __device__ bool keep(int z, int y0, int n, bool any) const {
     for (int i = threadIdx.x; i < n; i += blockDim.x) occ[(size_t)z * V + y0 + i] = any;
-    if (any && threadIdx.x == 0) {
-      atomicMin(&found->x, z);
-      atomicMax(&found->y, z);
-    }
     return any;
   }
-  __device__ float2 load(int z, int y, int x) const {
-    const size_t i = ((size_t)z * V + y) * V + x;
-    if (prenorm) {  // already t * (-1)^(x+y+z)
-      const float2 t = vol[i];
-      if (otf) otf[i] = (t.x != 0.f) ? 1 : 0;
-      return t;
-    }
-    const float2 v = vol[i];
-    const int c0 = cnt[i];
+  __device__ float2 raw(int z, int y, int x) const { return vol[((size_t)z * V + y) * V + x]; }
+  __device__ float2 value(float2 v, int z, int y, int x) const {
+    if constexpr (!SCAN) return v;
+    const int c0 = cnt[((size_t)z * V + y) * V + x];
     const float c = (float)(c0 == 0 ? 1 : c0);
-    float2 t = make_float2(v.x / c, v.y / c);
-    if (otf) otf[i] = (t.x != 0.f) ? 1 : 0;
-    if ((x + y + z) & 1) { t.x = -t.x; t.y = -t.y; }
+    const float2 t = make_float2(v.x / c, v.y / c);
+    return (x + y + z) & 1 ? make_float2(-t.x, -t.y) : t;
+  }
+  __device__ float2 load(int z, int y, int x) const {
+    const float2 t = value(raw(z, y, x), z, y, x);
+    if (SCAN && otf) otf[((size_t)z * V + y) * V + x] = (t.x != 0.f) ? 1 : 0;
     return t;
   }
   __device__ void store(int z, int y, int x, float2 v) const {
@@ -742,18 +790,25 @@ struct NormXOp {  // rows along x; a = z, line = y
   Dim<VT> V{};
 };
 
-template <int VT>
+// OCC: rows with occ 0 hold zeros and are not read. (At run time instead, a branch
+// around every load: dense 1024^3 spectra 3.5 -> 7.4 ms.)
+template <int VT, bool OCC>
 struct PlaneYOp {  // columns of each z plane; a = z, col = x, row = y
   static constexpr int kColThreads = 512;  // complex in and out
   static constexpr bool kBalancedCols = true;
   float2* buf;
   const float2* tw;
   const int2* band;
-  const uint8_t* occ;  // rows with occ 0 hold zeros and are not read; nullptr: none
+  const uint8_t* occ;
   __device__ bool skip(int z) const { return outside_band(band, z); }
   __device__ void begin(int) {}
   __device__ float2 load(int z, int x, int y) const {
-    if (occ && !occ[(size_t)z * V + y]) return make_float2(0.f, 0.f);
+    if constexpr (OCC) {
+      // a plane's view: an empty row's lanes read out of its range, without a
+      // branch that would end the batch of loads
+      const BufView p(buf + (size_t)z * V * V, (unsigned)V * V * sizeof(float2));
+      return p.f2(occ[(size_t)z * V + y] ? ((unsigned)y * V + x) * sizeof(float2) : ~0u, 0);
+    }
     return buf[((size_t)z * V + y) * V + x];
   }
   __device__ void store(int z, int x, int y, float2 v) const { buf[((size_t)z * V + y) * V + x] = v; }
@@ -893,21 +948,28 @@ static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, i
 }
 
 template <int VT>
-static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt, int prenorm,
+static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt,
                              int2* band, uint8_t* occ, int planes, float2* work,
                              float df3, float cte, float gsign, float* re,
                              float* im, uint8_t* otf, const FftTab& ft, int2 tiles,
                              hipStream_t s) {
-  if (occ) {
-    Timed tm("vol_band", s);
-    hipLaunchKernelGGL(k_band_start, dim3(1), dim3(1), 0, s, (int)V, band);
-  }
-  NormXOp<VT> x{vol, cnt, work, otf, ft.tw, prenorm, occ ? nullptr : band, occ, band, V};
-  PlaneYOp<VT> y{work, ft.tw, band, occ, V};
   ZOutOp<VT> z{work, re, im, ft.tw, df3, cte, gsign, band, 0, 0, V - 1, V};
   hipError_t e;
-  if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
-  if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
+  if (occ) {
+    NormXOp<VT, true> x{vol, cnt, work, otf, ft.tw, nullptr, occ, V};
+    if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
+    Timed tm("vol_band", s);
+    hipLaunchKernelGGL(k_band_found, dim3(1), dim3(kBandThreads), 0, s, (const uint4*)occ, (int)V,
+                       band);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    PlaneYOp<VT, true> y{work, ft.tw, band, occ, V};
+    if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
+  } else {
+    NormXOp<VT, false> x{vol, cnt, work, otf, ft.tw, band, nullptr, V};
+    if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
+    PlaneYOp<VT, false> y{work, ft.tw, band, nullptr, V};
+    if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
+  }
   return vol_z<VT>(V, z, planes, ft, tiles.y, s);
 }
 
@@ -972,7 +1034,7 @@ static hipError_t contrast_spectrum_v(Dim<VT> V, const float* re, const float* i
                                       float scale, const int2* band, const FftTab& ft,
                                       hipStream_t s) {
   ContrastZOp<VT> z{re, im, work, ft.tw, band, 0, V - 1, V};
-  PlaneYOp<VT> y{work, ft.tw, band, nullptr, V};
+  PlaneYOp<VT, false> y{work, ft.tw, band, nullptr, V};
   SpectrumXOp<VT> x{work, ft.tw, scale, band, V};
   hipError_t e;
   if ((e = vol_cols<VT, false, false>(V, z, ft, "fwd_vol_z", 0, s)) != hipSuccess) return e;
@@ -1047,18 +1109,18 @@ k_cap_weights(const int32_t* __restrict__ cnt, const AngleGeo* __restrict__ ageo
   X(1024)
 
 hipError_t launch_finalize(int V, const float2* vol, const int32_t* cnt,
-                           int prenorm, int2* band, uint8_t* occ, int planes, float2* work,
-                           float df3, float cte, float gsign, float* out_re, float* out_im,
+                           int2* band, uint8_t* occ, int planes, float2* work, float df3,
+                           float cte, float gsign, float* out_re, float* out_im,
                            uint8_t* otf, const FftTab& ft, int2 tiles, hipStream_t s) {
   switch (V) {
 #define X(n)                                                                                   \
   case n:                                                                                      \
-    return finalize_v<n>(Dim<n>{}, vol, cnt, prenorm, band, occ, planes, work, df3, cte, gsign, \
+    return finalize_v<n>(Dim<n>{}, vol, cnt, band, occ, planes, work, df3, cte, gsign, \
                          out_re, out_im, otf, ft, tiles, s);
     MTD_VOL_SIZES(X)
 #undef X
   }
-  return finalize_v<0>(Dim<0>(V), vol, cnt, prenorm, band, occ, planes, work, df3, cte, gsign,
+  return finalize_v<0>(Dim<0>(V), vol, cnt, band, occ, planes, work, df3, cte, gsign,
                        out_re, out_im, otf, ft, tiles, s);
 }
 

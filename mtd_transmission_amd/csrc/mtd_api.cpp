@@ -1423,7 +1423,7 @@ int mtd_ewald_accumulate(mtd_ctx* ctx, const mtd_geom* g, const float* fields,
 
 // scale > 0: output factor in place of delta_f^3 * (-1/(2 n0 kv^2)).
 static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
-                         const int32_t* counts, int prenorm, int2* band, float* index_re,
+                         const int32_t* counts, int2* band, float* index_re,
                          float* index_im, uint8_t* otf, double scale = 0) {
   const int V = g->dim_final;
   float2* work = (float2*)ws_get(ctx, WS_VWORK, (size_t)V * V * V * sizeof(float2));
@@ -1432,7 +1432,7 @@ static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
   uint8_t* occ = nullptr;
   if (!band) {
     band = (int2*)ws_get(ctx, WS_BAND, sizeof(int2));
-    occ = (uint8_t*)ws_get(ctx, WS_OCC, (size_t)V * V);
+    occ = (uint8_t*)ws_get(ctx, WS_OCC, ((size_t)V * V + 15) / 16 * 16);
     if (!band || !occ) return set_err(ctx, MTD_ERR_HIP, "out of device memory (volume band)");
   }
   if (!work || !tabs) return set_err(ctx, MTD_ERR_HIP, "out of device memory (volume work)");
@@ -1445,7 +1445,7 @@ static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
   // the caps of illuminations inside the pupil span this many planes
   const double R = g->rayon, nx = g->nxmax;
   const int planes = occ ? 0 : 2 * (int)std::ceil(R - std::sqrt(std::max(R * R - nx * nx, 0.0))) + 1;
-  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, prenorm, band, occ, planes,
+  return hip_check(ctx, launch_finalize(V, (const float2*)vol, counts, band, occ, planes,
                                         work, df3, (float)cte, gsign, index_re, index_im, otf, twV,
                                         make_int2(ctx->vol_rows_tile, ctx->vol_cols_tile),
                                         ctx->stream),
@@ -1457,7 +1457,7 @@ int mtd_finalize(mtd_ctx* ctx, const mtd_geom* g, const float* vol, const int32_
   CtxScope scope(ctx);
   MTD_TRY(validate(ctx, g, 0, NEED_VOL));
   if (!vol || !counts || !index_re || !index_im) return set_err(ctx, MTD_ERR_ARG, "null array");
-  return finalize_impl(ctx, g, vol, counts, 0, nullptr, index_re, index_im, otf);
+  return finalize_impl(ctx, g, vol, counts, nullptr, index_re, index_im, otf);
 }
 
 // ---- Born forward model and its adjoint ----------------------------------
@@ -1585,7 +1585,7 @@ static int adjoint_impl(mtd_ctx* ctx, const mtd_geom* g, const float* spectra,
                          pre ? 4 | 2 : 4, band, t.q));
   }
   const double tp = tomo_pixel(g);
-  return finalize_impl(ctx, g, (const float*)vol, nullptr, 1, band, out_re, out_im, nullptr,
+  return finalize_impl(ctx, g, (const float*)vol, nullptr, band, out_re, out_im, nullptr,
                        tp * tp * tp);
 }
 
@@ -1787,7 +1787,7 @@ int mtd_reconstruct_plain(mtd_ctx* ctx, const mtd_geom* g, const void* holos, in
   // only in the height band that holds hits; the inverse transform treats the
   // rest as the zeros it is and never reads it.
   MTD_TRY(scatter_impl(ctx, g, F, 0, pos, A, (float*)vol, nullptr, 1 | 2, band));
-  return finalize_impl(ctx, g, (const float*)vol, nullptr, 1, band, index_re, index_im, nullptr);
+  return finalize_impl(ctx, g, (const float*)vol, nullptr, band, index_re, index_im, nullptr);
 }
 
 // ---------------------------------------------------------------------------

@@ -155,21 +155,26 @@ struct has_line : std::false_type {};
 template <class Op>
 struct has_line<Op, std::void_t<decltype(std::declval<Op&>().line(0, 0))>> : std::true_type {};
 
-// An operation may define keep(batch, first line, lines, any), called once by
-// every thread of a row block after its loads, with whether any loaded value
-// of the block's lines is not zero (NaN is not zero): the block then leaves
-// its lines alone when it returns false.
+// An operation with a static constexpr bool kScans = true defines keep(batch,
+// first line, lines, any), called once by every thread of a row block after its
+// loads, with whether any value of the block's lines is not zero (NaN is not
+// zero): the block then leaves its lines alone when it returns false. The
+// compiled row pass scans what raw(batch, line, element) reads, and makes the
+// transform's input of it with value(raw, batch, line, element) only if the block
+// goes on; where flags() holds, store_flags(batch, first line, lines, bytes) gets
+// a byte per element, 1 where the input's real part is not zero (nullptr:
+// nowhere).
 template <class Op, class = void>
-struct has_keep : std::false_type {};
+struct op_scans : std::false_type {};
 template <class Op>
-struct has_keep<Op, std::void_t<decltype(std::declval<const Op&>().keep(0, 0, 0, false))>>
-    : std::true_type {};
+struct op_scans<Op, std::void_t<decltype(Op::kScans)>>
+    : std::integral_constant<bool, Op::kScans> {};
 
 template <int L, bool INV, class Op, int TV = 0>
 __global__ void __launch_bounds__(256) k_rows(Op op) {
   using F = Fft2<L, INV>;
   constexpr int NT = rows_nt_tv<L, TV>();
-  __shared__ float lds[NT * F::LDS_ROW];
+  __shared__ __attribute__((aligned(16))) float lds[NT * F::LDS_ROW];
   const int2 ab = xcd_block();
   const int a = ab.x;
   if (skip_batch(op, a)) return;  // block-uniform, before the barrier
@@ -178,14 +183,28 @@ __global__ void __launch_bounds__(256) k_rows(Op op) {
   op.begin(a);
   if constexpr (has_line<Op>::value) op.line(a, line);
   float2 v[F::L1], u[F::L2];
+  if constexpr (!op_scans<Op>::value) {
 #pragma unroll
-  for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.load(a, line, F::L2 * n1 + n2);
-  if constexpr (has_keep<Op>::value) {
-    if (op.scans()) {  // uniform
-      bool any = false;
+    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.load(a, line, F::L2 * n1 + n2);
+  } else {
+    bool any = false;
 #pragma unroll
-      for (int n1 = 0; n1 < F::L1; ++n1) any = any || v[n1].x != 0.f || v[n1].y != 0.f;
-      if (!op.keep(a, ab.y * NT, NT, __syncthreads_or(any))) return;  // block-uniform
+    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.raw(a, line, F::L2 * n1 + n2);
+#pragma unroll
+    for (int n1 = 0; n1 < F::L1; ++n1) any = any || v[n1].x != 0.f || v[n1].y != 0.f;
+    any = __syncthreads_or(any);
+    const bool flags = op.flags();  // uniform
+    if (flags && !any) op.store_flags(a, ab.y * NT, NT, nullptr);
+    if (!op.keep(a, ab.y * NT, NT, any)) return;  // block-uniform
+#pragma unroll
+    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.value(v[n1], a, line, F::L2 * n1 + n2);
+    if (flags) {
+      uint8_t* f = (uint8_t*)lds;
+#pragma unroll
+      for (int n1 = 0; n1 < F::L1; ++n1) f[r * L + F::L2 * n1 + n2] = v[n1].x != 0.f;
+      __syncthreads();
+      op.store_flags(a, ab.y * NT, NT, f);
+      __syncthreads();
     }
   }
   F::run(v, u, n2, typename F::Row{lds + r * F::LDS_ROW}, op.tw);
