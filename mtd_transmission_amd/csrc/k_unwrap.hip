@@ -42,7 +42,7 @@
 // 52 bytes per pixel bound the passes. The same method on the 2C x 2C extension
 // (half-empty transforms, both gradients with their trigonometry on every
 // pixel three times) moved about 300. Measured, all unwrapping kernels, that
-// form against this one: 300 crops of 250^2 3217 -> 610 us, 400 of 128^2 813 ->
+// form against this one: 300 crops of 250^2 3217 -> 536 us, 400 of 128^2 813 ->
 // 144 us, 48 of 182^2 (runtime-length FFTs) 986 -> 182 us.
 #include <cfloat>
 
@@ -162,14 +162,17 @@ __device__ __forceinline__ void line_gradient(const float2 (&z)[Fft2<C, false>::
   for (int n1 = 0; n1 < F::L1; ++n1) g[n1] = v[n1].y * z[n1].x - v[n1].x * z[n1].y;
 }
 
-// Column blocks: NC adjacent columns, 32 where that keeps the block within
-// MAXT threads and divides C, else 16 (the last block may run past C). The
+// Column blocks: NC adjacent columns, the most of 32 (where it divides C), 16 and
+// 8 that keep the block within MAXT threads (the last block may run past C). The
 // gradient passes hold a line's phasors beside a transform: waves per SIMD
 // that leave them in registers (at 4 waves, crops of 160 to 256 spilled up to
-// 138 of them), in blocks of at most 256 threads so that 3 fit.
+// 138 of them), in blocks of at most 256 threads so that 3 fit: with 16 columns a
+// 250-line block had 7 waves of the CU's 12, and one block was all that fit
+// (300 crops: 321 -> 247 us with 8).
 template <int C, int MAXT>
 constexpr int unw_nc() {
-  return 32 * Fft2<C, false>::T <= MAXT && C % 32 == 0 ? 32 : 16;
+  constexpr int T = Fft2<C, false>::T;
+  return 32 * T <= MAXT && C % 32 == 0 ? 32 : 16 * T <= MAXT ? 16 : 8;
 }
 template <int C, int MAXT>
 constexpr int unw_threads() {
