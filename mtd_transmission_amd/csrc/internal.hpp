@@ -309,8 +309,9 @@ hipError_t launch_angle_geo(const int* posx, const int* posy, int A, int nxmax,
                             AngleGeo* ageo, hipStream_t s);
 // Height band [band.x, band.y] that holds every hit of the non-skipped angles
 // (empty: x > y), from the pupil's extreme radii.
-hipError_t launch_band(const AngleGeo* ageo, int A, int V, const double* htab, int r2max,
-                       int2* band, hipStream_t s);
+hipError_t launch_geo_band(const int* posx, const int* posy, int A, int nxmax, double R2,
+                           const double* htab, int r2tab, AngleGeo* ageo, int V, int r2max,
+                           int2* band, hipStream_t s);
 // band == nullptr: every voxel of the volume (and counts) is written;
 // otherwise only the planes of the band are, and [zlo, zhi] is a host-side
 // bound of the band (only height windows meeting it are launched).

@@ -36,12 +36,10 @@ __device__ __forceinline__ double round_away(double x) {
   return (fabs(x - t) >= 0.5) ? t + copysign(1.0, x) : t;
 }
 
-__global__ void k_angle_geo(const int* __restrict__ posx,
-                            const int* __restrict__ posy, int A, int nx,
-                            double R2, const double* __restrict__ htab,
-                            int r2tab, AngleGeo* __restrict__ ageo) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= A) return;
+__device__ __forceinline__ AngleGeo angle_geo(const int* __restrict__ posx,
+                                             const int* __restrict__ posy, int a, int nx,
+                                             double R2, const double* __restrict__ htab,
+                                             int r2tab) {
   AngleGeo g;
   g.fx = posx[a] - nx;
   g.fy = posy[a] - nx;
@@ -50,7 +48,15 @@ __global__ void k_angle_geo(const int* __restrict__ posx,
   g.skip = round_away(fz2) < 0.0;
   g.pad = 0;
   g.fz = (!g.skip && r2 < r2tab) ? htab[r2] : 0.0;
-  ageo[a] = g;
+  return g;
+}
+
+__global__ void k_angle_geo(const int* __restrict__ posx,
+                            const int* __restrict__ posy, int A, int nx,
+                            double R2, const double* __restrict__ htab,
+                            int r2tab, AngleGeo* __restrict__ ageo) {
+  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a < A) ageo[a] = angle_geo(posx, posy, a, nx, R2, htab, r2tab);
 }
 
 struct GatherArgs {
@@ -498,38 +504,48 @@ hipError_t launch_angle_geo(const int* posx, const int* posy, int A, int nxmax,
   return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256)
-k_band(const AngleGeo* __restrict__ ageo, int A, int V, const double* __restrict__ htab,
-       int r2max, int2* __restrict__ band) {
-  __shared__ int red[2][4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// The angle table and the hit band in one launch: a single block, since a launch
+// costs more than the angles (600 angles: 4.7 us each for the two, a call on
+// small volumes has about 15 launches).
+constexpr int kGeoThreads = 1024;
+__global__ void __launch_bounds__(kGeoThreads)
+k_geo_band(const int* __restrict__ posx, const int* __restrict__ posy, int A, int nx, double R2,
+           const double* __restrict__ htab, int r2tab, AngleGeo* __restrict__ ageo, int V,
+           int r2max, int2* __restrict__ band) {
+  __shared__ int2 red[kGeoThreads / 64];
+  const int tid = threadIdx.x;
   int lo = 0x7fffffff, hi = -0x7fffffff;
-  for (int a = tid; a < A; a += 256) {
-    const AngleGeo ag = ageo[a];
+  const double rim = htab[r2max], top = htab[0];
+  for (int a = tid; a < A; a += kGeoThreads) {
+    const AngleGeo ag = angle_geo(posx, posy, a, nx, R2, htab, r2tab);
+    ageo[a] = ag;
     if (ag.skip) continue;
     // hits of angle a lie between the heights at the pupil's rim and centre
-    lo = min(lo, (int)round_away(htab[r2max] - ag.fz) + V / 2);
-    hi = max(hi, (int)round_away(htab[0] - ag.fz) + V / 2);
+    lo = min(lo, (int)round_away(rim - ag.fz) + V / 2);
+    hi = max(hi, (int)round_away(top - ag.fz) + V / 2);
   }
   for (int o = 32; o > 0; o >>= 1) {
     lo = min(lo, __shfl_xor(lo, o, 64));
     hi = max(hi, __shfl_xor(hi, o, 64));
   }
-  if (lane == 0) { red[0][wave] = lo; red[1][wave] = hi; }
+  if (tid % 64 == 0) red[tid / 64] = make_int2(lo, hi);
   __syncthreads();
-  if (tid == 0) {
-    lo = min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3]));
-    hi = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
-    lo = max(lo, 0);
-    hi = min(hi, V - 1);
-    band[0] = lo <= hi ? make_int2(lo, hi) : make_int2(1, 0);
+  if (tid) return;
+  for (int w = 1; w < kGeoThreads / 64; ++w) {
+    lo = min(lo, red[w].x);
+    hi = max(hi, red[w].y);
   }
+  lo = max(lo, 0);
+  hi = min(hi, V - 1);
+  band[0] = lo <= hi ? make_int2(lo, hi) : make_int2(1, 0);
 }
 
-hipError_t launch_band(const AngleGeo* ageo, int A, int V, const double* htab, int r2max,
-                       int2* band, hipStream_t s) {
+hipError_t launch_geo_band(const int* posx, const int* posy, int A, int nxmax, double R2,
+                           const double* htab, int r2tab, AngleGeo* ageo, int V, int r2max,
+                           int2* band, hipStream_t s) {
   Timed tm("ewald_band", s);
-  hipLaunchKernelGGL(k_band, dim3(1), dim3(256), 0, s, ageo, A, V, htab, r2max, band);
+  hipLaunchKernelGGL(k_geo_band, dim3(1), dim3(kGeoThreads), 0, s, posx, posy, A, nxmax, R2, htab,
+                     r2tab, ageo, V, r2max, band);
   return hipGetLastError();
 }
 

@@ -1358,12 +1358,13 @@ static int scatter_impl(mtd_ctx* ctx, const mtd_geom* g, const float2* spec, int
     AngleGeo* agw = (AngleGeo*)ws_get(ctx, WS_AGEO, (size_t)std::max(A, 1) * sizeof(AngleGeo));
     scratch = ws_get(ctx, WS_GATHER, gather_scratch_bytes(g->dim_final, A));
     if (!agw || !scratch) return set_err(ctx, MTD_ERR_HIP, "out of device memory (angle table)");
-    if (A > 0)
+    if (band)
+      MTD_TRY(hip_check(ctx, launch_geo_band(posspec, posspec + A, A, g->nxmax, t.R2, t.htab,
+                                             t.r2tab, agw, g->dim_final, t.r2max, band,
+                                             ctx->stream), "angle geometry and hit band"));
+    else if (A > 0)
       MTD_TRY(hip_check(ctx, launch_angle_geo(posspec, posspec + A, A, g->nxmax, t.R2, t.htab,
                                               t.r2tab, agw, ctx->stream), "angle geometry"));
-    if (band)
-      MTD_TRY(hip_check(ctx, launch_band(agw, A, g->dim_final, t.htab, t.r2max, band,
-                                         ctx->stream), "hit band"));
     ag = agw;
   }
   // Host-side bound of the hit band: heights h(r2) - fz with h(r2) in
@@ -1474,11 +1475,13 @@ static int call_geometry(mtd_ctx* ctx, const mtd_geom* g, const int32_t* posspec
   AngleGeo* ag = (AngleGeo*)ws_get(ctx, WS_AGEO, (size_t)std::max(A, 1) * sizeof(AngleGeo));
   int2* band = (int2*)ws_get(ctx, WS_BAND, sizeof(int2));
   if (!ag || !band) return set_err(ctx, MTD_ERR_HIP, "out of device memory (angle table)");
-  MTD_TRY(hip_check(ctx, launch_angle_geo(posspec, posspec + A, A, g->nxmax, t.R2, t.htab,
-                                          t.r2tab, ag, ctx->stream), "angle geometry"));
   if (with_band)
-    MTD_TRY(hip_check(ctx, launch_band(ag, A, g->dim_final, t.htab, t.r2max, band, ctx->stream),
-                      "hit band"));
+    MTD_TRY(hip_check(ctx, launch_geo_band(posspec, posspec + A, A, g->nxmax, t.R2, t.htab, t.r2tab,
+                                           ag, g->dim_final, t.r2max, band, ctx->stream),
+                      "angle geometry and hit band"));
+  else
+    MTD_TRY(hip_check(ctx, launch_angle_geo(posspec, posspec + A, A, g->nxmax, t.R2, t.htab,
+                                            t.r2tab, ag, ctx->stream), "angle geometry"));
   b->pos = posspec;
   b->ag = ag;
   b->band = band;
@@ -1506,9 +1509,9 @@ int mtd_born_plan(mtd_ctx* ctx, const mtd_geom* g, const int32_t* posspec, int A
   MTD_TRY(hip_check(ctx, hipMemcpyAsync(pos, posspec, (size_t)2 * A * sizeof(int32_t),
                                         hipMemcpyDeviceToDevice, ctx->stream),
                     "plan speculars"));
-  MTD_TRY(hip_check(ctx, launch_angle_geo(pos, pos + A, A, g->nxmax, t.R2, t.htab, t.r2tab, ag,
-                                          ctx->stream), "angle geometry"));
-  MTD_TRY(hip_check(ctx, launch_band(ag, A, V, t.htab, t.r2max, band, ctx->stream), "hit band"));
+  MTD_TRY(hip_check(ctx, launch_geo_band(pos, pos + A, A, g->nxmax, t.R2, t.htab, t.r2tab, ag, V,
+                                         t.r2max, band, ctx->stream),
+                    "angle geometry and hit band"));
   MTD_TRY(hip_check(ctx, launch_gather_prepass(ag, A, 2 * g->nxmax, g->nxmax, V, t.htab,
                                                t.r2max, scratch, ctx->stream),
                     "gather prepass"));
