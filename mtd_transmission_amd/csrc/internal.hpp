@@ -338,8 +338,6 @@ hipError_t launch_contrast_spectrum(int V, const float* re, const float* im, flo
                                    hipStream_t s);
 // One fused FISTA step with the smoothed TV gradient (k_tv.hip).
 hipError_t launch_stamp(unsigned long long* out, hipStream_t s);
-hipError_t launch_residual(float2* S, const float2* y, const float* w, const float* q2, int A,
-                           int C2, hipStream_t s);
 hipError_t launch_tv_start(float* x, float* z, size_t n, int positivity, hipStream_t s);
 hipError_t launch_tv_fista(int V, const float* z, const float* gd, float* x, float* zn,
                            float sd, float lam, float eps, float step, float beta,
@@ -348,10 +346,11 @@ hipError_t launch_tv_fista(int V, const float* z, const float* gd, float* x, flo
 hipError_t launch_cap_weights(const int32_t* cnt, const AngleGeo* ageo, int A,
                               const double* htab, const float* q, int r2max, int nx, int C,
                               int V, float* w, hipStream_t s);
-// Per-angle cap samples -i q(|fd|^2) vol[voxel] into spec[A][C][C] (+posSpec frame).
+// Per-angle cap samples -i q(|fd|^2) vol[voxel] into spec[A][C][C] (+posSpec frame);
+// y: the weighted residual q w (samples - y) instead (w NULL: 1).
 hipError_t launch_cap_sample(const float2* vol, const AngleGeo* ageo, int A, const double* htab,
-                             const float* q2, int r2max, int nx, int C, int V, float2* spec,
-                             hipStream_t s);
+                             const float* q2, int r2max, int nx, int C, int V, const float2* y,
+                             const float* w, float2* spec, hipStream_t s);
 // band: heights outside it are zero and are not read; vol is then already divided
 // by its counts and centring-signed (gather flag 1). occ != nullptr (V^2 bytes,
 // rounded up to 16): the band is not known and is found by the first pass into

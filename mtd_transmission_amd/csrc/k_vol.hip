@@ -1066,30 +1066,71 @@ static hipError_t contrast_spectrum_v(Dim<VT> V, const float* re, const float* i
 // outside the pupil, of skipped angles, or whose height leaves the volume
 // are 0, and so are bins whose voxel would leave the volume laterally (a
 // caller's specular outside the crop; the accumulation has no hit there).
-__global__ void __launch_bounds__(256)
-k_cap_sample(const float2* __restrict__ vol, const AngleGeo* __restrict__ ageo,
+// With RES the solver's weighted residual is stored instead, q * w * (S - y) (w
+// NULL: 1; the real factors applied one after the other): q is the factor the
+// adjoint's gather would apply per hit, so the adjoint can skip it. Bins that no
+// cap reads are 0 there, and their y and w are not read. One pass in place of
+// two: 400 angles of 128^2, 43 + 35 -> 55 us (blocks of 256 columns left half of
+// the threads without a bin there).
+constexpr int kCapX = 64, kCapY = 4;
+constexpr int kCapA = 8;  // angles a thread samples, their loads in flight together
+template <bool RES>
+__global__ void __launch_bounds__(kCapX * kCapY)
+k_cap_sample(const float2* __restrict__ vol, const AngleGeo* __restrict__ ageo, int A,
              const double* __restrict__ htab, const float* __restrict__ q2, int r2max, int nx,
-             int C, int V, float2* __restrict__ spec) {
-  // grid (column blocks, rows, angles): no division by the runtime C; the
-  // forward factor is read from the C x C pupil-frame table (coalesced)
-  const int a = blockIdx.z, row = blockIdx.y;
-  const int col = blockIdx.x * 256 + threadIdx.x;
-  if (col >= C) return;
-  const int i = row * C + col;
+             int C, int V, const float2* __restrict__ y, const float* __restrict__ w,
+             float2* __restrict__ spec) {
+#pragma clang fp contract(off)
+  // grid (column blocks, row blocks, angle groups): no division by the runtime
+  // C; the forward factor is read from the C x C pupil-frame table (coalesced)
+  const int col = blockIdx.x * kCapX + threadIdx.x, row = blockIdx.y * kCapY + threadIdx.y;
+  if (col >= C || row >= C) return;
+  const int a0 = blockIdx.z * kCapA, i = row * C + col;
+  const size_t C2 = (size_t)C * C;
   const int fdx = col - nx, fdy = row - nx;
   const int r2 = fdx * fdx + fdy * fdy;
-  const AngleGeo ag = ageo[a];
-  float2 s = make_float2(0.f, 0.f);
-  if (!ag.skip && r2 <= r2max) {
-    const int z = (int)round_away(htab[r2] - ag.fz) + V / 2;
-    const int X = fdx - ag.fx + V / 2, Y = fdy - ag.fy + V / 2;
-    if (z >= 0 && z < V && X >= 0 && X < V && Y >= 0 && Y < V) {
-      const float2 t = vol[((size_t)z * V + Y) * V + X];
-      const float w = q2[i];
-      s = make_float2(w * t.y, -(w * t.x));
-    }
+  if (r2 > r2max) {
+    for (int a = a0; a < min(a0 + kCapA, A); ++a) spec[a * C2 + i] = make_float2(0.f, 0.f);
+    return;
   }
-  spec[(size_t)a * C * C + i] = s;
+  const double h = htab[r2];
+  const float q = q2[i];
+  // voxel 0 stands in for a bin without one, so that no load hangs on a branch
+  size_t vi[kCapA];
+  bool in[kCapA], live[kCapA];
+  float2 t[kCapA], m[kCapA];
+  float k[kCapA];
+#pragma unroll
+  for (int j = 0; j < kCapA; ++j) {
+    const AngleGeo ag = ageo[min(a0 + j, A - 1)];
+    const int z = (int)round_away(h - ag.fz) + V / 2;
+    const int X = fdx - ag.fx + V / 2, Y = fdy - ag.fy + V / 2;
+    live[j] = !ag.skip;
+    in[j] = !ag.skip && z >= 0 && z < V && X >= 0 && X < V && Y >= 0 && Y < V;
+    vi[j] = in[j] ? ((size_t)z * V + Y) * V + X : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < kCapA; ++j) {
+    t[j] = vol[vi[j]];
+    if constexpr (RES) m[j] = y[min(a0 + j, A - 1) * C2 + i];
+  }
+  if (RES && w) {  // uniform
+#pragma unroll
+    for (int j = 0; j < kCapA; ++j) k[j] = w[min(a0 + j, A - 1) * C2 + i];
+  } else {
+#pragma unroll
+    for (int j = 0; j < kCapA; ++j) k[j] = 1.f;
+  }
+#pragma unroll
+  for (int j = 0; j < kCapA; ++j) {
+    if (a0 + j >= A) break;  // uniform
+    float2 s = in[j] ? make_float2(q * t[j].y, -(q * t[j].x)) : make_float2(0.f, 0.f);
+    if constexpr (RES) {
+      s = live[j] ? make_float2((s.x - m[j].x) * k[j] * q, (s.y - m[j].y) * k[j] * q)
+                  : make_float2(0.f, 0.f);
+    }
+    spec[(a0 + j) * C2 + i] = s;
+  }
 }
 
 // Data weights of the adjoint-iterative form: w = 1 / (q(|fd|^2)^2 * hits of
@@ -1153,12 +1194,18 @@ hipError_t launch_contrast_spectrum(int V, const float* re, const float* im, flo
 }
 
 hipError_t launch_cap_sample(const float2* vol, const AngleGeo* ageo, int A, const double* htab,
-                             const float* q2, int r2max, int nx, int C, int V, float2* spec,
-                             hipStream_t s) {
+                             const float* q2, int r2max, int nx, int C, int V, const float2* y,
+                             const float* w, float2* spec, hipStream_t s) {
   Timed tm("cap_sample", s);
   if (A <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_cap_sample, dim3((C + 255) / 256, C, A), dim3(256), 0, s, vol, ageo,
-                     htab, q2, r2max, nx, C, V, spec);
+  const dim3 grid((C + kCapX - 1) / kCapX, (C + kCapY - 1) / kCapY, (A + kCapA - 1) / kCapA),
+      block(kCapX, kCapY);
+  if (y)
+    hipLaunchKernelGGL((k_cap_sample<true>), grid, block, 0, s, vol, ageo, A, htab, q2, r2max, nx, C,
+                       V, y, w, spec);
+  else
+    hipLaunchKernelGGL((k_cap_sample<false>), grid, block, 0, s, vol, ageo, A, htab, q2, r2max, nx, C,
+                       V, nullptr, nullptr, spec);
   return hipGetLastError();
 }
 

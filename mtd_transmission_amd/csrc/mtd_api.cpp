@@ -1521,9 +1521,10 @@ int mtd_born_plan(mtd_ctx* ctx, const mtd_geom* g, const int32_t* posspec, int A
   return MTD_OK;
 }
 
-int mtd_forward_spectra(mtd_ctx* ctx, const mtd_geom* g, const float* dn_re, const float* dn_im,
-                        const int32_t* posspec, int A, float* spectra) {
-  CtxScope scope(ctx);
+// y: the solver's weighted residual q w (spectra - y) in place of the spectra
+static int forward_impl(mtd_ctx* ctx, const mtd_geom* g, const float* dn_re, const float* dn_im,
+                        const int32_t* posspec, int A, const float* y, const float* w,
+                        float* spectra) {
   MTD_TRY(validate(ctx, g, A, NEED_VOL));
   if (A == 0) return MTD_OK;
   if (!dn_re || !spectra) return set_err(ctx, MTD_ERR_ARG, "null array");
@@ -1545,8 +1546,14 @@ int mtd_forward_spectra(mtd_ctx* ctx, const mtd_geom* g, const float* dn_re, con
                                                   ctx->stream),
                     "contrast spectrum"));
   return hip_check(ctx, launch_cap_sample(work, geo.ag, A, t.htab, t.q2, t.r2max, g->nxmax, C, V,
-                                          (float2*)spectra, ctx->stream),
+                                          (const float2*)y, w, (float2*)spectra, ctx->stream),
                    "cap sampling");
+}
+
+int mtd_forward_spectra(mtd_ctx* ctx, const mtd_geom* g, const float* dn_re, const float* dn_im,
+                        const int32_t* posspec, int A, float* spectra) {
+  CtxScope scope(ctx);
+  return forward_impl(ctx, g, dn_re, dn_im, posspec, A, nullptr, nullptr, spectra);
 }
 
 // pre: the spectra already carry the forward factor q of their bin (the
@@ -1666,20 +1673,14 @@ int mtd_tv_fista_step(mtd_ctx* ctx, int V, const float* z, const float* grad_dat
 static int tv_loop(mtd_ctx* ctx, const mtd_geom* g, const float* y, const float* w, int A,
                    int n_iter, float lam, float eps, float inv_kappa, int positivity, float* x,
                    float* z, float* zn, float* gd, float* S) {
-  const int V = g->dim_final, C = 2 * g->nxmax;
+  const int V = g->dim_final;
   const size_t nv = (size_t)V * V * V;
   const float step = (float)(1.0 / (1.0 + 12.0 * (double)lam / (double)eps));
   MTD_TRY(hip_check(ctx, launch_tv_start(x, z, nv, positivity, ctx->stream), "solver start"));
   double t = 1.0;
-  EwaldTables et;
-  MTD_TRY(ewald_tables(ctx, g, &et));
-  MTD_TRY(born_weights(ctx, g, &et));
   for (int k = 1; k <= n_iter; ++k) {
-    MTD_TRY(mtd_forward_spectra(ctx, g, z, nullptr, nullptr, A, S));
     // W (S - y) times q: the adjoint's gather then takes the spectra as is
-    MTD_TRY(hip_check(ctx, launch_residual((float2*)S, (const float2*)y, w, et.q2, A, C * C,
-                                           ctx->stream),
-                      "residual"));
+    MTD_TRY(forward_impl(ctx, g, z, nullptr, nullptr, A, y, w, S));
     MTD_TRY(adjoint_impl(ctx, g, S, nullptr, A, gd, nullptr, true));
     const double tn = 0.5 * (1.0 + std::sqrt(1.0 + 4.0 * t * t));
     MTD_TRY(mtd_tv_fista_step(ctx, V, z, gd, x, zn, inv_kappa, lam, eps, step,
