@@ -355,7 +355,15 @@ k_form_field(const float2* __restrict__ iu, const float2* __restrict__ crop,
 // per-angle forward spectrum
 // G[y][x] = field_U[(y+NX)%C][(x+NX)%C] * w[(y+NX)%C] * w[(x+NX)%C]
 // ---------------------------------------------------------------------------
-template <int CT>
+// KIND: what the rows are made of, at compile time: a branch on it around each
+// load kept a line's loads from going out as one batch, and the other kinds'
+// code took registers. Fields, 400 of 250^2: 136 -> 111 us; unwrapped, 300 of 250^2:
+// 120 -> 98; in the fused row pass, 200 of 512^2: 465 -> 366 (212 -> 146 VGPRs), no
+// change at 256^2 and 128^2 but for the spills that are gone.
+constexpr int kFwdAny = -2;     // from_iu, mode and phu say
+constexpr int kFwdFields = -1;  // fields
+                                // >= 0: IU, mode in bits 0 and 1, bit 2: phu
+template <int CT, int KIND>
 struct FwdRowOp {
   const float2* src;      // fields (U frame) or IU
   const float2* crop;
@@ -374,16 +382,21 @@ struct FwdRowOp {
   int Y;
   double wy;
   RowPoly pp, pa;
+  __device__ __forceinline__ bool iu() const { return KIND == kFwdAny ? from_iu != 0 : KIND >= 0; }
+  __device__ __forceinline__ int md() const { return KIND < 0 ? mode : KIND & 3; }
+  __device__ __forceinline__ bool unw() const {
+    return KIND < 0 ? phu_a != nullptr : (KIND & 4) != 0;
+  }
   __device__ void begin(int a) {
     cph = coef + (size_t)a * 2 * NCOEF;
     phu_a = phu ? phu + (size_t)a * C * C : nullptr;
-    if (from_iu && !(mode & 2))
+    if (iu() && !(md() & 2))
       sn = spec_norm_of(crop + (size_t)a * C * C, C, posx[a], posy[a]);
   }
   __device__ void line(int, int y) {
     Y = (y + C / 2) % C;
     wy = win[Y];
-    if (from_iu && (mode & 2)) {
+    if (iu() && (md() & 2)) {
       pp = row_poly(cph, (double)Y);
       pa = row_poly(cph + NCOEF, (double)Y);
     }
@@ -393,20 +406,20 @@ struct FwdRowOp {
     const int X = (x + C / 2) % C;
     const float w = (float)(win[X] * wy);
     float2 f;
-    if (mode & 2) {
-      if (!phu_a && (mode & 1)) {
+    if (md() & 2) {
+      if (!unw() && (md() & 1)) {
         f = form_born_wrapped(u, row_poly_at(pp, (double)X), row_poly_at(pa, (double)X));
       } else {
-        const float phf = phu_a ? phu_a[Y * C + X] : atan2f(u.y, u.x);
-        f = form_from(u, phf, row_poly_at(pp, (double)X), row_poly_at(pa, (double)X), sn, mode);
+        const float phf = unw() ? phu_a[Y * C + X] : atan2f(u.y, u.x);
+        f = form_from(u, phf, row_poly_at(pp, (double)X), row_poly_at(pa, (double)X), sn, md());
       }
     } else {
-      f = form_from(u, 0.f, 0.0, 0.0, sn, mode);
+      f = form_from(u, 0.f, 0.0, 0.0, sn, md());
     }
     return make_float2(f.x * w, f.y * w);
   }
   __device__ float2 load(int a, int y, int x) const {
-    if (from_iu) return form_iu(x, src[((size_t)a * C + y) * C + x]);
+    if (iu()) return form_iu(x, src[((size_t)a * C + y) * C + x]);
     const int X = (x + C / 2) % C;
     const float w = (float)(win[X] * wy);
     const float2 f = src[((size_t)a * C + Y) * C + X];
@@ -486,10 +499,10 @@ struct QLoad {
   }
 };
 
-template <int CT>
+template <int CT, int KIND>
 struct QRowOp {
   QLoad<CT> ql;
-  FwdRowOp<CT> f;  // field formation, window and output (from_iu = 1)
+  FwdRowOp<CT, KIND> f;  // field formation, window and output (from_iu = 1)
   const float2* tw;
   __device__ void begin(int a) {
     ql.begin(a, f.C);
@@ -614,12 +627,23 @@ static hipError_t fwd_c(Dim<CT> C, const float2* src, int from_iu, const float2*
                         const int* posy, int A, const double* win,
                         const FftTab& ft, float dx2, int shift_pos, const float* beta2,
                         float2* work, float2* out, hipStream_t s) {
-  FwdRowOp<CT> r{src, crop, coef, posx, posy, win, work, ft.tw, from_iu, mode, phu,
-                 make_float2(0.f, 0.f), nullptr, nullptr};
-  r.C = C;
   FwdColOp<CT> c{work, out, posx, posy, ft.tw, dx2, shift_pos, beta2, 0, 0, 0, 0, C};
-  return rows_cols<CT, false>(C, r, c, A, ft, from_iu ? "fwd_rows_field" : "fwd_rows",
-                              "fwd_cols", s);
+  const char* rows = from_iu ? "fwd_rows_field" : "fwd_rows";
+#define MTD_FWD(K)                                                                           \
+  {                                                                                          \
+    FwdRowOp<CT, K> r{src, crop, coef, posx, posy, win, work, ft.tw, from_iu, mode, phu,     \
+                      make_float2(0.f, 0.f), nullptr, nullptr};                              \
+    r.C = C;                                                                                 \
+    return rows_cols<CT, false>(C, r, c, A, ft, rows, "fwd_cols", s);                        \
+  }
+  if (!from_iu) MTD_FWD(kFwdFields)
+  switch ((mode & 3) | (phu ? 4 : 0)) {
+    case 3: MTD_FWD(3)  // Born, wrapped
+    case 6: MTD_FWD(6)  // Rytov and Born, unwrapped
+    case 7: MTD_FWD(7)
+  }
+  MTD_FWD(kFwdAny)
+#undef MTD_FWD
 }
 
 template <int CT>
@@ -753,14 +777,18 @@ static hipError_t fused_c(const float2* q, const int* posx, const int* posy, int
   }
   hipError_t e = lsq_c<C>(Dim<C>{}, ius, nullptr, A, plan, coef, s, 1);
   if (e != hipSuccess) return e;
-  FwdRowOp<C> f{nullptr, nullptr, coef, posx, posy, win, work, tw, 1, mode, nullptr,
-                make_float2(0.f, 0.f), nullptr, nullptr};
-  QRowOp<C> r{QLoad<C>{q, posx, posy, tw, 0, make_float2(0.f, 0.f)}, f, tw};
-  {
-    Timed tm("fwd_rows_field", s);
-    hipLaunchKernelGGL((k_rows2<C, true, false, QRowOp<C>>), rows_grid<C>(A), rows_block<C>(), 0,
-                       s, r);
+  const QLoad<C> ql{q, posx, posy, tw, 0, make_float2(0.f, 0.f)};
+#define MTD_QROW(K)                                                                           \
+  {                                                                                           \
+    Timed tm("fwd_rows_field", s);                                                            \
+    FwdRowOp<C, K> f{nullptr, nullptr, coef, posx, posy, win, work, tw, 1, mode, nullptr,     \
+                     make_float2(0.f, 0.f), nullptr, nullptr};                                \
+    QRowOp<C, K> r{ql, f, tw};                                                                \
+    hipLaunchKernelGGL((k_rows2<C, true, false, QRowOp<C, K>>), rows_grid<C>(A),              \
+                       rows_block<C>(), 0, s, r);                                             \
   }
+  if ((mode & 3) == 3) MTD_QROW(3) else MTD_QROW(kFwdAny)
+#undef MTD_QROW
   FwdColOp<C> c{work, out, posx, posy, tw, dx2, 0, beta2, 0, 0, 0, 0};
   Timed tm("fwd_cols", s);
   hipLaunchKernelGGL((k_cols<C, false, FwdColOp<C>>), (cols_grid<C, FwdColOp<C>>(A)),
