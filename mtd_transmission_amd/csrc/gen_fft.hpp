@@ -152,7 +152,11 @@ __device__ __forceinline__ void gen_stockham(const GenLines& x, const GenPlan& p
 }
 
 // Forward transforms of the block's lines, in place (elements [0, L) of each).
-// Begins after the caller's barrier, ends with one.
+// Begins after the caller's barrier, ends with one. RAW (Bluestein): the lines
+// come times the chirp and with zeros from L to W, and are left without the
+// conjugate and the chirp of the way out (gen_out), which saves two round trips
+// through LDS.
+template <bool RAW = false>
 __device__ __forceinline__ void gen_fft(const GenLines& x, const GenPlan& p) {
   if (!p.chirp) {
     gen_stockham(x, p);
@@ -160,10 +164,12 @@ __device__ __forceinline__ void gen_fft(const GenLines& x, const GenPlan& p) {
   }
   const int L = p.L, W = p.W, l = threadIdx.x & (x.nl() - 1);
   const int n0 = threadIdx.x >> x.lnl, dn = blockDim.x >> x.lnl;
-  // x_n w_n, zero-padded to W
-  for (int n = n0; n < W; n += dn)
-    x.set(l, n, n < L ? cmul(x.get(l, n), p.chirp[n]) : make_float2(0.f, 0.f));
-  __syncthreads();
+  if (!RAW) {
+    // x_n w_n, zero-padded to W
+    for (int n = n0; n < W; n += dn)
+      x.set(l, n, n < L ? cmul(x.get(l, n), p.chirp[n]) : make_float2(0.f, 0.f));
+    __syncthreads();
+  }
 #pragma unroll 1
   for (int half = 0; half < 2; ++half) {
     gen_stockham(x, p);
@@ -174,14 +180,22 @@ __device__ __forceinline__ void gen_fft(const GenLines& x, const GenPlan& p) {
         const float2 z = cmul(x.get(l, k), p.bk[k]);
         x.set(l, k, make_float2(z.x, -z.y));
       }
-    } else {
+    } else if (!RAW) {
       for (int k = n0; k < L; k += dn) {
         const float2 c = x.get(l, k);
         x.set(l, k, cmul(make_float2(c.x, -c.y), p.chirp[k]));
       }
+    } else {
+      break;
     }
     __syncthreads();
   }
+}
+
+// bin k of a RAW transform
+__device__ __forceinline__ float2 gen_out(const GenLines& x, const GenPlan& p, int l, int k) {
+  const float2 c = x.get(l, k);
+  return p.chirp ? cmul(make_float2(c.x, -c.y), p.chirp[k]) : c;
 }
 
 // real and imaginary parts exchanged: before and after gen_fft, the backward
@@ -201,6 +215,31 @@ __device__ __forceinline__ void gen_each(int lnl, int n, Fn&& fn) {
   } else {
     const int l = threadIdx.x & ((1 << lnl) - 1);
     for (int i = threadIdx.x >> lnl; i < n; i += blockDim.x >> lnl) fn(l, i);
+  }
+}
+
+// This thread's share of nl lines of n elements, brought in KB at a time: ld(line,
+// element) of all of them, then st(line, element, value). One by one, as gen_each
+// goes, a load's whole latency passed before the next (one to two dozen of them:
+// the most of a block's time). ld is also called on repeats of the last element.
+template <bool ROWS, int KB, class Ld, class St>
+__device__ __forceinline__ void gen_load(int lnl, int n, Ld&& ld, St&& st) {
+  const int lm = (1 << lnl) - 1;
+  const int i0 = ROWS ? threadIdx.x : threadIdx.x >> lnl;
+  const int di = ROWS ? blockDim.x : blockDim.x >> lnl;
+  for (int q = 0; i0 + (ROWS ? q >> lnl : q) * di < n; q += KB) {
+    float2 v[KB];
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      const int l = (ROWS ? q + j : threadIdx.x) & lm;
+      v[j] = ld(l, min(i0 + (ROWS ? (q + j) >> lnl : q + j) * di, n - 1));
+    }
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      const int l = (ROWS ? q + j : threadIdx.x) & lm;
+      const int i = i0 + (ROWS ? (q + j) >> lnl : q + j) * di;
+      if (i < n) st(l, i, v[j]);
+    }
   }
 }
 
@@ -226,32 +265,41 @@ k_gen(Op op, GenPlan p, int nlines, int lnl, int pitch) {
   const GenLines x{(gen_lds_v2*)gen_lds, lnl, pitch};
   const int nact = min(1 << lnl, nlines - line0), L = p.L;
   static_assert(ROWS || !has_line<Op>::value, "per-line state is for rows");
-  if constexpr (has_line<Op>::value) {
-    for (int l = 0; l < 1 << lnl; ++l) {
-      if (l < nact) op.line(a, line0 + l);
-      for (int n = threadIdx.x; n < L; n += blockDim.x)
-        x.set(l, n, l < nact ? gen_swap<INV>(op.load(a, line0 + l, n)) : make_float2(0.f, 0.f));
+  bool any = false;
+  // lines past the last repeat it: they are transformed but not stored
+  auto load = [&](int l, int n) {
+    const int line = line0 + min(l, nact - 1);
+    float2 v;
+    if constexpr (has_line<Op>::value) {
+      Op o = op;
+      o.line(a, line);
+      v = o.load(a, line, n);
+    } else {
+      v = op.load(a, line, n);
     }
+    if constexpr (op_scans<Op>::value) any = any || v.x != 0.f || v.y != 0.f;
+    return gen_swap<INV>(v);
+  };
+  constexpr int KB = has_line<Op>::value ? 4 : 8;
+  auto set = [&](int l, int n, float2 v) { x.set(l, n, v); };
+  if (p.chirp) {  // uniform
+    gen_load<ROWS, KB>(lnl, L, [&](int l, int n) { return cmul(load(l, n), p.chirp[n]); }, set);
+    gen_each<false>(lnl, p.W - L, [&](int l, int n) { x.set(l, L + n, make_float2(0.f, 0.f)); });
   } else {
-    bool any = false;
-    gen_each<ROWS>(lnl, L, [&](int l, int n) {
-      const float2 v = l < nact ? op.load(a, line0 + l, n) : make_float2(0.f, 0.f);
-      if constexpr (op_scans<Op>::value) any = any || v.x != 0.f || v.y != 0.f;
-      x.set(l, n, gen_swap<INV>(v));
-    });
-    if constexpr (op_scans<Op>::value) {
-      if (!op.keep(a, line0, nact, __syncthreads_or(any))) return;
-    }
+    gen_load<ROWS, KB>(lnl, L, load, set);
+  }
+  if constexpr (op_scans<Op>::value) {
+    if (!op.keep(a, line0, nact, __syncthreads_or(any))) return;
   }
   __syncthreads();
-  gen_fft(x, p);
+  gen_fft<true>(x, p);
   gen_each<ROWS>(lnl, L, [&](int l, int n) {
     if (l >= nact) return;
     if constexpr (has_store2<Op>::value) {
-      op.store2(a, line0 + l, n, gen_swap<INV>(x.get(l, n)),
-                gen_swap<INV>(x.get(l, n ? L - n : 0)));
+      op.store2(a, line0 + l, n, gen_swap<INV>(gen_out(x, p, l, n)),
+                gen_swap<INV>(gen_out(x, p, l, n ? L - n : 0)));
     } else {
-      op.store(a, line0 + l, n, gen_swap<INV>(x.get(l, n)));
+      op.store(a, line0 + l, n, gen_swap<INV>(gen_out(x, p, l, n)));
     }
   });
 }

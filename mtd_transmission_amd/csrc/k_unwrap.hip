@@ -380,9 +380,8 @@ k_unw_grad_gen(const float2* __restrict__ iu, GenPlan p, int C, const float2* __
     const int i = wrap(dct_src(m, C) + h), j = wrap(line0 + l + h);
     return unit_phasor(ROWS ? iu_a[(size_t)j * C + i] : iu_a[(size_t)i * C + j]);
   };
-  gen_each<ROWS>(lnl, C, [&](int l, int m) {
-    x.set(l, m, l < nact ? phasor(l, m) : make_float2(0.f, 0.f));
-  });
+  gen_load<ROWS, 4>(lnl, C, [&](int l, int m) { return phasor(min(l, nact - 1), m); },
+                    [&](int l, int m, float2 v) { x.set(l, m, v); });
   __syncthreads();
   // forward, derivative, backward (through the exchange of parts), and for
   // the columns the packed forward transform
@@ -425,11 +424,10 @@ k_unw_poisson_gen(const float2* __restrict__ H, GenPlan p, int C, const float2* 
   const int nact = min(1 << lnl, C - line0);
   const GenLines x{(gen_lds_v2*)gen_lds, lnl, pitch};
   const size_t base = ((size_t)a * C + line0) * C;
-  gen_each<true>(lnl, C, [&](int l, int m) {
-    float2 v = make_float2(0.f, 0.f);
-    if (l < nact) v = H[base + (size_t)l * C + dct_src(m, C)];
-    x.set(l, m, make_float2(m < C / 2 ? v.x : -v.x, v.y));
-  });
+  gen_load<true, 8>(
+      lnl, C,
+      [&](int l, int m) { return H[base + (size_t)min(l, nact - 1) * C + dct_src(m, C)]; },
+      [&](int l, int m, float2 v) { x.set(l, m, make_float2(m < C / 2 ? v.x : -v.x, v.y)); });
   __syncthreads();
 #pragma unroll 1
   for (int pass = 0; pass < 2; ++pass) {
