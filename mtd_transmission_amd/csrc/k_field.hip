@@ -363,6 +363,13 @@ k_form_field(const float2* __restrict__ iu, const float2* __restrict__ crop,
 constexpr int kFwdAny = -2;     // from_iu, mode and phu say
 constexpr int kFwdFields = -1;  // fields
                                 // >= 0: IU, mode in bits 0 and 1, bit 2: phu
+// The windowed value rounded to FP32 before the transform, never contracted into
+// its first additions: a spectrum's values, and with them the OTF's zeros, do not
+// depend on what the compiler inlines.
+__device__ __forceinline__ float2 windowed(float2 f, float w) {
+#pragma clang fp contract(off)
+  return make_float2(f.x * w, f.y * w);
+}
 template <int CT, int KIND>
 struct FwdRowOp {
   const float2* src;      // fields (U frame) or IU
@@ -416,14 +423,14 @@ struct FwdRowOp {
     } else {
       f = form_from(u, 0.f, 0.0, 0.0, sn, md());
     }
-    return make_float2(f.x * w, f.y * w);
+    return windowed(f, w);
   }
   __device__ float2 load(int a, int y, int x) const {
     if (iu()) return form_iu(x, src[((size_t)a * C + y) * C + x]);
     const int X = (x + C / 2) % C;
     const float w = (float)(win[X] * wy);
     const float2 f = src[((size_t)a * C + Y) * C + X];
-    return make_float2(f.x * w, f.y * w);
+    return windowed(f, w);
   }
   __device__ void store(int a, int y, int x, float2 v) const {
     out[((size_t)a * C + y) * C + x] = v;
