@@ -940,7 +940,7 @@ static hipError_t vol_cols(Dim<VT> V, const Op& op, const FftTab& ft, const char
   }
 }
 
-// The height pass. Volumes of 512 and 1024 fold the band (k_cols_fold): planes is
+// The height pass. Volumes of 448, 512 and from 576 on fold the band (k_cols_fold): planes is
 // the band's height expected from the geometry, 0 where only the device knows
 // (then both forms are launched and the blocks of the one that does not apply
 // return). 512^3, band 151: 335 -> 278 us; 1024^3, band 302: 5.05 -> 2.43 ms.

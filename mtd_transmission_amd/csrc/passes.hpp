@@ -306,9 +306,14 @@ inline dim3 cols_b_block() {
 // volumes column by column and reading a band of 0.295 V planes, with no
 // transform, takes at V = 1024 4.8, 2.85 and 2.23 ms with 16, 32 and 64 columns
 // a block (64-, 128- and 256-byte pieces), at V = 512 459, 254 and 241 us.
+// The lengths it is built for: those whose L/R has a square split (all threads in
+// both steps) and whose whole transform left 9 to 16 columns a block, and 448 and
+// 512. Height pass alone at 4.7 to 8 bins per pupil radius (96 bins): 448^3 242 ->
+// 202 us, 576^3 1077 -> 473, 640^3 1136 -> 607, 704^3 1567 -> 840, 768^3 2140 -> 969.
 template <int L>
 constexpr int cols_fold_r() {
-  return L / 256;
+  return L == 512 ? 2 : L == 576 ? 4 : L == 640 ? 10 : L == 704 ? 11 : L == 768 ? 3
+         : L == 1024 ? 4 : L == 448 ? 7 : 1;
 }
 template <int L>
 constexpr int cols_fold_nc() {
@@ -328,7 +333,7 @@ struct op_cols_fold<Op, std::void_t<decltype(Op::kFoldCols)>>
     : std::integral_constant<bool, Op::kFoldCols> {};
 template <int L>
 constexpr bool cols_fold_fits() {
-  return L == 512 || L == 1024;
+  return cols_fold_r<L>() > 1;
 }
 // band elements [lo, hi] in the register path
 template <int L>

@@ -112,14 +112,16 @@ def test_finalize_sparse(gpu_ctx, V, kind):
 
 
 def _fold_bands(V):
-    nb = {512: 192, 1024: 368}[V]  # planes a block holds in registers, in sixteens
+    # planes a block holds in registers
+    nb = {448: 168, 512: 192, 576: 216, 640: 232, 704: 256, 768: 288, 1024: 368}[V]
     return [(0, 1), (V - 1, V - 1), (0, nb - 1), (V - nb, V - 1), (7, nb - 1), (7, nb), (16, 16 + nb),
             (V // 2 - nb // 2, V // 2 + nb // 2), (0, V - 1)]
 
 
-@pytest.mark.parametrize("V,lo,hi", [(V, *b) for V in (512, 1024) for b in _fold_bands(V)])
+@pytest.mark.parametrize("V,lo,hi", [(V, *b) for V in (448, 512, 576, 640, 704, 768, 1024)
+                                     for b in _fold_bands(V)])
 def test_finalize_folded_height_pass(gpu_ctx, V, lo, hi):
-    """The height pass folds a band of planes onto 256: bands at the edges of the
+    """The height pass folds a band of planes onto a short transform: bands at the edges of the
     volume and of what a block holds in registers, against the closed form of a
     few normalised deltas at 100000 voxels. Bound: 30 roundings of 2^-24 over
     the three passes' 29 radix-2 levels at 1024, rounded to 2e-6."""
