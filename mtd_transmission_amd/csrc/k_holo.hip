@@ -464,30 +464,27 @@ static hipError_t cols_n(const float2* t1, int A, const float2* tw, int C,
 }
 
 // ---------------------------------------------------------------------------
-// Hologram sides without a compiled FFT: two real rows of the windowed,
-// sign-modulated hologram per complex transform, as k_holo_rows packs them
-// (their kept bins into t1[a][y][d], untiled, without the 1/2 of the
-// separation), then one transform per kept column (its C kept bins, / (2 N^2)
-// and signed). The specular is then found from the crops (no argmax partials).
+// Hologram sides without a compiled FFT: one complex transform per row of
+// the windowed, sign-modulated hologram (its C kept bins into t1[a][y][d],
+// untiled), then one per kept column (its C kept bins, / N^2 and signed).
+// The specular is then found from the crops (no argmax partials).
+// One row per transform: two (their bins as sums and differences) would halve
+// the row pass, but round each row's faint bins by the other row's size
+// (gen_fft.hpp says what came of it).
 // ---------------------------------------------------------------------------
 template <typename TIn>
-struct HoloRowGenOp {  // line: rows 2 line and 2 line + 1
+struct HoloRowGenOp {
   const TIn* holos;
   const float* ws;  // (float)tukey1d(N)[i] * (-1)^i
   float2* t1;
   int N, C, x0;
   __device__ void begin(int) {}
-  __device__ float2 load(int a, int line, int x) const {
-    const TIn* h = holos + ((size_t)a * N + 2 * line) * N + x;
-    const float w = ws[x];
-    return make_float2((float)h[0] * (w * ws[2 * line]), (float)h[N] * (w * ws[2 * line + 1]));
+  __device__ float2 load(int a, int y, int x) const {
+    return make_float2((float)holos[((size_t)a * N + y) * N + x] * (ws[x] * ws[y]), 0.f);
   }
-  __device__ void store2(int a, int line, int k, float2 zk, float2 zm) const {
+  __device__ void store(int a, int y, int k, float2 v) const {
     const int d = k - x0;
-    if (d < 0 || d >= C) return;
-    float2* q = t1 + ((size_t)a * N + 2 * line) * C + d;
-    q[0] = make_float2(zk.x + zm.x, zk.y - zm.y);
-    q[C] = make_float2(zk.y + zm.y, zm.x - zk.x);
+    if (d >= 0 && d < C) t1[((size_t)a * N + y) * C + d] = v;
   }
 };
 
@@ -512,13 +509,13 @@ static hipError_t rows_gen(int N, int dtype, const void* holos, int A, const flo
   switch (dtype) {
     case MTD_U8:
       return launch_gen<false, true>(HoloRowGenOp<uint8_t>{(const uint8_t*)holos, win, t1, N, C, x0},
-                                     p, N / 2, A, s);
+                                     p, N, A, s);
     case MTD_U16:
       return launch_gen<false, true>(
-          HoloRowGenOp<uint16_t>{(const uint16_t*)holos, win, t1, N, C, x0}, p, N / 2, A, s);
+          HoloRowGenOp<uint16_t>{(const uint16_t*)holos, win, t1, N, C, x0}, p, N, A, s);
     default:
       return launch_gen<false, true>(HoloRowGenOp<float>{(const float*)holos, win, t1, N, C, x0},
-                                     p, N / 2, A, s);
+                                     p, N, A, s);
   }
 }
 
@@ -568,7 +565,7 @@ hipError_t launch_holo_cols(int N, const float2* t1, int A, const FftTab& ft,
   if (qtw) return hipErrorInvalidValue;  // the fused column IDFT is for compiled sides
   if (!ft.gen) return hipErrorInvalidValue;
   Timed tm("holo_cols", s);
-  const float scale = (float)(0.5 / ((double)N * (double)N));
+  const float scale = (float)(1.0 / ((double)N * (double)N));
   return launch_gen<false, false>(HoloColGenOp{t1, crop, N, C, x0, y0, scale}, *ft.gen, C, A, s);
 }
 

@@ -43,7 +43,7 @@
 // (half-empty transforms, both gradients with their trigonometry on every
 // pixel three times) moved about 300. Measured, all unwrapping kernels, that
 // form against this one: 300 crops of 250^2 3217 -> 536 us, 400 of 128^2 813 ->
-// 144 us, 48 of 182^2 (runtime-length FFTs) 986 -> 182 us.
+// 144 us, 48 of 182^2 (runtime-length FFTs) 986 -> 118 us.
 #include <cfloat>
 
 #include "dft.hpp"
@@ -387,15 +387,15 @@ k_unw_grad_gen(const float2* __restrict__ iu, GenPlan p, int C, const float2* __
   // the columns the packed forward transform
 #pragma unroll 1
   for (int pass = 0; pass < (ROWS ? 2 : 3); ++pass) {
-    gen_fft(x, p);
+    gen_fft<false, false>(x, p);
     if (pass == 0) {
       gen_pairs(x, C, [&](int, int k, float2 V, float2 Vr) {
-        return gen_swap<true>(deriv_bin(V, Vr, k, C, tw4));
+        return gen_swap(deriv_bin(V, Vr, k, C, tw4));
       });
     } else if (pass == 1) {
       gen_each<ROWS>(lnl, C, [&](int l, int m) {
         if (l >= nact) return;
-        const float2 w = gen_swap<true>(x.get(l, m)), z = phasor(l, m);
+        const float2 w = gen_swap(x.get(l, m)), z = phasor(l, m);
         const float g = w.y * z.x - w.x * z.y;
         const int n = dct_src(m, C);
         if (ROWS) gx[base + (size_t)(line0 + l) * C + n] = m < h ? g : -g;
@@ -431,16 +431,16 @@ k_unw_poisson_gen(const float2* __restrict__ H, GenPlan p, int C, const float2* 
   __syncthreads();
 #pragma unroll 1
   for (int pass = 0; pass < 2; ++pass) {
-    gen_fft(x, p);
+    gen_fft<false, false>(x, p);
     if (pass == 0) {
       gen_pairs(x, C, [&](int l, int k, float2 V, float2 Vr) {
         const float2 e = tw4[k];
-        return gen_swap<true>(poisson_bin(dct_p(V, e), dct_q(Vr, e), e, k, line0 + l, C));
+        return gen_swap(poisson_bin(dct_p(V, e), dct_q(Vr, e), e, k, line0 + l, C));
       });
     }
   }
   gen_each<true>(lnl, C, [&](int l, int m) {
-    if (l < nact) out[base + (size_t)l * C + dct_src(m, C)] = gen_swap<true>(x.get(l, m)).x;
+    if (l < nact) out[base + (size_t)l * C + dct_src(m, C)] = gen_swap(x.get(l, m)).x;
   });
 }
 

@@ -142,92 +142,51 @@ static const int* tile_order(mtd_ctx* ctx, int V) {
 // ---------------------------------------------------------------------------
 // runtime-length FFT plans (gen_fft.hpp)
 // ---------------------------------------------------------------------------
-// L as a product of as few radices as possible (gen_radix_ok), the smallest of
-// them as large as possible (a pass over a line has L / R butterflies); false
-// where a prime above 13 divides L
+// radices of L from {8, 4, 2, 3, 5, 7, 11, 13}, in this order; false if another
+// prime divides L
 static bool gen_factor(int L, std::vector<int>& f) {
+  f.clear();
   int n = L;
-  for (int p : {2, 3, 5, 7, 11, 13})
-    while (n % p == 0) n /= p;
-  if (L < 2 || n != 1) return false;
-  // a product of k radices in descending order, the last at most the one before
-  std::vector<int> cur, best;
-  for (int k = 1; k <= kGenMaxPasses && best.empty(); ++k) {
-    auto rec = [&](auto&& self, int rest, int left, int most) -> void {
-      if (left == 1) {
-        if (rest > most || !gen_radix_ok(rest)) return;
-        if (best.empty() || rest > best.back()) {
-          best = cur;
-          best.push_back(rest);
-        }
-        return;
-      }
-      for (int r = std::min(most, rest); r >= 2; --r)
-        if (rest % r == 0 && gen_radix_ok(r)) {
-          cur.push_back(r);
-          self(self, rest / r, left - 1, r);
-          cur.pop_back();
-        }
-    };
-    rec(rec, L, k, kGenMaxRadix);
-  }
-  f = best;
-  return !f.empty();
+  while (n % 8 == 0) { f.push_back(8); n /= 8; }
+  while (n % 4 == 0) { f.push_back(4); n /= 4; }
+  while (n % 2 == 0) { f.push_back(2); n /= 2; }
+  for (int r : {3, 5, 7, 11, 13})
+    while (n % r == 0) { f.push_back(r); n /= r; }
+  return L >= 2 && n == 1 && (int)f.size() <= kGenMaxPasses;
 }
 
-static int next_pow2(int n) {
+static int bluestein_len(int L) {
   int W = 1;
-  while (W < n) W *= 2;
+  while (W < 2 * L - 1) W *= 2;
   return W;
 }
 
 bool gen_len_ok(int L) {
   if (L < 2) return false;
   std::vector<int> f;
-  return (gen_factor(L, f) ? L : next_pow2(2 * L - 1)) <= kGenMaxLen;
+  return (gen_factor(L, f) ? L : bluestein_len(L)) <= kGenMaxLen;
 }
 
-// Bluestein's working length: of the products of radices from 2L - 1 to the
-// next power of two, the one with the fewest points times passes over LDS (the
-// load and store of the line counted as one more pass)
-static int bluestein_len(int L, std::vector<int>& f) {
-  int best = 0;
-  for (int W = 2 * L - 1; W <= next_pow2(2 * L - 1); ++W) {
-    std::vector<int> c;
-    if (gen_factor(W, c) && W / c.back() <= kGenThreads &&
-        (!best || W * ((int)c.size() + 1) < best * ((int)f.size() + 1))) {
-      best = W;
-      f = c;
-    }
+// in-place radix-2 FFT (forward, unnormalised) of a power-of-two length, in
+// long double: the host side of the Bluestein tables
+static void fft_pow2_host(std::vector<std::complex<long double>>& a) {
+  const size_t n = a.size();
+  for (size_t i = 1, j = 0; i < n; ++i) {
+    size_t bit = n >> 1;
+    for (; j & bit; bit >>= 1) j ^= bit;
+    j ^= bit;
+    if (i < j) std::swap(a[i], a[j]);
   }
-  return best;
-}
-
-// forward DFT (unnormalised) in long double by the same factors: the host side
-// of the Bluestein tables
-static void dft_host(std::vector<std::complex<long double>>& a, const std::vector<int>& f) {
-  const int n = (int)a.size();
   const long double pi = 3.14159265358979323846264338327950288L;
-  std::vector<std::complex<long double>> w(n), b(n);
-  for (int k = 0; k < n; ++k) {
-    const long double ang = -2 * pi * (long double)k / (long double)n;
-    w[k] = {std::cos(ang), std::sin(ang)};
-  }
-  // Stockham passes, as on the device
-  int Ns = 1;
-  for (int R : f) {
-    const int nb = n / R, step = n / (Ns * R);
-    for (int j = 0; j < nb; ++j) {
-      const int k = j % Ns, d = (j / Ns) * Ns * R + k;
-      for (int s = 0; s < R; ++s) {
-        std::complex<long double> sum = 0;
-        for (int r = 0; r < R; ++r)
-          sum += a[j + r * nb] * w[(long)r * (k * step + s * nb) % n];
-        b[d + s * Ns] = sum;
+  for (size_t len = 2; len <= n; len <<= 1) {
+    for (size_t i = 0; i < n; i += len)
+      for (size_t k = 0; k < len / 2; ++k) {
+        const long double ang = -2 * pi * (long double)k / (long double)len;
+        const std::complex<long double> w(std::cos(ang), std::sin(ang));
+        const std::complex<long double> u = a[i + k], v = a[i + k + len / 2] * w;
+        a[i + k] = u + v;
+        a[i + k + len / 2] = u - v;
       }
-    }
-    a.swap(b);
-    Ns *= R;
   }
 }
 
@@ -239,15 +198,14 @@ static const GenPlan* gen_plan(mtd_ctx* ctx, int L) {
   p.L = L;
   std::vector<int> f;
   const bool direct = gen_factor(L, f);
-  p.W = direct ? L : bluestein_len(L, f);
+  p.W = direct ? L : bluestein_len(L);
+  if (!direct) gen_factor(p.W, f);
   p.nf = (int)f.size();
   for (int i = 0; i < p.nf; ++i) {
     p.f[i] = f[i];
-    p.bfly = std::max(p.bfly, p.W / f[i]);
+    const int held = f[i] * gen_per_thread(f[i]);
+    p.threads = std::max(p.threads, (p.W + held - 1) / held);
   }
-  // a thread holds one butterfly: beyond the even lengths that transforms have
-  // here (3993 = 3 11^3 would need 1331 threads)
-  if (p.bfly > kGenThreads) return nullptr;
   p.tw = twiddle(ctx, p.W);
   if (!p.tw) return nullptr;
   if (!direct) {
@@ -264,7 +222,7 @@ static const GenPlan* gen_plan(mtd_ctx* ctx, int L) {
       b[n] = std::conj(w);
       if (n > 0) b[p.W - n] = std::conj(w);
     }
-    dft_host(b, f);
+    fft_pow2_host(b);
     std::vector<float2> bk(p.W);
     for (int k = 0; k < p.W; ++k)
       bk[k] = make_float2((float)(b[k].real() / p.W), (float)(b[k].imag() / p.W));
