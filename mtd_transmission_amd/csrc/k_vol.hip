@@ -1002,11 +1002,11 @@ static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt,
 // per voxel; x, y and z in that order with the band cut last took 39. Measured
 // at 416^3, 200 angles: 606 -> 246 us, at 256^3 (400 angles) 116 -> 71 us.
 // ---------------------------------------------------------------------------
-template <int VT, bool CPLX>
+template <int VT>
 struct ContrastZOp {  // lines along z of the contrast volume; a = y, col = x, row = z
   static constexpr bool kBalancedCols = true;
   const float* re;
-  const float* im;  // CPLX
+  const float* im;  // nullptr: real contrast
   float2* out;
   const float2* tw;
   const int2* band;
@@ -1018,18 +1018,9 @@ struct ContrastZOp {  // lines along z of the contrast volume; a = y, col = x, r
   }
   __device__ float2 load(int y, int x, int z) const {
     const size_t i = ((size_t)z * V + y) * V + x;
-    float2 t = make_float2(re[i], CPLX ? im[i] : 0.f);
+    float2 t = make_float2(re[i], im ? im[i] : 0.f);
     if ((x + y + z) & 1) { t.x = -t.x; t.y = -t.y; }
     return t;
-  }
-  // the same for column x0 + c, with y, x0 and z uniform over the wave and
-  // c < 64 its lane: scalar addresses, zeros past the row
-  __device__ __forceinline__ float2 load_wave(int y, int x0, int c, int z) const {
-    const size_t i = ((size_t)z * V + y) * V + x0;
-    const unsigned n = min(64, V - x0) * 4;
-    const float2 t = make_float2(BufView(re + i, n).f1(c * 4, 0),
-                                 CPLX ? BufView(im + i, n).f1(c * 4, 0) : 0.f);
-    return (x0 + c + y + z) & 1 ? make_float2(-t.x, -t.y) : t;
   }
   __device__ void store(int y, int x, int z, float2 v) const {
     if (z < lo || z > hi) return;
@@ -1054,29 +1045,15 @@ struct SpectrumXOp {  // rows along x of the band's planes, in place; a = z, lin
   Dim<VT> V{};
 };
 
-template <int VT, bool CPLX>
-static hipError_t contrast_z(Dim<VT> V, const ContrastZOp<VT, CPLX>& z, const FftTab& ft,
-                             hipStream_t s) {
-  if constexpr (VT > 0 && cols_band_fits<VT>()) {
-    Timed tm("fwd_vol_z", s);
-    hipLaunchKernelGGL((k_cols_band<VT, false, ContrastZOp<VT, CPLX>>), cols_band_grid<VT>(VT),
-                       dim3(cols_band_threads<VT>()), 0, s, z);
-    return hipGetLastError();
-  } else {
-    return vol_cols<VT, false, false>(V, z, ft, "fwd_vol_z", 0, s);
-  }
-}
-
 template <int VT>
 static hipError_t contrast_spectrum_v(Dim<VT> V, const float* re, const float* im, float2* work,
                                       float scale, const int2* band, const FftTab& ft,
                                       hipStream_t s) {
+  ContrastZOp<VT> z{re, im, work, ft.tw, band, 0, V - 1, V};
   PlaneYOp<VT, false> y{work, ft.tw, band, nullptr, V};
   SpectrumXOp<VT> x{work, ft.tw, scale, band, V};
   hipError_t e;
-  e = im ? contrast_z(V, ContrastZOp<VT, true>{re, im, work, ft.tw, band, 0, V - 1, V}, ft, s)
-         : contrast_z(V, ContrastZOp<VT, false>{re, im, work, ft.tw, band, 0, V - 1, V}, ft, s);
-  if (e != hipSuccess) return e;
+  if ((e = vol_cols<VT, false, false>(V, z, ft, "fwd_vol_z", 0, s)) != hipSuccess) return e;
   if ((e = vol_cols<VT, false, false>(V, y, ft, "fwd_vol_y", 0, s)) != hipSuccess) return e;
   return vol_rows<VT, false, false>(V, x, ft, "fwd_vol_x", 0, s);
 }

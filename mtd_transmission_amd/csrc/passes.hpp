@@ -43,10 +43,6 @@ struct BufView {
     return __builtin_bit_cast(float2,
                               __builtin_amdgcn_raw_buffer_load_b64(r, lane_bytes, uni_bytes, 0));
   }
-  __device__ __forceinline__ float f1(unsigned lane_bytes, unsigned uni_bytes) const {
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_raw_buffer_load_b32(r, lane_bytes, uni_bytes, 0));
-  }
 };
 
 // Row passes: NT transforms per block (at most 256 threads, 64 KiB LDS).
@@ -429,105 +425,6 @@ __global__ void __launch_bounds__(cols_fold_threads<L>(), 4) k_cols_fold(Op op) 
 #pragma unroll
     for (int k2 = 0; k2 < L2; ++k2) op.store_wave(a, c0, c, R * (n2 + L1 * k2) + r, u[k2]);
   }
-}
-
-// The other direction: the column transform of which only a band of outputs
-// [op.lo, op.hi] is kept. Decimation in time: X[k] is the sum over r < R of
-// W_L^(r k) F_r[k mod M], F_r the (L/R = M)-point transform of the elements z = R n +
-// r. A block runs the R short transforms one after the other on 64 columns (256-byte
-// pieces of float planes) and adds each up in the band's outputs, NB registers a
-// thread. A band of more goes in rounds of NB * T outputs, each reading the input
-// again. Scalar loads for all twiddles, as in k_cols_fold. The forward model's height
-// pass: 256^3 30.5 -> 24.4 us, 416^3 163 -> 137 (its whole transform is a 13-wave block,
-// one per CU); 512^3 205 -> 209, which keeps the whole transform.
-template <int L>
-constexpr int cols_band_r() {
-  return L == 256 ? 4 : L == 416 ? 2 : 1;
-}
-template <int L>
-constexpr bool cols_band_fits() {
-  return cols_band_r<L>() > 1;
-}
-template <int L>
-constexpr int cols_band_nb() {
-  constexpr int T = Fft2<L / cols_band_r<L>(), false>::L1;
-  return (36 * L / 100 + T - 1) / T;
-}
-template <int L>
-constexpr int cols_band_threads() {
-  return 64 * Fft2<L / cols_band_r<L>(), false>::T;
-}
-template <int L, bool INV, class Op>
-__global__ void __launch_bounds__(cols_band_threads<L>(), 4) k_cols_band(Op op) {
-  constexpr int R = cols_band_r<L>(), M = L / R, NC = 64, NB = cols_band_nb<L>();
-  using F = Fft2<M, INV>;
-  constexpr int L1 = F::L1, L2 = F::L2;
-  __shared__ float lds[NC * F::LDS_COL];
-  const int2 ab = xcd_block();
-  const int a = ab.x, c0 = ab.y * NC;
-  const int c = threadIdx.x % NC;
-  const int n2 = __builtin_amdgcn_readfirstlane(threadIdx.x / NC);  // uniform over the wave
-  op.begin(a);
-  typedef float v2f __attribute__((ext_vector_type(2)));
-  const auto* tw = (const __attribute__((address_space(4))) v2f*)op.tw;
-  const typename F::template Col<NC> x{lds + c};
-  // Thread n2 < L1 holds X[n2 + L1 k2] of a short transform, so the band's outputs
-  // k = L1 (b + j) + n2: k mod M is n2 + L1 ((b + j) mod L2). The rotation by b of the
-  // second step's outputs is a phase on its inputs, W_L2^(b n).
-  const int b0 = op.lo > 0 ? op.lo / L1 : 0;
-  for (int b = b0; L1 * b <= op.hi; b += NB) {  // uniform; one round for most bands
-    float2 e[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) e[j] = make_float2(0.f, 0.f);
-#pragma unroll 1
-    for (int r = 0; r < R; ++r) {
-      float2 v[L1], u[L2];
-#pragma unroll
-      for (int n1 = 0; n1 < L1; ++n1) v[n1] = op.load_wave(a, c0, c, R * (L2 * n1 + n2) + r);
-      if constexpr (L1 > 1) RegFFT<L1, INV>::run(v);
-      // step twiddle W_M^(n2 k1) and the rotation's W_L2^(b n2): R (n2 k1 + L1 b n2)
-#pragma unroll
-      for (int k1 = 0; k1 < L1; ++k1) {
-        const v2f q = tw[R * (n2 * (k1 + L1 * b) % M)];
-        v[k1] = cmul(v[k1], make_float2(q.x, INV ? -q.y : q.y));
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k1 = 0; k1 < L1; ++k1) *x.at(k1, n2) = v[k1].x;
-      __syncthreads();
-      if (n2 < L1) {
-#pragma unroll
-        for (int n = 0; n < L2; ++n) u[n].x = *x.at(n2, n);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k1 = 0; k1 < L1; ++k1) *x.at(k1, n2) = v[k1].y;
-      __syncthreads();
-      if (n2 < L1) {
-#pragma unroll
-        for (int n = 0; n < L2; ++n) u[n].y = *x.at(n2, n);
-        RegFFT<L2, INV>::run(u);
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          const v2f q = tw[r * (L1 * (b + j) + n2) % L];
-          const float2 t = cmul(u[j % L2], make_float2(q.x, INV ? -q.y : q.y));
-          e[j] = make_float2(e[j].x + t.x, e[j].y + t.y);
-        }
-      }
-    }
-    if (n2 < L1) {
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        const int k = L1 * (b + j) + n2;
-        if (k >= op.lo && k <= op.hi && (L % NC == 0 || c0 + c < L)) op.store(a, c0 + c, k, e[j]);
-      }
-    }
-  }
-}
-// the last block may reach past L: load_wave gives zeros there
-template <int L>
-inline dim3 cols_band_grid(int A) {
-  return dim3((L + 63) / 64, A);
 }
 
 // An operation may define mid_line(batch, line), called once per transform
