@@ -331,11 +331,10 @@ hipError_t launch_gather_prepass(const AngleGeo* ageo, int A, int C, int nxmax, 
 void gather_tile_order_host(int V, int* order);
 size_t gather_scratch_bytes(int V, int A);
 // Born forward model: work = centred 3-D spectrum of the contrast (re, im;
-// im may be nullptr) times scale (Tp^3 * gsign), stored only on the heights
-// of the device band.
+// im may be nullptr), unnormalised and but for the sign (-1)^(3V/2), stored only
+// on the heights of the device band.
 hipError_t launch_contrast_spectrum(int V, const float* re, const float* im, float2* work,
-                                   float scale, const int2* band, const FftTab& ft,
-                                   hipStream_t s);
+                                   const int2* band, const FftTab& ft, hipStream_t s);
 // One fused FISTA step with the smoothed TV gradient (k_tv.hip).
 hipError_t launch_stamp(unsigned long long* out, hipStream_t s);
 hipError_t launch_tv_start(float* x, float* z, size_t n, int positivity, hipStream_t s);
@@ -346,11 +345,12 @@ hipError_t launch_tv_fista(int V, const float* z, const float* gd, float* x, flo
 hipError_t launch_cap_weights(const int32_t* cnt, const AngleGeo* ageo, int A,
                               const double* htab, const float* q, int r2max, int nx, int C,
                               int V, float* w, hipStream_t s);
-// Per-angle cap samples -i q(|fd|^2) vol[voxel] into spec[A][C][C] (+posSpec frame);
-// y: the weighted residual q w (samples - y) instead (w NULL: 1).
+// Per-angle cap samples -i fac / h(|fd|^2) vol[voxel] into spec[A][C][C] (+posSpec
+// frame); y: the weighted residual q w (samples - y) instead (w NULL: 1; q2: the
+// factors q in the pupil frame).
 hipError_t launch_cap_sample(const float2* vol, const AngleGeo* ageo, int A, const double* htab,
-                             const float* q2, int r2max, int nx, int C, int V, const float2* y,
-                             const float* w, float2* spec, hipStream_t s);
+                             double fac, const float* q2, int r2max, int nx, int C, int V,
+                             const float2* y, const float* w, float2* spec, hipStream_t s);
 // band: heights outside it are zero and are not read; vol is then already divided
 // by its counts and centring-signed (gather flag 1). occ != nullptr (V^2 bytes,
 // rounded up to 16): the band is not known and is found by the first pass into

@@ -392,6 +392,7 @@ struct EwaldTables {
   const float* beta2;  // C x C, pupil frame: beta at fd = (c - NXMAX, r - NXMAX), 0 outside
   const float* q;      // Born forward weights per r2 <= r2max (born_weights)
   const float* q2;     // the same in the C x C pupil frame, 0 outside the pupil
+  double qR;           // q(r2) = qR / h(r2) before rounding
   int r2tab;
   int r2max;
   double R2;
@@ -469,6 +470,8 @@ static int ewald_tables(mtd_ctx* ctx, const mtd_geom* g, EwaldTables* t) {
   t->beta = d_b;
   t->beta2 = d_b2;
   t->q = nullptr;
+  t->q2 = nullptr;
+  t->qR = 0;
   t->r2tab = r2tab;
   t->r2max = r2max;
   t->R2 = R2;
@@ -1233,6 +1236,7 @@ static int born_weights(mtd_ctx* ctx, const mtd_geom* g, EwaldTables* t) {
   // |(-1/(2 PI)) * (-i PI/k0) * (-2 kv^2 n0)|
   const double c = (1.0 / (2 * PI)) * (PI / k0) * (2 * kv * kv * g->n0);
   const double R = g->rayon;
+  t->qR = c * R;
   const auto key = std::make_tuple(bits_of(R), t->r2max, bits_of(g->lambda), bits_of(g->n0));
   const int nx = g->nxmax, C = 2 * nx;
   const auto key2 = std::make_tuple(bits_of(R), t->r2max, bits_of(g->lambda), bits_of(g->n0), nx);
@@ -1498,13 +1502,13 @@ static int forward_impl(mtd_ctx* ctx, const mtd_geom* g, const float* dn_re, con
   const bool tabs = fft_tab(ctx, V, vol_len_supported(V), &twV);
   if (!work || !tabs) return set_err(ctx, MTD_ERR_HIP, "out of device memory");
   const double tp = tomo_pixel(g);
-  const float gsign = ((V / 2) & 1) ? -1.f : 1.f;
-  MTD_TRY(hip_check(ctx, launch_contrast_spectrum(V, dn_re, dn_im, work,
-                                                  (float)(tp * tp * tp) * gsign, geo.band, twV,
+  const double gsign = ((V / 2) & 1) ? -1 : 1;
+  MTD_TRY(hip_check(ctx, launch_contrast_spectrum(V, dn_re, dn_im, work, geo.band, twV,
                                                   ctx->stream),
                     "contrast spectrum"));
-  return hip_check(ctx, launch_cap_sample(work, geo.ag, A, t.htab, t.q2, t.r2max, g->nxmax, C, V,
-                                          (const float2*)y, w, (float2*)spectra, ctx->stream),
+  return hip_check(ctx, launch_cap_sample(work, geo.ag, A, t.htab, t.qR * tp * tp * tp * gsign, t.q2,
+                                          t.r2max, g->nxmax, C, V, (const float2*)y, w,
+                                          (float2*)spectra, ctx->stream),
                    "cap sampling");
 }
 
