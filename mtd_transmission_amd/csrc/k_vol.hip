@@ -712,7 +712,11 @@ __device__ __forceinline__ bool outside_band(const int2* band, int z) {
 // k_band_found takes the band of planes that did from it. The y pass reads no
 // empty row and skips the planes outside, the height pass reads the band alone.
 // On a spectrum of 400 angles at 512^3, band about a third, with the OTF: x 733 ->
-// 393, y 450 -> 114, z 532 -> 280 us; on a dense spectrum all three 1.61 -> 1.69 ms.
+// 393, y 450 -> 114, z 532 -> 280 us. Waves that found something read their counts
+// ahead of the block's answer: with the counts after it, a dense spectrum took
+// longer than without the look (1024^3, all three passes: 15.5 ms without, 16.7 with
+// counts after, 14.8 now; 512^3 1570, 1403 and 1401 us; 512^3 with a third of the
+// planes occupied 1567, 752 and 750). Sides up to kScanOver go without.
 // (With every voxel's count read and divided by before the scan, the OTF stored a
 // byte at a time and two atomics on one word for the band: x 557 us.)
 constexpr int kBandThreads = 1024;
@@ -757,19 +761,20 @@ k_band_found(const uint4* __restrict__ occ, int V, int2* __restrict__ band) {
   *band = hi < 0 ? make_int2(V, -1) : make_int2(lo / V, hi / V);
 }
 
-template <int VT, bool SCAN>
+// What the x pass transforms: the gather's normalised volume, already times
+// (-1)^(x+y+z); a spectrum and its counts; these without a look for their band.
+enum NormKind { kNormDone, kNormScan, kNormAll };
+template <int VT, NormKind KIND>
 struct NormXOp {  // rows along x; a = z, line = y
-  // SCAN: a spectrum and its counts, band not known; otherwise the gather's
-  // normalised volume, already times (-1)^(x+y+z)
-  static constexpr bool kScans = SCAN;
+  static constexpr bool kScans = KIND == kNormScan;
   const float2* vol;
   const int32_t* cnt;
   float2* out;
   uint8_t* otf;
   const float2* tw;
-  const int2* band;
-  uint8_t* occ;  // SCAN
-  __device__ bool skip(int z) const { return !SCAN && outside_band(band, z); }
+  const int2* band;  // kNormDone
+  uint8_t* occ;      // kNormScan
+  __device__ bool skip(int z) const { return KIND == kNormDone && outside_band(band, z); }
   __device__ void begin(int) {}
   // The OTF (nonzero real parts) goes through LDS to whole words, and only the
   // rows that hold something read their counts and divide.
@@ -788,16 +793,16 @@ struct NormXOp {  // rows along x; a = z, line = y
     return any;
   }
   __device__ float2 raw(int z, int y, int x) const { return vol[((size_t)z * V + y) * V + x]; }
-  __device__ float2 value(float2 v, int z, int y, int x) const {
-    if constexpr (!SCAN) return v;
-    const int c0 = cnt[((size_t)z * V + y) * V + x];
+  __device__ int part(int z, int y, int x) const { return cnt[((size_t)z * V + y) * V + x]; }
+  __device__ float2 value(float2 v, int c0, int z, int y, int x) const {
     const float c = (float)(c0 == 0 ? 1 : c0);
     const float2 t = make_float2(v.x / c, v.y / c);
     return (x + y + z) & 1 ? make_float2(-t.x, -t.y) : t;
   }
   __device__ float2 load(int z, int y, int x) const {
-    const float2 t = value(raw(z, y, x), z, y, x);
-    if (SCAN && otf) otf[((size_t)z * V + y) * V + x] = (t.x != 0.f) ? 1 : 0;
+    if constexpr (KIND == kNormDone) return raw(z, y, x);
+    const float2 t = value(raw(z, y, x), part(z, y, x), z, y, x);
+    if (otf) otf[((size_t)z * V + y) * V + x] = (t.x != 0.f) ? 1 : 0;
     return t;
   }
   __device__ void store(int z, int y, int x, float2 v) const {
@@ -972,7 +977,7 @@ static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt,
   ZOutOp<VT> z{work, re, im, ft.tw, df3, cte, gsign, band, 0, 0, V - 1, V};
   hipError_t e;
   if (occ) {
-    NormXOp<VT, true> x{vol, cnt, work, otf, ft.tw, nullptr, occ, V};
+    NormXOp<VT, kNormScan> x{vol, cnt, work, otf, ft.tw, nullptr, occ, V};
     if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
     Timed tm("vol_band", s);
     hipLaunchKernelGGL(k_band_found, dim3(1), dim3(kBandThreads), 0, s, (const uint4*)occ, (int)V,
@@ -981,8 +986,14 @@ static hipError_t finalize_v(Dim<VT> V, const float2* vol, const int32_t* cnt,
     PlaneYOp<VT, true> y{work, ft.tw, band, occ, V};
     if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
   } else {
-    NormXOp<VT, false> x{vol, cnt, work, otf, ft.tw, band, nullptr, V};
-    if ((e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s)) != hipSuccess) return e;
+    if (band) {
+      NormXOp<VT, kNormDone> x{vol, cnt, work, otf, ft.tw, band, nullptr, V};
+      e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s);
+    } else {
+      NormXOp<VT, kNormAll> x{vol, cnt, work, otf, ft.tw, nullptr, nullptr, V};
+      e = vol_rows<VT, true, true>(V, x, ft, "vol_x", tiles.x, s);
+    }
+    if (e != hipSuccess) return e;
     PlaneYOp<VT, false> y{work, ft.tw, band, nullptr, V};
     if ((e = vol_cols<VT, true, true>(V, y, ft, "vol_y", tiles.y, s)) != hipSuccess) return e;
   }

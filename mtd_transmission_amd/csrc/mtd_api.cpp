@@ -1393,7 +1393,7 @@ static int finalize_impl(mtd_ctx* ctx, const mtd_geom* g, const float* vol,
   FftTab twV;
   const bool tabs = fft_tab(ctx, V, vol_len_supported(V), &twV);
   uint8_t* occ = nullptr;
-  if (!band) {
+  if (!band && V > kScanOver) {
     band = (int2*)ws_get(ctx, WS_BAND, sizeof(int2));
     occ = (uint8_t*)ws_get(ctx, WS_OCC, ((size_t)V * V + 15) / 16 * 16);
     if (!band || !occ) return set_err(ctx, MTD_ERR_HIP, "out of device memory (volume band)");

@@ -160,8 +160,9 @@ struct has_line<Op, std::void_t<decltype(std::declval<Op&>().line(0, 0))>> : std
 // loads, with whether any value of the block's lines is not zero (NaN is not
 // zero): the block then leaves its lines alone when it returns false. The
 // compiled row pass scans what raw(batch, line, element) reads, and makes the
-// transform's input of it with value(raw, batch, line, element) only if the block
-// goes on; where flags() holds, store_flags(batch, first line, lines, bytes) gets
+// transform's input of it with value(raw, part, batch, line, element) only if the
+// block goes on. part(batch, line, element) is the input's other part, read by the
+// waves that found something (1 for the others); where flags() holds, store_flags(batch, first line, lines, bytes) gets
 // a byte per element, 1 where the input's real part is not zero (nullptr:
 // nowhere).
 template <class Op, class = void>
@@ -192,12 +193,20 @@ __global__ void __launch_bounds__(256) k_rows(Op op) {
     for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.raw(a, line, F::L2 * n1 + n2);
 #pragma unroll
     for (int n1 = 0; n1 < F::L1; ++n1) any = any || v[n1].x != 0.f || v[n1].y != 0.f;
+    int part[F::L1];
+    if (__any(any)) {  // ahead of the barrier: one more trip to memory after it otherwise
+#pragma unroll
+      for (int n1 = 0; n1 < F::L1; ++n1) part[n1] = op.part(a, line, F::L2 * n1 + n2);
+    } else {
+#pragma unroll
+      for (int n1 = 0; n1 < F::L1; ++n1) part[n1] = 1;
+    }
     any = __syncthreads_or(any);
     const bool flags = op.flags();  // uniform
     if (flags && !any) op.store_flags(a, ab.y * NT, NT, nullptr);
     if (!op.keep(a, ab.y * NT, NT, any)) return;  // block-uniform
 #pragma unroll
-    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.value(v[n1], a, line, F::L2 * n1 + n2);
+    for (int n1 = 0; n1 < F::L1; ++n1) v[n1] = op.value(v[n1], part[n1], a, line, F::L2 * n1 + n2);
     if (flags) {
       uint8_t* f = (uint8_t*)lds;
 #pragma unroll
