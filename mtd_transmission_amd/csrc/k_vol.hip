@@ -566,6 +566,11 @@ k_fill_planes(float2* __restrict__ vol, int32_t* __restrict__ cnt, int V, int z0
   }
 }
 
+// Spectrum and counts that the fill takes a part of: beyond the 256 MiB of the last
+// cache. What stays in it the gather writes beside its sums in one launch (A angles,
+// gather alone / with the fill, us: 256^3 A 30 33 / 43, A 400 89 / 105; 288^3 A 60 53 / 63, A 400
+// 146 / 144; 304^3 A 60 94 / 84, A 400 181 / 168; 320^3 A 1 112 / 93).
+constexpr size_t kFillOver = 288u << 20;
 // the windowed gather with height windows of ZW voxels (LDS: 10 B per
 // voxel of the 256 x ZW block, 8 without counts) and batches of KB list entries
 template <int ZW, int KB>
@@ -580,7 +585,7 @@ static hipError_t gather_windows(const GatherArgs& g, int ntx, int tiles, const 
   int w0 = std::max(zlo, 0) / ZW, w1 = std::min(zhi, V - 1) / ZW;
   if (!band) {
     const bool al = ((uintptr_t)g.vol | (g.cnt ? (uintptr_t)g.cnt : 0)) % 16 == 0;
-    if (g.cnt && al) {
+    if (g.cnt && al && (size_t)V * V * V * 12 > kFillOver) {
       const int z1 = std::min((w1 + 1) * ZW, V);
       const size_t words = (size_t)(w0 * ZW + V - z1) * V * V / 4 * 3;
       if (words) {
