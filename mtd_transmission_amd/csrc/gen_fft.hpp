@@ -51,6 +51,7 @@ constexpr int kGenMaxPasses = 8;
 constexpr int kGenThreads = 512;     // most threads of a block
 constexpr int kGenLdsBytes = 65536;  // most LDS of a block
 constexpr int kGenMaxLen = 4096;     // most points of a line in LDS
+constexpr int kGenBlocks = 256;      // blocks that give every CU one
 
 struct GenPlan {
   int L;                   // transform length
@@ -85,12 +86,15 @@ inline int gen_pitch(int lnl, bool rows) { return rows && lnl > 0 ? (1 << lnl) +
 
 // log2 of the lines per block: up to 32 (128-byte segments of float columns)
 // as far as LDS and the threads allow, 16 where 32 would leave a CU fewer than
-// four blocks
-inline int gen_lnl(const GenPlan& p, bool rows) {
+// four blocks; fewer where the launch would leave CUs without a block (rows and
+// columns of 24 crops of 20^2: 20 us with 32 lines a block, 13 with 4; with half
+// or a quarter of the CUs as the aim 13 and 15; 6 of 300^2 31 and 35, now 30)
+inline int gen_lnl(const GenPlan& p, bool rows, int nlines, int batches) {
   int l = 5;
   auto bytes = [&](int k) { return (size_t)gen_pitch(k, rows) * p.W * sizeof(float2); };
   if (bytes(5) > 40960) l = 4;
   while (l > 0 && (bytes(l) > (size_t)kGenLdsBytes || (p.threads << l) > kGenThreads)) --l;
+  while (l > 1 && ((nlines - 1) >> l) + 1 < kGenBlocks / batches) --l;
   return l;
 }
 
@@ -329,7 +333,7 @@ template <bool INV, bool ROWS, class Op>
 inline hipError_t launch_gen(const Op& op, const GenPlan& p, int nlines, int batches,
                              hipStream_t s) {
   if (nlines <= 0 || batches <= 0) return hipSuccess;
-  const int lnl = gen_lnl(p, ROWS), pitch = gen_pitch(lnl, ROWS);
+  const int lnl = gen_lnl(p, ROWS, nlines, batches), pitch = gen_pitch(lnl, ROWS);
   hipLaunchKernelGGL((k_gen<INV, ROWS, Op>), dim3(gen_groups(nlines, lnl), batches),
                      dim3(gen_threads(p, lnl)), (size_t)pitch * p.W * sizeof(float2), s, op, p,
                      nlines, lnl, pitch);

@@ -463,7 +463,7 @@ struct UnwOutGenOp {  // pairs of columns (2 col, 2 col + 1)
 
 static hipError_t unwrap_gen(int C, const float2* iu, int A, const GenPlan& p, const float2* tw4,
                              float* gx, float2* H, float* phu, hipStream_t s) {
-  const int lr = gen_lnl(p, true), lc = gen_lnl(p, false);
+  const int lr = gen_lnl(p, true, C, A), lc = gen_lnl(p, false, C, A);
   const int pr = gen_pitch(lr, true), pc = gen_pitch(lc, false);
   const size_t mr = (size_t)pr * p.W * sizeof(float2), mc = (size_t)pc * p.W * sizeof(float2);
   const dim3 gr(gen_groups(C, lr), A), gc(gen_groups(C, lc), A);
