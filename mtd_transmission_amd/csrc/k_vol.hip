@@ -951,9 +951,11 @@ static hipError_t vol_cols(Dim<VT> V, const Op& op, const FftTab& ft, const char
 }
 
 // The height pass. Volumes of 448, 512 and from 576 on fold the band (k_cols_fold): planes is
-// the band's height expected from the geometry, 0 where only the device knows
-// (then both forms are launched and the blocks of the one that does not apply
-// return). 512^3, band 151: 335 -> 278 us; 1024^3, band 302: 5.05 -> 2.43 ms.
+// the band's height expected from the geometry, 0 where there is none. Only the
+// device knows the band, and a specular past the pupil's rim makes it wider than
+// expected: both forms are launched, and the blocks of the one that does not apply
+// return (9 us of 2110 at 512^3, nothing to be seen at 1024^3).
+// 512^3, band 151: 335 -> 278 us; 1024^3, band 302: 5.05 -> 2.43 ms.
 template <int VT>
 static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, int tile,
                         hipStream_t s) {
@@ -962,11 +964,11 @@ static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, i
     constexpr int T = Fft2<VT / cols_fold_r<VT>(), false>::T;
     if (planes == 0 || cols_fold_narrow<VT>(T - 1, T - 1 + planes - 1)) {
       Timed tm("vol_z", s);
-      z.only = planes ? 0 : 1;
+      z.only = 1;
       hipLaunchKernelGGL((k_cols_fold<VT, true, ZOutOp<VT>>), dim3(VT / cols_fold_nc<VT>(), VT),
                          dim3(cols_fold_threads<VT>()), 0, s, z);
       const hipError_t e = hipGetLastError();
-      if (planes || e != hipSuccess) return e;
+      if (e != hipSuccess) return e;
       z.only = 2;
     }
   }

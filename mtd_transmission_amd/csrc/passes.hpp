@@ -306,10 +306,10 @@ inline dim3 cols_b_block() {
 // (L/R)-point transform over z mod L/R of x[z] exp(+-2 pi i r z / L), folded. A
 // block loads its band once into registers (NB values a thread) and then runs R
 // short transforms, so it holds 64 columns where the whole transform held 16 or
-// 32: the stores, one plane after the other, become 256-byte pieces. A band of
-// more than NB*T elements is folded from memory, read once per residue (correct,
-// but on a dense spectrum 1.6 -> 2.0 ms for all three passes at 512^3, 15 -> 25 ms
-// at 1024^3): callers that expect one take the whole transform (cols_fold_narrow).
+// 32: the stores, one plane after the other, become 256-byte pieces. For bands of
+// cols_fold_narrow only; the others take the whole transform (folded from memory,
+// read once per residue, they took longer: 640^3, band 0.43 of the height, z
+// pass and all 2536 -> 3271 us, 1024^3 8676 -> 10297).
 //
 // The float outputs' piece is what bounds the height pass. Storing two V^3 float
 // volumes column by column and reading a band of 0.295 V planes, with no
@@ -335,11 +335,6 @@ constexpr int cols_fold_nb() {
   return (36 * L / 100 + Fft2<L / cols_fold_r<L>(), false>::T - 1) /
          Fft2<L / cols_fold_r<L>(), false>::T;
 }
-template <class Op, class = void>
-struct op_cols_fold : std::false_type {};
-template <class Op>
-struct op_cols_fold<Op, std::void_t<decltype(Op::kFoldCols)>>
-    : std::integral_constant<bool, Op::kFoldCols> {};
 template <int L>
 constexpr bool cols_fold_fits() {
   return cols_fold_r<L>() > 1;
@@ -372,13 +367,9 @@ __global__ void __launch_bounds__(cols_fold_threads<L>(), 4) k_cols_fold(Op op) 
   // the first step's input is a phase on its output k1, W_L1^(b k1), which the
   // step twiddle takes along
   const int b = op.lo > 0 ? op.lo / T : 0;
-  const int nj = op.hi >= op.lo ? op.hi / T - b + 1 : 0;
-  const bool fits = cols_fold_narrow<L>(op.lo, op.hi);
   float2 e[NB];
-  if (fits) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) e[j] = op.load_wave(a, c0, c, T * (b + j) + n2);
-  }
+  for (int j = 0; j < NB; ++j) e[j] = op.load_wave(a, c0, c, T * (b + j) + n2);
   // the table is constant: scalar loads
   typedef float v2f __attribute__((ext_vector_type(2)));
   const auto* tw = (const __attribute__((address_space(4))) v2f*)op.tw;
@@ -386,31 +377,16 @@ __global__ void __launch_bounds__(cols_fold_threads<L>(), 4) k_cols_fold(Op op) 
 #pragma unroll 1
   for (int r = 0; r < R; ++r) {
     float2 v[L1], u[L2];
-    if (fits) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        const v2f q = tw[r * (T * (b + j) + n2) % L];
-        const float2 w = make_float2(q.x, INV ? -q.y : q.y);
-        const float2 t = cmul(e[j], w);
-        if (j < L1) v[j] = t;
-        else v[j % L1] = make_float2(v[j % L1].x + t.x, v[j % L1].y + t.y);
-      }
-#pragma unroll
-      for (int j = NB; j < L1; ++j) v[j] = make_float2(0.f, 0.f);
-    } else {
-#pragma unroll
-      for (int j = 0; j < L1; ++j) v[j] = make_float2(0.f, 0.f);
-      for (int j0 = 0; j0 < nj; j0 += L1) {
-#pragma unroll
-        for (int j = 0; j < L1; ++j) {
-          const int z = T * (b + j0 + j) + n2;
-          const v2f q = tw[(r * z) % L];
-          const float2 w = make_float2(q.x, INV ? -q.y : q.y);
-          const float2 t = cmul(op.load_wave(a, c0, c, z), w);
-          v[j] = make_float2(v[j].x + t.x, v[j].y + t.y);
-        }
-      }
+    for (int j = 0; j < NB; ++j) {
+      const v2f q = tw[r * (T * (b + j) + n2) % L];
+      const float2 w = make_float2(q.x, INV ? -q.y : q.y);
+      const float2 t = cmul(e[j], w);
+      if (j < L1) v[j] = t;
+      else v[j % L1] = make_float2(v[j % L1].x + t.x, v[j % L1].y + t.y);
     }
+#pragma unroll
+    for (int j = NB; j < L1; ++j) v[j] = make_float2(0.f, 0.f);
     RegFFT<L1, INV>::run(v);
 #pragma unroll
     for (int k1 = 1; k1 < L1; ++k1) {
