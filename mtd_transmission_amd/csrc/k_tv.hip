@@ -136,7 +136,6 @@ k_tv_fista(const float* __restrict__ z, const float* __restrict__ gd, float* __r
   }
 }
 
-// Data-term gradient of the weighted least squares on the spectra, in place:
 // Solver start: x = max(x, 0) when positivity holds, z = x.
 __global__ void __launch_bounds__(256)
 k_tv_start(float* __restrict__ x, float* __restrict__ z, size_t n, int positivity) {

@@ -165,8 +165,9 @@ __device__ __forceinline__ void line_gradient(const float2 (&z)[Fft2<C, false>::
 // Column blocks: NC adjacent columns, the most of 32 (where it divides C), 16 and
 // 8 that keep the block within MAXT threads (the last block may run past C). The
 // gradient passes hold a line's phasors beside a transform: waves per SIMD
-// that leave them in registers (at 4 waves, crops of 160 to 256 spilled up to
-// 138 of them), in blocks of at most 256 threads so that 3 fit: with 16 columns a
+// that leave nearly all of it in registers (at 4 waves, crops of 160 to 256 spilled up
+// to 138 of them; the column pass still keeps 16 bytes a thread in scratch at 128,
+// 48 at 192, 12 at 250, 148 and 184 at 224 and 256), in blocks of at most 256 threads so that 3 fit: with 16 columns a
 // 250-line block had 7 waves of the CU's 12, and one block was all that fit
 // (300 crops: 321 -> 247 us with 8).
 template <int C, int MAXT>

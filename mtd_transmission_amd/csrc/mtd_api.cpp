@@ -492,6 +492,8 @@ int validate(mtd_ctx* ctx, const mtd_geom* g, int A, int need) {
   if (!crop_len_supported(C) && !gen_len_ok(C))
     return set_err(ctx, MTD_ERR_UNSUPPORTED,
                    "crop side 2*NXMAX=" + std::to_string(C) + " beyond the FFT lengths built");
+  // the sides the unwrapping has always taken: it had transforms of the mirrored
+  // extension's 2C points, where it now has C-point ones
   if (g->c_aber && g->deroul == MTD_DEROUL_VOLKOV && !unwrap_len_supported(C) &&
       !gen_len_ok(2 * C))
     return set_err(ctx, MTD_ERR_UNSUPPORTED,

@@ -319,6 +319,9 @@ inline dim3 cols_b_block() {
 // both steps) and whose whole transform left 9 to 16 columns a block, and 448 and
 // 512. Height pass alone at 4.7 to 8 bins per pupil radius (96 bins): 448^3 242 ->
 // 202 us, 576^3 1077 -> 473, 640^3 1136 -> 607, 704^3 1567 -> 840, 768^3 2140 -> 969.
+// 256, 320 and 384 have the square split too, with 32 columns a block as they are:
+// with both launches (vol_z) they measured 34 -> 31, 78 -> 66 and 145 -> 132 us and are
+// not built yet.
 template <int L>
 constexpr int cols_fold_r() {
   return L == 512 ? 2 : L == 576 ? 4 : L == 640 ? 10 : L == 704 ? 11 : L == 768 ? 3
