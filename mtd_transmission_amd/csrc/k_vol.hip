@@ -22,6 +22,7 @@
 // backward 3-D FFT with both fftshift3D folded into (-1)^(x+y+z) sign flips,
 // times delta_f^3 and -1/(2 n0 kv^2), split into index and absorption.
 #include <algorithm>
+#include <optional>
 
 #include "dft.hpp"
 #include "gen_fft.hpp"
@@ -931,7 +932,8 @@ static hipError_t vol_rows(Dim<VT> V, const Op& op, const FftTab& ft, const char
 template <int VT, bool INV, bool TILES, class Op>
 static hipError_t vol_cols(Dim<VT> V, const Op& op, const FftTab& ft, const char* name, int tile,
                            hipStream_t s) {
-  Timed tm(name, s);
+  std::optional<Timed> tm;  // name NULL: the caller's
+  if (name) tm.emplace(name, s);
   if constexpr (VT > 0) {
     if constexpr (op_cols_balanced<Op>::value && cols_b_fits<VT>()) {
       hipLaunchKernelGGL((k_cols_b<VT, INV, Op>), cols_b_grid<VT>(VT), cols_b_block<VT>(), 0, s,
@@ -959,11 +961,11 @@ static hipError_t vol_cols(Dim<VT> V, const Op& op, const FftTab& ft, const char
 template <int VT>
 static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, int tile,
                         hipStream_t s) {
+  Timed tm("vol_z", s);
   if constexpr (VT > 0 && cols_fold_fits<VT>()) {
     // the band may begin at any element of its first group of T
     constexpr int T = Fft2<VT / cols_fold_r<VT>(), false>::T;
     if (planes == 0 || cols_fold_narrow<VT>(T - 1, T - 1 + planes - 1)) {
-      Timed tm("vol_z", s);
       z.only = 1;
       hipLaunchKernelGGL((k_cols_fold<VT, true, ZOutOp<VT>>), dim3(VT / cols_fold_nc<VT>(), VT),
                          dim3(cols_fold_threads<VT>()), 0, s, z);
@@ -972,7 +974,7 @@ static hipError_t vol_z(Dim<VT> V, ZOutOp<VT> z, int planes, const FftTab& ft, i
       z.only = 2;
     }
   }
-  return vol_cols<VT, true, true>(V, z, ft, "vol_z", tile, s);
+  return vol_cols<VT, true, true>(V, z, ft, nullptr, tile, s);
 }
 
 template <int VT>
